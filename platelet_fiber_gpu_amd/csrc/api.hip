@@ -91,7 +91,7 @@ void free_markers(Markers &m) {
   dfree(m.plt_lowest);
   dfree(m.m2t_start); dfree(m.m2t);
   dfree(m.tri_edge); dfree(m.edge_tri); dfree(m.ring_start); dfree(m.ring);
-  dfree(m.vn); dfree(m.en); dfree(m.km);
+  dfree(m.vn); dfree(m.en); dfree(m.km); dfree(m.tri_n);
   dfree(m.contact_slot); dfree(m.contact_list);
   dfree(m.m2e_start); dfree(m.m2e_nbr); dfree(m.m2e_l0);
   dfree(m.rec_tri); dfree(m.rec_r1); dfree(m.rec_r2);
@@ -1159,6 +1159,7 @@ pfg_status load_impl(pfg_handle *h, const pfg_model &M, const int32_t *minst,
   ALLOC_FILL(m.vn, 0.0, m.bend ? (size_t)3 * n : 0);
   ALLOC_FILL(m.en, 0.0, m.bend ? (size_t)3 * m.n_tedges : 0);
   ALLOC_FILL(m.km, 0.0, m.bend ? (size_t)n : 0);
+  ALLOC_FILL(m.tri_n, 0.0, m.bend ? (size_t)3 * M.n_tri : 0);
   {
     const bool contact = p.contact_a != 0.f && M.n_platelets >= 2;
     const size_t np = (size_t)M.n_platelets;

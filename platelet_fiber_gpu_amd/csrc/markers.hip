@@ -550,6 +550,11 @@ __device__ void triangle_geometry(const MArgs &a, int t) {
   const double St = 0.5 * nn;
   const double cx = (x0 + x1 + x2) / 3.0, cy = (y0 + y1 + y2) / 3.0, cz = (z0 + z1 + z2) / 3.0;
   a.m.tri_S[t] = St;
+  if (a.m.bend) { /* the bending chain's node normals are means of these */
+    a.m.tri_n[3 * (int64_t)t] = nx;
+    a.m.tri_n[3 * (int64_t)t + 1] = ny;
+    a.m.tri_n[3 * (int64_t)t + 2] = nz;
+  }
   a.m.tri_V[t] = (cx * nx + cy * ny + cz * nz) * St / 3.0; /* sem_kernel.cu:806-808 */
   /* per vertex slot s: dS/dx_s = -(L_s x n)/2 with L_s = x_{s+1} - x_{s+2}
    * and the inward n_elem (sem_kernel.cu:1688-1690, 1719-1721), and the
@@ -574,37 +579,52 @@ __device__ void triangle_geometry(const MArgs &a, int t) {
 
 /* ---------------- membrane bending ---------------- */
 
-/* Quadratic 6-node triangle: N_k = a xi^2 + b eta^2 + c xi eta + d xi + e eta + f
- * with rows {a, b, c, d, e, f} of the standard quadratic Lagrange triangle
- * (nodes at the vertices, then the midpoints of v0v1, v0v2, v1v2), and the
- * natural coordinates of the 6 nodes (sem_kernel.cu:94-107). */
-__constant__ double QN[6][6] = {{2, 2, 4, -3, -3, 1}, {2, 0, 0, -1, 0, 0},
-                                {0, 2, 0, 0, -1, 0},  {-4, 0, -4, 4, 0, 0},
-                                {0, -4, -4, 0, 4, 0}, {0, 0, 4, 0, 0, 0}};
-__constant__ double QXE[6][2] = {{0, 0}, {1, 0}, {0, 1}, {0.5, 0}, {0, 0.5}, {0.5, 0.5}};
-
-/* Forward elimination with partial pivoting and unit pivots on a 3 x 4
- * augmented matrix (gaussian_elimination, sem_kernel.cu:249-284). */
-__device__ inline void gauss3x4(double g[12]) {
+/* Forward elimination with partial pivoting and unit pivots on a 3 x 3
+ * matrix with NR right-hand sides (gaussian_elimination,
+ * sem_kernel.cu:249-284, which has one).  A column without a pivot leaves
+ * the pivot row i where it is, so i is a run-time value: every row i can
+ * have at column j is written out, which keeps all indices constants and
+ * the matrix in registers (with run-time rows it lay in scratch memory). */
+template <int NR>
+__device__ inline void gauss3(double (&m)[3][3 + NR]) {
   int i = 0;
-  for (int j = 0; j < 3 && i < 3; ++j) {
-    int maxi = i;
-    for (int k = i + 1; k < 3; ++k)
-      if (fabs(g[k * 4 + j]) > fabs(g[maxi * 4 + j])) maxi = k;
-    if (g[maxi * 4 + j] == 0.0) continue;
-    double initial = 0.0;
-    for (int k = j; k < 4; ++k) {
-      const double b = g[i * 4 + k];
-      g[i * 4 + k] = g[maxi * 4 + k];
-      g[maxi * 4 + k] = b;
-      if (k == j) initial = g[i * 4 + j];
-      g[i * 4 + k] /= initial;
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+#pragma unroll
+    for (int ii = j; ii >= 0; --ii) { /* downward: the row that follows is not met again */
+      if (i != ii) continue;
+      int piv = ii;
+      double best = fabs(m[ii][j]);
+#pragma unroll
+      for (int k = ii + 1; k < 3; ++k) {
+        const double v = fabs(m[k][j]);
+        if (v > best) {
+          best = v;
+          piv = k;
+        }
+      }
+      if (best == 0.0) continue;
+#pragma unroll
+      for (int k = ii + 1; k < 3; ++k) {
+        const bool swap = piv == k;
+#pragma unroll
+        for (int c = j; c < 3 + NR; ++c) {
+          const double u = m[ii][c], v = m[k][c];
+          m[ii][c] = swap ? v : u;
+          m[k][c] = swap ? u : v;
+        }
+      }
+      const double initial = m[ii][j];
+#pragma unroll
+      for (int c = j; c < 3 + NR; ++c) m[ii][c] /= initial;
+#pragma unroll
+      for (int k = ii + 1; k < 3; ++k) {
+        const double f = m[k][j];
+#pragma unroll
+        for (int c = j; c < 3 + NR; ++c) m[k][c] -= f * m[ii][c];
+      }
+      i = ii + 1;
     }
-    for (int k = i + 1; k < 3; ++k) {
-      const double f = g[k * 4 + j];
-      for (int l = j; l < 4; ++l) g[k * 4 + l] -= f * g[i * 4 + l];
-    }
-    ++i;
   }
 }
 
@@ -615,56 +635,106 @@ __device__ inline void pos_d(const MArgs &a, int i, double x[3]) {
   x[2] = p.z;
 }
 
-/* Unit normal -(e12 x e13)/|e12 x e13| of triangle t (sem_kernel.cu:793-803). */
-__device__ inline void tri_unit_normal(const MArgs &a, int t, double n[3]) {
-  double p0[3], p1[3], p2[3];
-  pos_d(a, a.m.tri[3 * t], p0);
-  pos_d(a, a.m.tri[3 * t + 1], p1);
-  pos_d(a, a.m.tri[3 * t + 2], p2);
-  const double e12[3] = {p1[0] - p0[0], p1[1] - p0[1], p1[2] - p0[2]};
-  const double e13[3] = {p2[0] - p0[0], p2[1] - p0[1], p2[2] - p0[2]};
-  n[0] = e12[1] * e13[2] - e12[2] * e13[1];
-  n[1] = e12[2] * e13[0] - e12[0] * e13[2];
-  n[2] = e12[0] * e13[1] - e12[1] * e13[0];
-  const double nn = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
-  n[0] /= -nn;
-  n[1] /= -nn;
-  n[2] /= -nn;
+template <int G>
+__device__ inline double group_sum_d(double v) {
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, G);
+  return v;
 }
 
-/* Node normal k (k < n: vertex k; else the midpoint of triangle edge k - n):
- * mean of the unit normals of its triangles, normalised
- * (sem_calculate_A_kernel and sem_surface_tension_kernel,
- * sem_kernel.cu:810-820, 874-900). */
-__device__ void bend_normal(const MArgs &a, int k) {
-  double s[3] = {0.0, 0.0, 0.0}, nt[3];
+/* Lanes per vertex in the bending chain: a vertex of a closed mesh has six
+ * triangles and neighbours on average, each a dependent walk of gathers and
+ * FP64 divisions of its own, so the launches are bound by the latency of one
+ * lane's walk and a lane per triangle shortens it six times over. */
+constexpr int BEND_LANES = 8;
+
+/* Normal of vertex v: the mean of its triangles' unit normals, normalised
+ * (sem_calculate_A_kernel, sem_kernel.cu:810-820). */
+__device__ void bend_vertex_normal(const MArgs &a, int v, int lane) {
+  const int q0 = a.m.m2t_start[v], cnt = a.m.m2t_start[v + 1] - q0;
+  if (cnt == 0) return; /* the whole group leaves together */
+  double s[3] = {0.0, 0.0, 0.0};
+  for (int q = lane; q < cnt; q += BEND_LANES) {
+    const double *t = a.m.tri_n + 3 * (int64_t)(a.m.m2t[q0 + q] / 3);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) s[d] += t[d];
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) s[d] = group_sum_d<BEND_LANES>(s[d]) / cnt;
+  if (lane != 0) return;
+  const double nn = sqrt(s[0] * s[0] + s[1] * s[1] + s[2] * s[2]);
+#pragma unroll
+  for (int d = 0; d < 3; ++d) a.m.vn[3 * (int64_t)v + d] = s[d] / nn;
+}
+
+/* Normal of the midpoint of triangle edge e: the same over its one or two
+ * triangles (sem_surface_tension_kernel, sem_kernel.cu:874-900). */
+__device__ void bend_edge_normal(const MArgs &a, int e) {
+  double s[3] = {0.0, 0.0, 0.0};
   int cnt = 0;
-  double *out;
-  if (k < a.m.n) {
-    for (int q = a.m.m2t_start[k]; q < a.m.m2t_start[k + 1]; ++q, ++cnt) {
-      tri_unit_normal(a, a.m.m2t[q] / 3, nt);
-      s[0] += nt[0];
-      s[1] += nt[1];
-      s[2] += nt[2];
-    }
-    out = a.m.vn + 3 * (int64_t)k;
-  } else {
-    const int e = k - a.m.n;
-    for (int j = 0; j < 2; ++j) {
-      const int q = a.m.edge_tri[2 * e + j];
-      if (q < 0) continue;
-      tri_unit_normal(a, q / 3, nt);
-      s[0] += nt[0];
-      s[1] += nt[1];
-      s[2] += nt[2];
-      ++cnt;
-    }
-    out = a.m.en + 3 * (int64_t)e;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int q = a.m.edge_tri[2 * e + j];
+    if (q < 0) continue;
+    const double *t = a.m.tri_n + 3 * (int64_t)(q / 3);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) s[d] += t[d];
+    ++cnt;
   }
   if (cnt == 0) return;
+#pragma unroll
   for (int d = 0; d < 3; ++d) s[d] /= cnt;
   const double nn = sqrt(s[0] * s[0] + s[1] * s[1] + s[2] * s[2]);
-  for (int d = 0; d < 3; ++d) out[d] = s[d] / nn;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) a.m.en[3 * (int64_t)e + d] = s[d] / nn;
+}
+
+/* Trace of the curvature tensor at vertex s of a 6-node triangle (natural
+ * coordinates (0,0), (1,0), (0,1) of the three vertices).  s differs between
+ * the lanes of a wavefront and enters as values, not as an index. */
+__device__ inline double bend_trace(const double (&xc)[6][3], const double (&nc)[6][3], int s) {
+  const double xi = s == 1 ? 1.0 : 0.0, et = s == 2 ? 1.0 : 0.0;
+  /* rows {a, b, c, d, e, f}: N_k = a xi^2 + b eta^2 + c xi eta + d xi + e eta + f
+   * of the standard quadratic Lagrange triangle (vertices, then the
+   * midpoints of v0v1, v0v2, v1v2; sem_kernel.cu:94-107) */
+  constexpr double N[6][6] = {{2, 2, 4, -3, -3, 1}, {2, 0, 0, -1, 0, 0},
+                              {0, 2, 0, 0, -1, 0},  {-4, 0, -4, 4, 0, 0},
+                              {0, -4, -4, 0, 4, 0}, {0, 0, 4, 0, 0, 0}};
+  double A1[3] = {0, 0, 0}, A2[3] = {0, 0, 0}, A3[3] = {0, 0, 0}, A4[3] = {0, 0, 0};
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    const double dxi = 2.0 * N[k][0] * xi + N[k][2] * et + N[k][3];
+    const double det = 2.0 * N[k][1] * et + N[k][2] * xi + N[k][4];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      A1[d] += xc[k][d] * dxi;
+      A2[d] += nc[k][d] * dxi;
+      A3[d] += xc[k][d] * det;
+      A4[d] += nc[k][d] * det;
+    }
+  }
+  /* K x_xi = n_xi, K x_eta = n_eta, K n = 0: the three rows of K have one
+   * matrix and a right-hand side each; only K[r][r] enters the trace */
+  double m[3][6];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    m[0][c] = A1[c];
+    m[1][c] = A3[c];
+    m[2][c] = s == 0 ? nc[0][c] : (s == 1 ? nc[1][c] : nc[2][c]);
+    m[0][3 + c] = A2[c];
+    m[1][3 + c] = A4[c];
+    m[2][3 + c] = 0.0;
+  }
+  gauss3<3>(m);
+  double tr = 0.0;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const double k2 = m[2][3 + r];
+    const double k1 = m[1][3 + r] - k2 * m[1][2];
+    const double k0 = m[0][3 + r] - k2 * m[0][2] - k1 * m[0][1];
+    tr += r == 0 ? k0 : (r == 1 ? k1 : k2);
+  }
+  return tr;
 }
 
 /* Mean curvature of vertex v: at its node of every incident 6-node triangle
@@ -672,55 +742,38 @@ __device__ void bend_normal(const MArgs &a, int k) {
  * K n = 0 row by row (solve_linear_eqns); km = trace of the mean K / 2
  * (sem_calculate_Kapa_kernel and sem_calculate_m_kernel,
  * sem_kernel.cu:950-1100; the symmetrisation there keeps the trace). */
-__device__ void bend_km(const MArgs &a, int v) {
+__device__ void bend_km(const MArgs &a, int v, int lane) {
   const int q0 = a.m.m2t_start[v], cnt = a.m.m2t_start[v + 1] - q0;
   if (cnt == 0) return;
   double tr = 0.0;
-  for (int q = q0; q < q0 + cnt; ++q) {
-    const int t = a.m.m2t[q] / 3, s = a.m.m2t[q] % 3;
-    double xc[6][3], nc[6][3];
+  for (int q = lane; q < cnt; q += BEND_LANES) {
+    const int e3 = a.m.m2t[q0 + q], t = e3 / 3, s = e3 - 3 * t;
+    int vk[3], ek[3];
+#pragma unroll
     for (int k = 0; k < 3; ++k) {
-      const int vk = a.m.tri[3 * t + k];
-      pos_d(a, vk, xc[k]);
-      for (int d = 0; d < 3; ++d) nc[k][d] = a.m.vn[3 * (int64_t)vk + d];
-      const int e = a.m.tri_edge[3 * t + k];
-      for (int d = 0; d < 3; ++d) nc[3 + k][d] = a.m.en[3 * (int64_t)e + d];
+      vk[k] = a.m.tri[3 * t + k];
+      ek[k] = a.m.tri_edge[3 * t + k];
     }
+    double xc[6][3], nc[6][3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      pos_d(a, vk[k], xc[k]);
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        nc[k][d] = a.m.vn[3 * (int64_t)vk[k] + d];
+        nc[3 + k][d] = a.m.en[3 * (int64_t)ek[k] + d];
+      }
+    }
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
       xc[3][d] = 0.5 * (xc[0][d] + xc[1][d]);
       xc[4][d] = 0.5 * (xc[0][d] + xc[2][d]);
       xc[5][d] = 0.5 * (xc[1][d] + xc[2][d]);
     }
-    const double xi = QXE[s][0], et = QXE[s][1];
-    double A1[3] = {0, 0, 0}, A2[3] = {0, 0, 0}, A3[3] = {0, 0, 0}, A4[3] = {0, 0, 0};
-    for (int k = 0; k < 6; ++k) {
-      const double dxi = 2.0 * QN[k][0] * xi + QN[k][2] * et + QN[k][3];
-      const double det = 2.0 * QN[k][1] * et + QN[k][2] * xi + QN[k][4];
-      for (int d = 0; d < 3; ++d) {
-        A1[d] += xc[k][d] * dxi;
-        A2[d] += nc[k][d] * dxi;
-        A3[d] += xc[k][d] * det;
-        A4[d] += nc[k][d] * det;
-      }
-    }
-    for (int r = 0; r < 3; ++r) { /* row r of K; only K[r][r] enters km */
-      double g[12];
-      for (int c = 0; c < 3; ++c) {
-        g[c] = A1[c];
-        g[4 + c] = A3[c];
-        g[8 + c] = nc[s][c];
-      }
-      g[3] = A2[r];
-      g[7] = A4[r];
-      g[11] = 0.0;
-      gauss3x4(g);
-      const double k2 = g[11];
-      const double k1 = g[7] - k2 * g[6];
-      const double k0 = g[3] - k2 * g[2] - k1 * g[1];
-      tr += r == 0 ? k0 : (r == 1 ? k1 : k2);
-    }
+    tr += bend_trace(xc, nc, s);
   }
-  a.m.km[v] = 0.5 * tr / cnt;
+  tr = group_sum_d<BEND_LANES>(tr);
+  if (lane == 0) a.m.km[v] = 0.5 * tr / cnt;
 }
 
 __device__ inline double dist_d(const double a[3], const double b[3]) {
@@ -764,21 +817,22 @@ __device__ void ring_term(const MArgs &a, int i, int r0, int c, int q, double *s
   } else if (aj < 0) {
     for (int k = 0; k < 3; ++k) ce[k] = ci2[k];
   } else { /* circumcentre: two bisector planes and the triangle's plane */
-    double g[12] = {0};
+    double m[3][4] = {};
+#pragma unroll
     for (int k = 0; k < 3; ++k) {
-      g[k] = rij[k];
-      g[4 + k] = ri2[k];
-      g[3] += cij[k] * rij[k];
-      g[7] += ci2[k] * ri2[k];
+      m[0][k] = rij[k];
+      m[1][k] = ri2[k];
+      m[0][3] += cij[k] * rij[k];
+      m[1][3] += ci2[k] * ri2[k];
     }
-    g[8] = (xj[1] - xi[1]) * (x2[2] - xi[2]) - (xj[2] - xi[2]) * (x2[1] - xi[1]);
-    g[9] = (xj[2] - xi[2]) * (x2[0] - xi[0]) - (xj[0] - xi[0]) * (x2[2] - xi[2]);
-    g[10] = (xj[0] - xi[0]) * (x2[1] - xi[1]) - (xj[1] - xi[1]) * (x2[0] - xi[0]);
-    g[11] = g[8] * xi[0] + g[9] * xi[1] + g[10] * xi[2];
-    gauss3x4(g);
-    ce[2] = g[11];
-    ce[1] = g[7] - ce[2] * g[6];
-    ce[0] = g[3] - ce[2] * g[2] - ce[1] * g[1];
+    m[2][0] = (xj[1] - xi[1]) * (x2[2] - xi[2]) - (xj[2] - xi[2]) * (x2[1] - xi[1]);
+    m[2][1] = (xj[2] - xi[2]) * (x2[0] - xi[0]) - (xj[0] - xi[0]) * (x2[2] - xi[2]);
+    m[2][2] = (xj[0] - xi[0]) * (x2[1] - xi[1]) - (xj[1] - xi[1]) * (x2[0] - xi[0]);
+    m[2][3] = m[2][0] * xi[0] + m[2][1] * xi[1] + m[2][2] * xi[2];
+    gauss3<1>(m);
+    ce[2] = m[2][3];
+    ce[1] = m[1][3] - ce[2] * m[1][2];
+    ce[0] = m[0][3] - ce[2] * m[0][2] - ce[1] * m[0][1];
   }
   double L1 = dist_d(xi, cij), L2 = dist_d(ce, cij);
   const double L3 = dist_d(xi, ce);
@@ -788,21 +842,16 @@ __device__ void ring_term(const MArgs &a, int i, int r0, int c, int q, double *s
   L2 = dist_d(ce, ci2);
   P = 0.5 * (L1 + L2 + L3);
   A += sqrt(P * (P - L1) * (P - L2) * (P - L3));
-  const double alpha = 1.0 / tan(acos(a1 / (dist_d(xi, x1) * dist_d(x1, xj))));
-  const double beta = 1.0 / tan(acos(a2 / (dist_d(xi, x2) * dist_d(x2, xj))));
+  /* cot(acos c) = c / sqrt(1 - c^2) */
+  const double c1 = a1 / (dist_d(xi, x1) * dist_d(x1, xj));
+  const double c2 = a2 / (dist_d(xi, x2) * dist_d(x2, xj));
+  const double alpha = c1 / sqrt((1.0 - c1) * (1.0 + c1));
+  const double beta = c2 / sqrt((1.0 - c2) * (1.0 + c2));
   *sum = 0.5 * (alpha + beta) * (a.m.km[j] - a.m.km[i]);
   *area = A;
 }
 
-template <int G>
-__device__ inline double group_sum_d(double v) {
-#pragma unroll
-  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, G);
-  return v;
-}
-
-/* roles: A = scatter markers into bins (blocks0), B = triangle terms (blocks1),
- * C = bending node normals, vertices then edge midpoints (blocks2) */
+/* roles: A = scatter markers into bins (blocks0), B = triangle terms (blocks1) */
 __global__ __launch_bounds__(256) void place_kernel(MArgs a) {
   int blk = blockIdx.x;
   if (a.roles & ROLE_A) {
@@ -828,21 +877,31 @@ __global__ __launch_bounds__(256) void place_kernel(MArgs a) {
 /* Membrane bending, launched only when it is on (separate kernels keep the
  * FP64 solves out of the register budget of the force pass):
  * bend_normal_kernel after the triangle pass, bend_km_kernel after it,
- * bend_force_kernel after the force pass (it adds to the marker forces). */
+ * bend_force_kernel after the force pass (it adds to the marker forces).
+ * Bound by latency (a few wavefronts per CU at most).  Three platelets of
+ * 958 elements: normals 6.6 -> 4.8 us, curvature 166 -> 4.7 us, force
+ * 23 -> 5.4 us, against a lane per vertex (normals, curvature: one lane walked
+ * six triangles, three eliminations each, in 256 B of scratch) and four. */
+/* workgroups of the vertices (blocks0), then of the edges */
 __global__ __launch_bounds__(256) void bend_normal_kernel(MArgs a) {
-  const int k = blockIdx.x * 256 + threadIdx.x;
-  if (k < a.m.n + a.m.n_tedges) bend_normal(a, k);
+  if ((int)blockIdx.x < a.blocks0) {
+    const int v = (blockIdx.x * 256 + threadIdx.x) / BEND_LANES;
+    if (v < a.m.n) bend_vertex_normal(a, v, threadIdx.x & (BEND_LANES - 1));
+    return;
+  }
+  const int e = ((int)blockIdx.x - a.blocks0) * 256 + threadIdx.x;
+  if (e < a.m.n_tedges) bend_edge_normal(a, e);
 }
 
 __global__ __launch_bounds__(256) void bend_km_kernel(MArgs a) {
-  const int v = blockIdx.x * 256 + threadIdx.x;
-  if (v < a.m.n) bend_km(a, v);
+  const int v = (blockIdx.x * 256 + threadIdx.x) / BEND_LANES;
+  if (v < a.m.n) bend_km(a, v, threadIdx.x & (BEND_LANES - 1));
 }
 
-/* Four lanes per vertex over its ring (sem_Laplace_Kapa_kernel,
+/* BEND_LANES lanes per vertex over its ring (sem_Laplace_Kapa_kernel,
  * sem_kernel.cu:1499-1638); lane 0 adds kbend (sum / A) n_i. */
 __global__ __launch_bounds__(256) void bend_force_kernel(MArgs a) {
-  constexpr int G = 4;
+  constexpr int G = BEND_LANES;
   const int i = (blockIdx.x * 256 + threadIdx.x) / G, lane = threadIdx.x & (G - 1);
   if (i >= a.m.n) return;
   const int r0 = a.m.ring_start[i], c = a.m.ring_start[i + 1] - r0;
@@ -3565,11 +3624,10 @@ hipError_t launch_place(pfg_handle *h, bool scatter, bool geometry) {
   if (grid == 0) return hipSuccess;
   hipLaunchKernelGGL(place_kernel, dim3(grid), dim3(256), 0, h->stream, a);
   if (geometry && h->m.bend) { /* node normals, then the mean curvature */
-    hipLaunchKernelGGL(bend_normal_kernel,
-                       dim3(blocks_for((int64_t)h->m.n + h->m.n_tedges, 256)), dim3(256), 0,
-                       h->stream, a);
-    hipLaunchKernelGGL(bend_km_kernel, dim3(blocks_for(h->m.n, 256)), dim3(256), 0,
-                       h->stream, a);
+    a.blocks0 = blocks_for((int64_t)h->m.n * BEND_LANES, 256);
+    hipLaunchKernelGGL(bend_normal_kernel, dim3(a.blocks0 + blocks_for(h->m.n_tedges, 256)),
+                       dim3(256), 0, h->stream, a);
+    hipLaunchKernelGGL(bend_km_kernel, dim3(a.blocks0), dim3(256), 0, h->stream, a);
   }
   return hipGetLastError();
 }
@@ -3687,7 +3745,7 @@ hipError_t launch_forces(pfg_handle *h, bool spread) {
     hipLaunchKernelGGL(forces_body_kernel, dim3(h->m.n_fbodies), dim3(256), 0, h->stream, a);
   }
   if (h->m.bend)
-    hipLaunchKernelGGL(bend_force_kernel, dim3(blocks_for((int64_t)h->m.n * 4, 256)),
+    hipLaunchKernelGGL(bend_force_kernel, dim3(blocks_for((int64_t)h->m.n * BEND_LANES, 256)),
                        dim3(256), 0, h->stream, a);
   if (contact_on(h)) {
     hipLaunchKernelGGL(contact_pairs_kernel, dim3(blocks_for(h->m.n, 256)), dim3(256), 0,

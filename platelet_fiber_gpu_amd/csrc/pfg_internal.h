@@ -180,6 +180,7 @@ struct Markers {
   int32_t *edge_tri = nullptr;   /* 2 per edge: 3 * triangle + slot, or -1   */
   int32_t *ring_start = nullptr, *ring = nullptr; /* empty ring: open vertex */
   double *vn = nullptr, *en = nullptr; /* unit normals of vertices, edges     */
+  double *tri_n = nullptr;       /* unit normals of the triangles            */
   double *km = nullptr;          /* mean curvature per vertex                */
   /* CSR marker -> mesh-edge partners with rest length */
   int n_edges = 0;
