@@ -1,8 +1,8 @@
 /*
  * pfg.h -- C ABI of the MI355X coupled platelet-fibrin step.
  *
- * One handle owns one lattice (D3Q19, populations in HBM as 64-cell x-blocks
- * of 19 direction chunks), one marker set
+ * One handle owns one lattice (D3Q19, populations in HBM as blocks of 64
+ * consecutive cells, 19 direction chunks each), one marker set
  * (platelet SEM elements and fibrin nodes), their topology and one HIP stream.
  * Every call returns a pfg_status; nothing calls exit().  Handles are
  * thread-compatible (one thread per handle at a time), not thread-safe.
@@ -487,22 +487,23 @@ pfg_status pfg_time_lb(pfg_handle *h, int nlaunch, double *ms_per_launch);
  * practical bandwidth reference; allocates its own buffers. */
 pfg_status pfg_copy_probe(int device, size_t bytes, int reps, double *gbs);
 
-/* LB-kernel launch tuning: lattice cells each lane updates along z (1, 2 or
- * 4; a wavefront updates one 64-cell x-block of that many rows).  Applies to
- * batches too; the overlap mode of a batch runs with 1 only. */
+/* LB-kernel launch tuning: lattice cells each lane updates (1, 2 or 4: a
+ * wavefront updates that many blocks of 64 cells).  Same results either way.
+ * Applies to batches too; the overlap mode and the persistent launch take 1. */
 pfg_status pfg_set_lb_tuning(pfg_handle *h, int cells_per_lane);
 /* Batches: enable = 1 runs the batched LB update as one persistent launch of
- * the workgroups the CUs hold at once, which take the x-block-row tasks of
- * all lattices from a device work queue (in the order of the workgroup
+ * the workgroups the CUs hold at once, which take the tasks (four blocks of
+ * 64 cells each) of all lattices from a device work queue (in the order of the workgroup
  * table) until it is empty; 0 (default) launches one workgroup per task.
  * Same results either way.  The queue resets itself at the end of each
  * launch, so captured steps carry no clearing node.  PFG_ERR_STATE when
  * enabled on a single-lattice handle. */
 pfg_status pfg_set_lb_persistent(pfg_handle *h, int enable);
 /* LB-kernel workgroup order: 0 as the hardware deals workgroups round-robin
- * to the 8 XCDs, 1 each XCD a contiguous range of rows, so that
+ * to the 8 XCDs, 1 each XCD a contiguous range of cells, so that
  * neighbouring rows share its L2.  Same results either way.  Default: 1
- * from 2^27 lattice cells up (single lattice), else 0.  In a batch the
+ * from 2^27 lattice cells up (single lattice) and while both copies of the
+ * populations fit 256 MiB, else 0.  In a batch the
  * ranges are taken from its workgroup table (the persistent launch has
  * per-XCD ranges of its own). */
 pfg_status pfg_set_lb_xcd_rows(pfg_handle *h, int enable);

@@ -293,14 +293,12 @@ pfg_status check_lattice_params(const pfg_params &p) {
   return PFG_OK;
 }
 
-/* Batched LB launch layout for h->lb_cpt z-cells per lane: each lattice's
- * workgroups (four wavefronts, one x-block row of lb_cpt z-cells each) and
- * the workgroup -> lattice table. */
+/* Batched LB launch layout: each lattice's workgroups (four wavefronts, a
+ * block of 64 cells each) and the workgroup -> lattice table. */
 hipError_t batch_layout(pfg_handle *h) {
   int64_t blk = 0;
   for (Inst &I : h->inst) {
-    const int64_t zrows = (I.p.nz + h->lb_cpt - 1) / h->lb_cpt;
-    I.lb_blocks = ((int64_t)I.nxb * I.p.ny * zrows + 3) / 4;
+    I.lb_blocks = (I.nfblk + 3) / 4;
     I.lb_block0 = blk;
     blk += I.lb_blocks;
   }
@@ -381,15 +379,15 @@ pfg_status create_impl(const pfg_params *ps, int K, int device, pfg_handle **out
     I.p.f16_scale_log2 = p.f16_scale_log2;
     I.N = (int64_t)I.p.nx * I.p.ny * I.p.nz;
     I.cell0 = cell;
-    I.nxb = (I.p.nx + XBLOCK - 1) / XBLOCK;
     I.fblk0 = fblk;
+    I.nfblk = (I.N + XBLOCK - 1) / XBLOCK;
     I.tnx = (I.p.nx + TILE_X - 1) / TILE_X;
     I.tny = (I.p.ny + TILE_Y - 1) / TILE_Y;
     I.tnz = (I.p.nz + TILE_Z - 1) / TILE_Z;
     I.ntiles = (int64_t)I.tnx * I.tny * I.tnz;
     I.tile0 = tile;
     cell += I.N;
-    fblk += (int64_t)I.nxb * I.p.ny * I.p.nz;
+    fblk += I.nfblk;
     tile += I.ntiles;
     flags = flags || I.p.use_flags;
   }
@@ -405,7 +403,6 @@ pfg_status create_impl(const pfg_params *ps, int K, int device, pfg_handle **out
     }
     h->N = cell;
     h->plane = (h->N + 255) / 256 * 256;
-    h->nxb = h->inst[0].nxb;
     const size_t fbytes = (size_t)h->esize * Q * XBLOCK * (size_t)fblk;
     for (int c = 0; c < 2; ++c) {
       if (hipMalloc(&h->f[c], fbytes) != hipSuccess) {
@@ -444,7 +441,7 @@ pfg_status create_impl(const pfg_params *ps, int K, int device, pfg_handle **out
     if (dalloc(h, &h->red, (size_t)4 * h->red_blocks) != hipSuccess) { st = PFG_ERR_ALLOC; break; }
     /* z-cells per lane of the LB kernel */
     h->lb_cpt = 1;
-    h->lb_xcd_rows = (K == 1 && h->N >= XCD_ROWS_MIN_CELLS) ? 1 : 0;
+    h->lb_xcd_rows = lb_default_xcd_rows(h);
     if (dalloc(h, &h->m.counters, N_COUNTERS) != hipSuccess) { st = PFG_ERR_ALLOC; break; }
     if (hipMemset(h->m.counters, 0, sizeof(int64_t) * N_COUNTERS) != hipSuccess) { st = PFG_ERR_DEVICE; break; }
     if (dalloc(h, &h->m.ticket, 1) != hipSuccess) { st = PFG_ERR_ALLOC; break; }
@@ -462,6 +459,8 @@ pfg_status create_impl(const pfg_params *ps, int K, int device, pfg_handle **out
       if (hipMemset(h->solid, 0, (size_t)h->N) != hipSuccess) { st = PFG_ERR_DEVICE; break; }
       if (dalloc(h, &h->bbmask, (size_t)h->N) != hipSuccess) { st = PFG_ERR_ALLOC; break; }
       if (hipMemset(h->bbmask, 0, sizeof(uint32_t) * h->N) != hipSuccess) { st = PFG_ERR_DEVICE; break; }
+      if (dalloc(h, &h->block_kind, (size_t)fblk) != hipSuccess) { st = PFG_ERR_ALLOC; break; }
+      if (hipMemset(h->block_kind, 0, sizeof(int32_t) * (size_t)fblk) != hipSuccess) { st = PFG_ERR_DEVICE; break; }
     }
     if (K > 1) {
       std::vector<int64_t> tile0((size_t)K + 1);
@@ -599,6 +598,7 @@ pfg_status pfg_destroy(pfg_handle *h) {
   dfree(h->tile_stamp);
   dfree(h->solid);
   dfree(h->bbmask);
+  dfree(h->block_kind);
   dfree(h->red);
   dfree(h->lb_block_inst);
   dfree(h->lb_queue);
@@ -1649,9 +1649,7 @@ static hipError_t run_stage(pfg_handle *h, int s) {
 static hipError_t enqueue_step(pfg_handle *h, hipEvent_t lb0, hipEvent_t lb1) {
   hipError_t e = hipSuccess;
   const bool markers = h->model_loaded && h->m.n > 0 && !h->fluid_only;
-  /* the row-split LB passes take one z-row per wavefront */
-  const bool overlap = markers && h->overlap && h->row_stamp && !lb0 && !lb1 &&
-                       (h->K == 1 || h->lb_cpt == 1);
+  const bool overlap = markers && h->overlap && h->row_stamp && !lb0 && !lb1;
   if (markers) {
     e = launch_begin(h, false, true);
     if (overlap) {
@@ -1833,7 +1831,7 @@ pfg_status pfg_set_step(pfg_handle *h, int64_t step) {
   if (h->m.fb_done) PFG_TRY(hipMemset(h->m.fb_done, 0xff, sizeof(int32_t) * (size_t)h->m.n_fbodies));
   if (h->row_stamp) {
     size_t rows = 0;
-    for (const Inst &I : h->inst) rows += (size_t)I.nxb * I.p.ny * I.p.nz;
+    for (const Inst &I : h->inst) rows += (size_t)I.nfblk;
     PFG_TRY(hipMemset(h->row_stamp, 0xff, sizeof(int32_t) * rows));
   }
   h->h_step = step;
@@ -1897,15 +1895,8 @@ pfg_status pfg_profile(pfg_handle *h, int nsteps, double *ms_total, double *ms_l
 pfg_status pfg_set_lb_tuning(pfg_handle *h, int cells_per_lane) {
   if (!h) return PFG_ERR_ARG;
   if (cells_per_lane != 1 && cells_per_lane != 2 && cells_per_lane != 4) return PFG_ERR_ARG;
-  if (cells_per_lane == h->lb_cpt) return PFG_OK;
-  hipSetDevice(h->device);
   h->lb_cpt = cells_per_lane;
   drop_graph(h);
-  if (h->K > 1) { /* the batched launch's workgroups depend on it */
-    PFG_TRY(hipStreamSynchronize(h->stream));
-    PFG_TRY(batch_layout(h));
-    PFG_TRY(upload_batch_args(h));
-  }
   return PFG_OK;
 }
 
@@ -1930,7 +1921,7 @@ struct Snapshot {
 
 size_t population_bytes(const pfg_handle *h) {
   size_t blocks = 0;
-  for (const Inst &I : h->inst) blocks += (size_t)I.nxb * I.p.ny * I.p.nz;
+  for (const Inst &I : h->inst) blocks += (size_t)I.nfblk;
   return (size_t)h->esize * Q * XBLOCK * blocks;
 }
 
@@ -1977,7 +1968,7 @@ hipError_t snapshot_copy(pfg_handle *h, Snapshot &S, bool save) {
       e = hipMemsetAsync(h->m.fb_done, 0xff, 4 * (size_t)h->m.n_fbodies, h->stream);
     if (e == hipSuccess && h->row_stamp) {
       size_t rows = 0;
-      for (const Inst &I : h->inst) rows += (size_t)I.nxb * I.p.ny * I.p.nz;
+      for (const Inst &I : h->inst) rows += (size_t)I.nfblk;
       e = hipMemsetAsync(h->row_stamp, 0xff, 4 * rows, h->stream);
     }
     if (e == hipSuccess) e = hipMemsetAsync(h->aux, 0, sizeof(float) * 3 * (size_t)h->plane, h->stream);
@@ -2018,13 +2009,8 @@ hipError_t apply_shape(pfg_handle *h, const Shape &s) {
   h->ib_staging = s.staging;
   h->overlap = s.overlap != 0;
   h->lb_persistent = h->K > 1 ? s.persistent : 0;
-  if (h->lb_cpt == s.cpt) return hipSuccess;
   h->lb_cpt = s.cpt;
-  if (h->K == 1) return hipSuccess;
-  /* the batched LB launch's workgroups follow the cells per lane */
-  hipError_t e = batch_layout(h);
-  if (e == hipSuccess) e = upload_batch_args(h);
-  return e;
+  return hipSuccess;
 }
 
 /* ms per step of `steps` steps from the snapshot (after `warm` steps from the
@@ -2072,13 +2058,14 @@ pfg_status pfg_autotune(pfg_handle *h, int steps, pfg_tuning *out) {
   /* knobs, tried one at a time from the automatic shape, each kept at its
    * fastest value before the next is tried (values 0 are the automatic
    * choices); a value replaces the best only when it is 1 % faster */
+  const int xcd0 = lb_default_xcd_rows(h);
   const int cpts[3] = {1, 2, 4}, lanes[7] = {64, 32, 16, 8, 4, 2, 1}, ovl[2] = {0, 1},
-            xcds[2] = {0, 1}, pers[2] = {0, 1}, fbod[2] = {1, 2};
+            xcds[2] = {xcd0, 1 - xcd0}, pers[2] = {0, 1}, fbod[2] = {1, 2};
   /* spreading forms that apply to this model */
   int stag[4] = {1, 2, 0, 0}, nstag = 2;
   if (h->m.n_bodies > 0) stag[nstag++] = 4;
   if (h->m.tile_gather_ok) stag[nstag++] = 3;
-  Shape best{1, 0, 0, 0, (h->K == 1 && h->N >= XCD_ROWS_MIN_CELLS) ? 1 : 0, 0, 0};
+  Shape best{1, 0, 0, 0, xcd0, 0, 0};
   const int warm = GRAPH_CHUNK;
   pfg_status st = PFG_OK;
   double best_ms = 0.0;
@@ -2087,7 +2074,7 @@ pfg_status pfg_autotune(pfg_handle *h, int steps, pfg_tuning *out) {
   st = e == hipSuccess ? time_shape(h, S, steps, warm, &best_ms) : from_hip(e);
   out->ms_default = best_ms;
   tried = 1;
-  /* knobs: 0 LB cells per lane, 1 LB row order, 5 the
+  /* knobs: 0 LB cells per lane, 1 LB block order, 5 the
    * persistent batched launch (batches), 6 the force pass by body, 2 force
    * lanes, 3 spreading form, 4 overlap */
   const int order[7] = {0, 1, 5, 6, 2, 3, 4};

@@ -17,15 +17,17 @@
  * not on the O(1) weights; FP16 values stay in the scaled space and only the
  * four moments are unscaled.
  *
- * Layout (blocked SoA): the cells of a lattice row are grouped in x-blocks of
- * 64 (one wavefront).  Block b = (x/64) + nxb*(y + ny*z) stores its 19
- * directions as 19 consecutive chunks of 64 values:
- *     element(d, x, y, z) = (b * 19 + d) * 64 + x % 64.
- * A wavefront updates one x-block: its 19 stores fill one contiguous
- * 19*64-value segment, and each of its loads comes from one chunk of an
- * upstream block (one of nine rows), so DRAM pages are reused across the
- * directions instead of streaming 38 separate planes.  The chunk base is
- * wavefront-uniform; the lane offset is one of three values per lane.
+ * Layout (blocked SoA): the cells i = x + nx (y + ny z) of a lattice are cut
+ * into blocks of 64 consecutive ones (one wavefront), across rows.  Block b
+ * stores its 19 directions as 19 consecutive chunks of 64 values:
+ *     element(d, i) = ((i / 64) * 19 + d) * 64 + i % 64.
+ * A wavefront updates one block: its 19 stores fill one contiguous
+ * 19*64-value segment, and each of its loads reads the 64 values of one
+ * direction at a constant offset in i (one run in two neighbouring blocks),
+ * so DRAM pages are reused across the directions instead of streaming 38
+ * separate planes.  Only the last block of a lattice is partly empty: blocks
+ * cut from each row, an earlier form, left a third of them empty in a batch
+ * of lattices of 32 to 96 cells in x.
  */
 #include <hip/hip_runtime.h>
 
@@ -41,7 +43,7 @@ namespace pfg {
 /* ---------------- storage formats ---------------- */
 
 /* load: the stored value as float (FP16 values stay scaled by 2^s);
- * put: store an already scaled value. */
+ * pack: an already scaled value as it is stored. */
 template <int S>
 struct Store;
 
@@ -50,7 +52,7 @@ struct Store<PFG_STORE_F32> {
   using T = float;
   static constexpr bool scaled = false;
   __device__ static inline float load(const T *p) { return *p; }
-  __device__ static inline void put(T *p, float v) { __builtin_nontemporal_store(v, p); }
+  __device__ static inline T pack(float v) { return v; }
 };
 
 template <>
@@ -60,9 +62,8 @@ struct Store<PFG_STORE_F16> {
   __device__ static inline float load(const T *p) {
     return (float)__builtin_bit_cast(_Float16, *p);
   }
-  __device__ static inline void put(T *p, float v) {
-    const _Float16 hv = (_Float16)v; /* round to nearest even */
-    __builtin_nontemporal_store(__builtin_bit_cast(uint16_t, hv), p);
+  __device__ static inline T pack(float v) {
+    return __builtin_bit_cast(uint16_t, (_Float16)v); /* round to nearest even */
   }
 };
 
@@ -73,29 +74,39 @@ struct Store<PFG_STORE_BF16> {
   __device__ static inline float load(const T *p) {
     return __builtin_bit_cast(float, ((uint32_t)*p) << 16);
   }
-  __device__ static inline void put(T *p, float v) {
+  __device__ static inline T pack(float v) {
     uint32_t u = __builtin_bit_cast(uint32_t, v);
     u += 0x7FFFu + ((u >> 16) & 1u); /* round to nearest even */
-    __builtin_nontemporal_store((uint16_t)(u >> 16), p);
+    return (uint16_t)(u >> 16);
   }
 };
 
-__device__ __host__ inline int64_t felem(int nxb, int ny, int d, int x, int y, int z) {
-  const int64_t b = (int64_t)(x >> 6) + (int64_t)nxb * (y + (int64_t)ny * z);
-  return (b * Q + d) * XBLOCK + (x & (XBLOCK - 1));
+/* Store value v; CACHED: through the caches, else streamed past them. */
+template <int S, bool CACHED>
+__device__ inline void put(typename Store<S>::T *p, float v) {
+  if (CACHED) *p = Store<S>::pack(v);
+  else __builtin_nontemporal_store(Store<S>::pack(v), p);
+}
+
+/* Element of direction d of cell i. */
+__device__ __host__ inline int64_t felem(int d, int64_t i) {
+  return ((i >> 6) * Q + d) * XBLOCK + (i & (XBLOCK - 1));
 }
 
 /* ---------------- the fused kernel ---------------- */
 
-/* STEP: every row, with the IB force in flagged tiles.  FIELDS: rho and u
- * only.  BULK / REGION: the rows whose stamp is not / is the current step
- * (rows that this step's IB stencils touch), without / with the IB force;
- * one z-row per wavefront. */
+/* STEP: every block, with the IB force in flagged tiles.  FIELDS: rho and u
+ * only.  BULK / REGION: the blocks whose stamp is not / is the current step
+ * (blocks that this step's IB stencils touch), without / with the IB force. */
 enum { LB_MODE_STEP = 0, LB_MODE_FIELDS = 1, LB_MODE_BULK = 2, LB_MODE_REGION = 3 };
 /* Flag bit of MODE: the lattice has velocity faces on z (compiled only into
  * the variant that needs it, which keeps the scalar registers and the
  * occupancy of the default kernels). */
 enum { LB_ZVEL = 4 };
+/* Flag bit of MODE: the new populations are stored through the caches (they
+ * fit the 256 MB cache in front of HBM together with the old ones, and the
+ * next step reads them from there); otherwise they are streamed past them. */
+enum { LB_CACHED = 8 };
 
 /* Velocity face z = 0 (s = +1) or z = nz-1 (s = -1) on the pulled
  * deviations (fluid3d_in_out_flow_boundary_kernel,
@@ -159,237 +170,252 @@ __device__ __forceinline__ void velocity_face(const LBArgs &a, int x, int y, int
   }
 }
 
-/* One wavefront per (x-block, y, CPT consecutive z); workgroup `blk` of the
- * lattice described by `a` (in memory that the whole workgroup reads), the
- * wavefront's place in it `wave` (default: its place in the launch's
- * workgroup). */
-template <int S, int CPT, int MODE>
-__device__ __forceinline__ void lb_update(const LBArgs &a, uint32_t blk, float *orho,
-                                          float *oux, float *ouy, float *ouz, int wave = -1) {
+/* The update of one cell from its pulled deviations: velocity face, moments,
+ * collision, stores (own: the cell's element of direction 0 in the new
+ * copy).  MODE as in lb_update. */
+template <int S, int MODE>
+__device__ __forceinline__ void lb_cell(const LBArgs &a, float (&dev)[Q], int x, int y, int z0,
+                                        int z1, int64_t idx, bool flagged, float ax, float ay,
+                                        float az, typename Store<S>::T *own, float *orho,
+                                        float *oux, float *ouy, float *ouz) {
   constexpr int M = MODE & 3;
-  constexpr bool ZV = (MODE & LB_ZVEL) != 0;
+  constexpr bool ZV = (MODE & LB_ZVEL) != 0, CACHED = (MODE & LB_CACHED) != 0;
+  using ST = Store<S>;
+  const float isc = ST::scaled ? a.inv_scale : 1.0f;
+  if (ZV && (z0 || z1)) velocity_face<ST>(a, x, y, z0 ? 1 : -1, dev);
+
+  /* moments: rho - 1 and momentum from deviations (sum_i w_i c_i = 0),
+   * over the nine pairs (d, opposite of d): the pair sum feeds the density,
+   * the pair difference the momentum.  -0.0f starts are exact no-ops. */
+  float drho = dev[0], jx = -0.0f, jy = -0.0f, jz = -0.0f;
+#pragma unroll
+  for (int d = 1; d < Q; ++d) {
+    if (d < BB[d]) {
+      const float s = dev[d] + dev[BB[d]], df = dev[d] - dev[BB[d]];
+      drho += s;
+      if (CX[d] > 0) jx += df; else if (CX[d] < 0) jx -= df;
+      if (CY[d] > 0) jy += df; else if (CY[d] < 0) jy -= df;
+      if (CZ[d] > 0) jz += df; else if (CZ[d] < 0) jz -= df;
+    }
+  }
+  if (ST::scaled) {
+    drho *= isc;
+    jx *= isc;
+    jy *= isc;
+    jz *= isc;
+  }
+  const float rho = 1.0f + drho;
+  float Fx = a.g[0], Fy = a.g[1], Fz = a.g[2];
+  if (flagged) {
+    Fx += ax;
+    Fy += ay;
+    Fz += az;
+  }
+  const float inv_rho = __builtin_amdgcn_rcpf(rho); /* hardware reciprocal, 1 ulp */
+  const float ux = (jx + 0.5f * Fx) * inv_rho;
+  const float uy = (jy + 0.5f * Fy) * inv_rho;
+  const float uz = (jz + 0.5f * Fz) * inv_rho;
+
+  if (M == LB_MODE_FIELDS) {
+    if (orho) orho[idx] = rho;
+    if (oux) oux[idx] = ux;
+    if (ouy) ouy[idx] = uy;
+    if (ouz) ouz[idx] = uz;
+    return;
+  }
+  if (flagged) { /* velocity for the IB interpolation of this step */
+    a.vel[idx] = make_float4(ux, uy, uz, 0.f);
+  }
+
+  /* BGK with Guo forcing, in deviation form and storage units:
+   *   out_d = (1-omega) dev_d + omega (feq_d - w_d) + guo w_d (3 (c_d-u).F + 9 (c_d.u)(c_d.F))
+   * split into the part even in c_d,
+   *   E = w_d [K0 + cu (4.5 omega rho cu + 9 guo cF)],
+   *   K0 = omega (drho - 1.5 rho u.u) - 3 guo u.F,
+   * and the odd part O = w_d (3 omega rho cu + 3 guo cF); the pair
+   * (d, opposite) takes E + O and E - O. */
+  const float usq = ux * ux + uy * uy + uz * uz;
+  const float uF = ux * Fx + uy * Fy + uz * Fz;
+  const float K0 = fmaf(-a.guo3, uF, a.omega * fmaf(-1.5f * rho, usq, drho));
+  const float Ab = a.om45 * rho, Cp = a.om3 * rho;
+  put<S, CACHED>(own, fmaf(a.keep, dev[0], a.ws[0] * K0));
+#pragma unroll
+  for (int d = 1; d < Q; ++d) {
+    if (d < BB[d]) {
+      const int k = d < 7 ? 1 : 2;
+      float cu = -0.0f, cF = -0.0f;
+      if (CX[d] > 0) { cu += ux; cF += Fx; } else if (CX[d] < 0) { cu -= ux; cF -= Fx; }
+      if (CY[d] > 0) { cu += uy; cF += Fy; } else if (CY[d] < 0) { cu -= uy; cF -= Fy; }
+      if (CZ[d] > 0) { cu += uz; cF += Fz; } else if (CZ[d] < 0) { cu -= uz; cF -= Fz; }
+      const float t = fmaf(a.gB[k], cF, (a.ws[k] * Ab) * cu);
+      const float E = fmaf(cu, t, a.ws[k] * K0);
+      const float O = fmaf(a.gD[k], cF, (a.ws[k] * Cp) * cu);
+      put<S, CACHED>(own + d * XBLOCK, fmaf(a.keep, dev[d], E + O));
+      put<S, CACHED>(own + BB[d] * XBLOCK, fmaf(a.keep, dev[BB[d]], E - O));
+    }
+  }
+}
+
+/* One wavefront per block of 64 cells; workgroup `blk` of the lattice
+ * described by `a` (in memory that the whole workgroup reads), the
+ * wavefront's place in it `wave` (default: its place in the launch's
+ * workgroup); cells outside [lo, hi) are left alone (field windows).
+ *
+ * Bound by HBM.  What keeps it there: a lane decodes its own (x, y, z) from
+ * the wavefront's first cell (64 cells meet few rows) and adds per-axis
+ * offsets, periodic wraps included, to its cell index, about 100 integer
+ * instructions that need no load; every load that does not depend on another
+ * (the tile stamp, the 19 populations) is issued before the first is waited
+ * for; the stamped tiles' force loads follow while the populations are in
+ * flight.  Against a kernel whose wavefronts took 64-cell blocks of whole
+ * rows from wavefront-uniform addresses (LB-only launches, us): 256 lattices
+ * of 32 to 96 cells per axis FP32 2540 -> 1800, FP16 1970 -> 1010; 201x99x75
+ * FP32 45 -> 30; 128^3 FP16 41 -> 26; 256x128x128 FP16 64 -> 55, FP32
+ * 109 -> 108; 1024x512x512 FP16 3600 -> 3330, FP32 6780 -> 6720; a 512x256x256
+ * tube with solid cells FP32 632 -> 587, FP16 342 -> 294. */
+template <int S, int MODE>
+__device__ __forceinline__ void lb_update(const LBArgs &a, uint32_t blk, float *orho,
+                                          float *oux, float *ouy, float *ouz, int wave = -1,
+                                          uint32_t lo = 0, uint32_t hi = ~0u) {
+  constexpr int M = MODE & 3;
   using ST = Store<S>;
   using T = typename ST::T;
-  constexpr int R = Q * XBLOCK; /* values per x-block */
+  constexpr uint32_t R = Q * XBLOCK; /* values per block */
   const T *__restrict__ fin = (const T *)a.fin;
   T *__restrict__ fout = (T *)a.fout;
   if (M != LB_MODE_FIELDS && a.halt != nullptr && *a.halt != 0) return;
-  const int lane = threadIdx.x & (XBLOCK - 1);
-  /* wavefront-uniform task decomposition in 32-bit arithmetic (x-blocks per
-   * lattice stay below 2^31) */
   const uint32_t task =
       blk * 4u + __builtin_amdgcn_readfirstlane(wave < 0 ? (int)(threadIdx.x >> 6) : wave);
-  const uint32_t rows = (uint32_t)a.nxb * (uint32_t)a.ny;
-  const uint32_t zc = task / rows;
-  if (zc * CPT >= (uint32_t)a.nz) return;
-  /* IB force tiles and rows are stamped with the step that touches them */
+  const uint32_t i0 = task * XBLOCK;
+  if (i0 >= a.ncell) return;
+  /* IB force tiles and blocks are stamped with the step that touches them */
   const int32_t step32 = M == LB_MODE_FIELDS ? 0 : (int32_t)*a.step;
   if (M == LB_MODE_BULK || M == LB_MODE_REGION) {
-    static_assert(M < LB_MODE_BULK || CPT == 1, "row modes update one z-row per wave");
-    const bool touched = a.row_stamp[task] == step32; /* task = x-block row */
+    const bool touched = a.row_stamp[task] == step32;
     if (touched != (M == LB_MODE_REGION)) return;
   }
-  const uint32_t rem = task - zc * rows;
-  const int y = (int)(rem / (uint32_t)a.nxb);
-  const int xb = (int)(rem - (uint32_t)y * a.nxb);
-  const int x = xb * XBLOCK + lane;
-  if (x >= a.nx) return;
-
-  /* lane offsets from the upstream chunk base (placed one block early, so all
-   * offsets are >= 0): centre, upstream x-1, upstream x+1.  Lanes at the ends
-   * of the row take their x-neighbour in the edge pass below. */
-  const bool xlo = x == 0, xhi = x == a.nx - 1;
-  const uint32_t o_c = R + lane;
-  const uint32_t o_m = xlo ? o_c : (lane > 0 ? R + lane - 1 : XBLOCK - 1);
-  const uint32_t o_p = xhi ? o_c : (lane < XBLOCK - 1 ? R + lane + 1 : 2 * R);
-
-  /* upstream rows, wavefront-uniform */
-  const int y0 = y == 0, y1 = y == a.ny - 1;
-  const int ym = y0 ? (a.periodic[1] ? a.ny - 1 : y) : y - 1;
-  const int yp = y1 ? (a.periodic[1] ? 0 : y) : y + 1;
-  const bool oym = y0 && !a.periodic[1], oyp = y1 && !a.periodic[1];
-
-  const float isc = ST::scaled ? a.inv_scale : 1.0f;
-
+  const int kind = a.block_kind != nullptr ? a.block_kind[task] : BLOCK_FLUID;
+  if (kind == BLOCK_SOLID) return;
+  const uint32_t lane = threadIdx.x & (XBLOCK - 1);
+  const uint32_t i = i0 + lane;
+  if (i < lo || i >= hi || i >= a.ncell) return;
+  uint32_t mask = 0;
+  if (kind == BLOCK_MIXED) {
+    mask = a.bbmask[i];
+    if (mask >> 31) return; /* solid cell */
+  }
+  const uint32_t nx = (uint32_t)a.nx, ny = (uint32_t)a.ny, nxy = nx * ny;
+  const uint32_t wz = i0 / nxy, wr = i0 - wz * nxy, wy = wr / nx, wx = wr - wy * nx;
+  /* rows and planes passed since the wavefront's first cell: at most one of a
+   * row longer than the wavefront; shorter ones by the reciprocal (v < 128,
+   * and (v + 1/2) / n is at least 1/128 from an integer) */
+  const uint32_t vx = wx + lane;
+  const uint32_t qy = nx > XBLOCK ? (vx >= nx ? 1u : 0u)
+                                  : (uint32_t)(((float)vx + 0.5f) * a.inv_nx);
+  const uint32_t vy = wy + qy;
+  const uint32_t qz = ny > XBLOCK ? (vy >= ny ? 1u : 0u)
+                                  : (uint32_t)(((float)vy + 0.5f) * a.inv_ny);
+  const int x = (int)(vx - qy * nx), y = (int)(vy - qz * ny), z = (int)(wz + qz);
+  int32_t stamp = 0;
+  if (M == LB_MODE_STEP || M == LB_MODE_REGION)
+    stamp = a.tile_stamp[(x >> TILE_SHIFT_X) +
+                         a.tnx * ((y >> TILE_SHIFT_Y) + a.tny * (z >> TILE_SHIFT_Z))];
+  /* offset to the upstream neighbour along each axis, 0 outside a wall (the
+   * edge pass replaces what that reads) */
+  const bool xlo = x == 0, xhi = x == a.nx - 1, ylo = y == 0, yhi = y == a.ny - 1,
+             zlo = z == 0, zhi = z == a.nz - 1;
+  const bool oxm = xlo && !a.periodic[0], oxp = xhi && !a.periodic[0];
+  const bool oym = ylo && !a.periodic[1], oyp = yhi && !a.periodic[1];
+  const bool ozm = zlo && !a.periodic[2], ozp = zhi && !a.periodic[2];
+  const int sx = a.nx, sy = (int)nxy, sz = (int)a.ncell;
+  const int xm = xlo ? (oxm ? 0 : sx - 1) : -1, xp = xhi ? (oxp ? 0 : 1 - sx) : 1;
+  const int ym = ylo ? (oym ? 0 : sy - sx) : -sx, yp = yhi ? (oyp ? 0 : sx - sy) : sx;
+  const int zm = zlo ? (ozm ? 0 : sz - sy) : -sy, zp = zhi ? (ozp ? 0 : sy - sz) : sy;
+  float dev[Q];
 #pragma unroll
-  for (int c = 0; c < CPT; ++c) {
-    const int z = zc * CPT + c;
-    if (z >= a.nz) return;
-    const int64_t idx = x + (int64_t)a.nx * (y + (int64_t)a.ny * z); /* cell index */
-    uint32_t mask = 0;
-    if (a.bbmask != nullptr) {
-      mask = a.bbmask[idx];
-      if (mask >> 31) continue; /* solid cell */
-    }
-    const int z0 = z == 0, z1 = z == a.nz - 1;
-    const int zm = z0 ? (a.periodic[2] ? a.nz - 1 : z) : z - 1;
-    const int zp = z1 ? (a.periodic[2] ? 0 : z) : z + 1;
-    const bool ozm = z0 && !a.periodic[2], ozp = z1 && !a.periodic[2];
-    const uint64_t bown = (uint32_t)xb + (uint32_t)a.nxb * (uint32_t)(y + a.ny * z);
-
-    /* the IB force of the tiles this step's stencils meet, read (and
-     * consumed: the next step's spreading adds into zeros) before the
-     * populations, so that its latency overlaps theirs */
-    bool flagged = false;
-    float ax = 0.f, ay = 0.f, az = 0.f;
-    if (M == LB_MODE_STEP || M == LB_MODE_REGION) {
-      const int tile = (x >> TILE_SHIFT_X) + a.tnx * ((y >> TILE_SHIFT_Y) + a.tny * (z >> TILE_SHIFT_Z));
-      flagged = a.tile_stamp[tile] == step32;
-      if (flagged) {
-        ax = a.aux[idx];
-        ay = a.aux[a.plane + idx];
-        az = a.aux[2 * a.plane + idx];
-        a.aux[idx] = 0.f;
-        a.aux[a.plane + idx] = 0.f;
-        a.aux[2 * a.plane + idx] = 0.f;
-      }
-    }
-
-    float dev[Q];
-#pragma unroll
-    for (int d = 0; d < Q; ++d) {
-      const int sy = CY[d] > 0 ? ym : (CY[d] < 0 ? yp : y);
-      const int sz = CZ[d] > 0 ? zm : (CZ[d] < 0 ? zp : z);
-      const uint64_t bsrc = (uint32_t)xb + (uint32_t)a.nxb * (uint32_t)(sy + a.ny * sz);
-      const T *base = fin + ((int64_t)(bsrc * Q + d) * XBLOCK - R);
-      const uint32_t o = CX[d] > 0 ? o_m : (CX[d] < 0 ? o_p : o_c);
-      dev[d] = ST::load(base + o);
-    }
-    /* edge pass: rows next to a wall (wavefront-uniform), row ends, solid
-     * neighbours.  Upstream cell outside a wall or solid: halfway bounce-back,
-     * the population leaving this cell returns plus the moving-wall momentum
-     * 6 w (c . u_wall) (z wall over y wall over x wall); otherwise the
-     * periodic x-neighbour. */
-    const bool edge = xlo || xhi || oym || oyp || ozm || ozp || mask != 0;
-    if (edge) {
-#pragma unroll
-      for (int d = 1; d < Q; ++d) {
-        const bool oz = CZ[d] > 0 ? ozm : (CZ[d] < 0 ? ozp : false);
-        const bool oy = CY[d] > 0 ? oym : (CY[d] < 0 ? oyp : false);
-        const bool xe = CX[d] > 0 ? xlo : (CX[d] < 0 ? xhi : false);
-        const bool ox = xe && !a.periodic[0];
-        if (oz || oy || ox || ((mask >> d) & 1u)) {
-          const int sxs = CX[d] > 0 ? 0 : 1, sys = CY[d] > 0 ? 0 : 1, szs = CZ[d] > 0 ? 0 : 1;
-          const float term = oz ? a.wall_term[2][szs][d]
-                                : (oy ? a.wall_term[1][sys][d] : (ox ? a.wall_term[0][sxs][d] : 0.f));
-          dev[d] = ST::load(fin + (bown * Q + BB[d]) * XBLOCK + lane) + term;
-        } else if (xe) { /* periodic wrap along x */
-          const int sx = CX[d] > 0 ? a.nx - 1 : 0;
-          const int sy = CY[d] > 0 ? ym : (CY[d] < 0 ? yp : y);
-          const int sz = CZ[d] > 0 ? zm : (CZ[d] < 0 ? zp : z);
-          dev[d] = ST::load(fin + felem(a.nxb, a.ny, d, sx, sy, sz));
-        }
-      }
-    }
-    if (ZV && (z0 || z1)) velocity_face<ST>(a, x, y, z0 ? 1 : -1, dev);
-
-    /* moments: rho - 1 and momentum from deviations (sum_i w_i c_i = 0),
-     * over the nine pairs (d, opposite of d): the pair sum feeds the density,
-     * the pair difference the momentum.  -0.0f starts are exact no-ops. */
-    float drho = dev[0], jx = -0.0f, jy = -0.0f, jz = -0.0f;
-#pragma unroll
-    for (int d = 1; d < Q; ++d) {
-      if (d < BB[d]) {
-        const float s = dev[d] + dev[BB[d]], df = dev[d] - dev[BB[d]];
-        drho += s;
-        if (CX[d] > 0) jx += df; else if (CX[d] < 0) jx -= df;
-        if (CY[d] > 0) jy += df; else if (CY[d] < 0) jy -= df;
-        if (CZ[d] > 0) jz += df; else if (CZ[d] < 0) jz -= df;
-      }
-    }
-    if (ST::scaled) {
-      drho *= isc;
-      jx *= isc;
-      jy *= isc;
-      jz *= isc;
-    }
-    const float rho = 1.0f + drho;
-    float Fx = a.g[0], Fy = a.g[1], Fz = a.g[2];
+  for (int d = 0; d < Q; ++d) {
+    const int off = (CX[d] > 0 ? xm : (CX[d] < 0 ? xp : 0)) +
+                    (CY[d] > 0 ? ym : (CY[d] < 0 ? yp : 0)) +
+                    (CZ[d] > 0 ? zm : (CZ[d] < 0 ? zp : 0));
+    const uint32_t src = i + (uint32_t)off;
+    dev[d] = ST::load(fin + d * XBLOCK + ((uint64_t)(src >> 6) * R + (src & (XBLOCK - 1))));
+  }
+  /* the IB force of the tiles this step's stencils meet, read and consumed
+   * (the next step's spreading adds into zeros) */
+  bool flagged = false;
+  float ax = 0.f, ay = 0.f, az = 0.f;
+  if (M == LB_MODE_STEP || M == LB_MODE_REGION) {
+    flagged = stamp == step32;
     if (flagged) {
-      Fx += ax;
-      Fy += ay;
-      Fz += az;
+      ax = a.aux[i];
+      ay = a.aux[a.plane + i];
+      az = a.aux[2 * a.plane + i];
+      a.aux[i] = 0.f;
+      a.aux[a.plane + i] = 0.f;
+      a.aux[2 * a.plane + i] = 0.f;
     }
-    const float inv_rho = __builtin_amdgcn_rcpf(rho); /* hardware reciprocal, 1 ulp */
-    const float ux = (jx + 0.5f * Fx) * inv_rho;
-    const float uy = (jy + 0.5f * Fy) * inv_rho;
-    const float uz = (jz + 0.5f * Fz) * inv_rho;
-
-    if (M == LB_MODE_FIELDS) {
-      if (orho) orho[idx] = rho;
-      if (oux) oux[idx] = ux;
-      if (ouy) ouy[idx] = uy;
-      if (ouz) ouz[idx] = uz;
-      continue;
-    }
-    if (flagged) { /* velocity for the IB interpolation of this step */
-      a.vel[idx] = make_float4(ux, uy, uz, 0.f);
-    }
-
-    /* BGK with Guo forcing, in deviation form and storage units:
-     *   out_d = (1-omega) dev_d + omega (feq_d - w_d) + guo w_d (3 (c_d-u).F + 9 (c_d.u)(c_d.F))
-     * split into the part even in c_d,
-     *   E = w_d [K0 + cu (4.5 omega rho cu + 9 guo cF)],
-     *   K0 = omega (drho - 1.5 rho u.u) - 3 guo u.F,
-     * and the odd part O = w_d (3 omega rho cu + 3 guo cF); the pair
-     * (d, opposite) takes E + O and E - O. */
-    const float usq = ux * ux + uy * uy + uz * uz;
-    const float uF = ux * Fx + uy * Fy + uz * Fz;
-    const float K0 = fmaf(-a.guo3, uF, a.omega * fmaf(-1.5f * rho, usq, drho));
-    const float Ab = a.om45 * rho, Cp = a.om3 * rho;
-    T *own = fout + bown * R + lane;
-    ST::put(own, fmaf(a.keep, dev[0], a.ws[0] * K0));
+  }
+  /* edge pass: upstream cell outside a wall or solid: halfway bounce-back,
+   * the population leaving this cell returns plus the moving-wall momentum
+   * 6 w (c . u_wall) (z wall over y wall over x wall). */
+  const uint64_t own = (uint64_t)task * R + lane;
+  if (oxm || oxp || oym || oyp || ozm || ozp || mask != 0) {
 #pragma unroll
     for (int d = 1; d < Q; ++d) {
-      if (d < BB[d]) {
-        const int k = d < 7 ? 1 : 2;
-        float cu = -0.0f, cF = -0.0f;
-        if (CX[d] > 0) { cu += ux; cF += Fx; } else if (CX[d] < 0) { cu -= ux; cF -= Fx; }
-        if (CY[d] > 0) { cu += uy; cF += Fy; } else if (CY[d] < 0) { cu -= uy; cF -= Fy; }
-        if (CZ[d] > 0) { cu += uz; cF += Fz; } else if (CZ[d] < 0) { cu -= uz; cF -= Fz; }
-        const float t = fmaf(a.gB[k], cF, (a.ws[k] * Ab) * cu);
-        const float E = fmaf(cu, t, a.ws[k] * K0);
-        const float O = fmaf(a.gD[k], cF, (a.ws[k] * Cp) * cu);
-        ST::put(own + d * XBLOCK, fmaf(a.keep, dev[d], E + O));
-        ST::put(own + BB[d] * XBLOCK, fmaf(a.keep, dev[BB[d]], E - O));
+      const bool oz = CZ[d] > 0 ? ozm : (CZ[d] < 0 ? ozp : false);
+      const bool oy = CY[d] > 0 ? oym : (CY[d] < 0 ? oyp : false);
+      const bool ox = CX[d] > 0 ? oxm : (CX[d] < 0 ? oxp : false);
+      if (oz || oy || ox || ((mask >> d) & 1u)) {
+        const int sxs = CX[d] > 0 ? 0 : 1, sys = CY[d] > 0 ? 0 : 1, szs = CZ[d] > 0 ? 0 : 1;
+        const float term = oz ? a.wall_term[2][szs][d]
+                              : (oy ? a.wall_term[1][sys][d] : (ox ? a.wall_term[0][sxs][d] : 0.f));
+        dev[d] = ST::load(fin + own + BB[d] * XBLOCK) + term;
       }
     }
   }
+  lb_cell<S, MODE>(a, dev, x, y, zlo, zhi, i, flagged, ax, ay, az, fout + own, orho, oux, ouy,
+                   ouz);
 }
 
-template <int S, int CPT, int MODE>
-__global__ __launch_bounds__(256) void lb_fused_kernel(LBArgs a, float *orho, float *oux,
-                                                       float *ouy, float *ouz) {
-  /* Workgroups are dealt round-robin to the 8 XCDs.  With xcd_rows each
-   * XCD takes a contiguous range of rows instead, so that neighbouring rows
-   * (which read each other's populations) share its L2; the autotuner picks
-   * the order (faster on large lattices, slower on small ones). */
-  uint32_t blk = blockIdx.x;
-  if (a.xcd_rows) {
-    const uint32_t q = gridDim.x / 8u;
-    if (blk < 8u * q) blk = (blk % 8u) * q + blk / 8u;
-  }
-  lb_update<S, CPT, MODE>(a, blk, orho, oux, ouy, ouz);
-}
-
-/* A batch of lattices in one launch: workgroup -> lattice through a table,
- * each lattice's arguments read from device memory.  xcd_rows: each XCD
- * takes a contiguous range of the table (as in the single-lattice kernel). */
-template <int S, int CPT, int MODE>
-__global__ __launch_bounds__(256) void lb_batch_kernel(const LBArgs *args,
-                                                       const int32_t *block_inst,
-                                                       int xcd_rows) {
+/* Workgroups are dealt round-robin to the 8 XCDs.  With xcd_rows each XCD
+ * takes a contiguous range of blocks instead, so that neighbouring blocks
+ * (which read each other's populations) share its L2; the autotuner picks
+ * the order. */
+__device__ inline uint32_t launch_block(int xcd_rows) {
   uint32_t blk = blockIdx.x;
   if (xcd_rows) {
     const uint32_t q = gridDim.x / 8u;
     if (blk < 8u * q) blk = (blk % 8u) * q + blk / 8u;
   }
-  const LBArgs &a = args[block_inst[blk]];
-  lb_update<S, CPT, MODE>(a, (uint32_t)(blk - a.block0), nullptr, nullptr, nullptr, nullptr);
+  return blk;
+}
+
+/* CPT: cells per lane, from blocks that follow each other.  WAVES: the
+ * wavefronts a SIMD holds at most. */
+template <int S, int CPT, int MODE, int WAVES>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void
+lb_fused_kernel(LBArgs a, float *orho, float *oux, float *ouy, float *ouz) {
+  const uint32_t blk = launch_block(a.xcd_rows) * CPT;
+  for (uint32_t c = 0; c < CPT; ++c) lb_update<S, MODE>(a, blk + c, orho, oux, ouy, ouz);
+}
+
+/* A batch of lattices in one launch: workgroup task -> lattice through a
+ * table of ntasks entries, each lattice's arguments read from device
+ * memory. */
+template <int S, int CPT, int MODE>
+__global__ __launch_bounds__(256) void lb_batch_kernel(const LBArgs *args,
+                                                       const int32_t *block_inst,
+                                                       uint32_t ntasks, int xcd_rows) {
+  const uint32_t blk = launch_block(xcd_rows) * CPT;
+  for (uint32_t c = 0; c < CPT; ++c) {
+    if (CPT > 1 && blk + c >= ntasks) return;
+    const LBArgs &a = args[block_inst[blk + c]];
+    lb_update<S, MODE>(a, (uint32_t)(blk + c - a.block0), nullptr, nullptr, nullptr, nullptr);
+  }
 }
 
 /* A batch of lattices in one persistent launch: a grid of resident
- * workgroups whose wavefronts take the table's x-block rows (of any
+ * workgroups whose wavefronts take the table's blocks (of any
  * lattice; row r is wavefront r % 4 of workgroup task r / 4) from a device
  * work queue until it is empty.  The rows are cut into LB_QUEUES contiguous
  * ranges, one per XCD (the hardware deals workgroup w to XCD w % 8), each
@@ -400,7 +426,7 @@ __global__ __launch_bounds__(256) void lb_batch_kernel(const LBArgs *args,
  * that are done; the last one resets every counter for the next launch (all
  * others have made their last grab by then), so a captured step needs no
  * clearing node. */
-template <int S, int CPT, int MODE>
+template <int S, int MODE>
 __global__ __launch_bounds__(256) void lb_batch_queue_kernel(const LBArgs *args,
                                                              const int32_t *block_inst,
                                                              uint32_t ntasks, uint32_t *queue) {
@@ -421,7 +447,7 @@ __global__ __launch_bounds__(256) void lb_batch_queue_kernel(const LBArgs *args,
       for (uint32_t row = t0; row < t1; ++row) {
         const uint32_t blk = row >> 2;
         const LBArgs &a = args[block_inst[blk]];
-        lb_update<S, CPT, MODE>(a, (uint32_t)(blk - a.block0), nullptr, nullptr, nullptr,
+        lb_update<S, MODE>(a, (uint32_t)(blk - a.block0), nullptr, nullptr, nullptr,
                                 nullptr, (int)(row & 3u));
       }
     }
@@ -442,18 +468,19 @@ __global__ __launch_bounds__(256) void lb_batch_queue_kernel(const LBArgs *args,
  * process ends; calls on one device share it. */
 static __device__ __align__(256) float scratch[FIELDS_SCRATCH_FLOATS];
 
-/* The fields pass over the x-block rows [t0, t1) (the rows of z-planes
- * [z0, z1)), one wavefront per row; o* point at cell 0 of the window's first
+/* The fields pass over the blocks [t0, t1) that hold the cells [lo, hi) of
+ * z-planes [z0, z1), one wavefront per block; o* point at cell 0 of the window's first
  * plane minus z0 planes, so that each cell lands at its offset in the window. */
 template <int S>
 __global__ __launch_bounds__(256) void lb_fields_window_kernel(LBArgs a, uint32_t blk0,
                                                                uint32_t t0, uint32_t t1,
+                                                               uint32_t lo, uint32_t hi,
                                                                float *orho, float *oux,
                                                                float *ouy, float *ouz) {
   const uint32_t blk = blk0 + blockIdx.x;
   const uint32_t task = blk * 4u + (threadIdx.x >> 6);
   if (task < t0 || task >= t1) return;
-  lb_update<S, 1, LB_MODE_FIELDS>(a, blk, orho, oux, ouy, ouz);
+  lb_update<S, LB_MODE_FIELDS>(a, blk, orho, oux, ouy, ouz, -1, lo, hi);
 }
 
 __global__ __launch_bounds__(256) void fill_zero_kernel(float *p, int64_t n) {
@@ -489,13 +516,13 @@ template <int S>
 static hipError_t fields_window_s(pfg_handle *h, const LBArgs &a, int z0, int z1,
                                   float *const win[4]) {
   const int64_t plane = (int64_t)a.nx * a.ny;
-  const uint32_t rows = (uint32_t)a.nxb * (uint32_t)a.ny;
-  const uint32_t t0 = (uint32_t)z0 * rows, t1 = (uint32_t)z1 * rows;
+  const uint32_t lo = (uint32_t)(plane * z0), hi = (uint32_t)(plane * z1);
+  const uint32_t t0 = lo / XBLOCK, t1 = (hi + XBLOCK - 1u) / XBLOCK;
   const uint32_t blk0 = t0 / 4u, blk1 = (t1 + 3u) / 4u;
   float *o[4];
   for (int c = 0; c < 4; ++c) o[c] = win[c] ? win[c] - (int64_t)z0 * plane : nullptr;
   hipLaunchKernelGGL(lb_fields_window_kernel<S>, dim3(blk1 - blk0), dim3(256), 0, h->stream, a,
-                     blk0, t0, t1, o[0], o[1], o[2], o[3]);
+                     blk0, t0, t1, lo, hi, o[0], o[1], o[2], o[3]);
   return hipGetLastError();
 }
 
@@ -568,10 +595,17 @@ __global__ void bbmask_kernel(LBArgs a, const uint8_t *solid, uint32_t *mask) {
   mask[idx] = m;
 }
 
-__device__ inline void cell_xyz(const LBArgs &a, int64_t idx, int &x, int &y, int &z) {
-  x = (int)(idx % a.nx);
-  y = (int)((idx / a.nx) % a.ny);
-  z = (int)(idx / ((int64_t)a.nx * a.ny));
+/* Kind of each block, from its cells' masks: a wavefront per block.  The
+ * update reads masks in mixed blocks only and leaves solid ones at once. */
+__global__ __launch_bounds__(256) void block_kind_kernel(const uint32_t *mask, uint32_t ncell,
+                                                         int32_t *kind) {
+  const uint32_t task = blockIdx.x * 4u + (threadIdx.x >> 6);
+  const uint32_t i = task * XBLOCK + (threadIdx.x & 63);
+  if (task * XBLOCK >= ncell) return;
+  const uint32_t m = i < ncell ? mask[i] : 0u;
+  const uint64_t in = __ballot(i < ncell), any = __ballot(m != 0), solid = __ballot(m >> 31);
+  if ((threadIdx.x & 63) == 0)
+    kind[task] = solid == in ? BLOCK_SOLID : (any != 0 ? BLOCK_MIXED : BLOCK_FLUID);
 }
 
 /* per_z: the inputs hold one value per z-plane (a velocity that varies
@@ -585,9 +619,7 @@ __global__ void init_eq_kernel(LBArgs a, void *dst0, void *dst1, const float *rh
   using T = typename ST::T;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= n) return;
-  int x, y, z;
-  cell_xyz(a, idx, x, y, z);
-  const int64_t src = per_z ? (int64_t)z : idx;
+  const int64_t src = per_z ? idx / ((int64_t)a.nx * a.ny) : idx;
   const float rho = rho_in ? rho_in[src] : 1.0f;
   const float ux = ux_in ? ux_in[src] : 0.f;
   const float uy = uy_in ? uy_in[src] : 0.f;
@@ -600,9 +632,9 @@ __global__ void init_eq_kernel(LBArgs a, void *dst0, void *dst1, const float *rh
     const float w = weight(d);
     const float cu = CX[d] * ux + CY[d] * uy + CZ[d] * uz;
     const float dev = w * drho + w * rho * (3.0f * cu + 4.5f * cu * cu - usq15);
-    const int64_t e = felem(a.nxb, a.ny, d, x, y, z);
-    ST::put((T *)dst0 + e, dev * sc);
-    ST::put((T *)dst1 + e, dev * sc);
+    const int64_t e = felem(d, idx);
+    put<S, false>((T *)dst0 + e, dev * sc);
+    put<S, false>((T *)dst1 + e, dev * sc);
   }
 }
 
@@ -614,14 +646,12 @@ __global__ void convert_plane_kernel(LBArgs a, void *stored, float *buf, int d, 
   using T = typename ST::T;
   const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (idx >= n) return;
-  int x, y, z;
-  cell_xyz(a, idx, x, y, z);
-  T *p = (T *)stored + felem(a.nxb, a.ny, d, x, y, z);
+  T *p = (T *)stored + felem(d, idx);
   const float w = weight(d);
   if (to_float) {
     buf[idx] = w + ST::load(p) * (ST::scaled ? a.inv_scale : 1.0f);
   } else {
-    ST::put(p, (buf[idx] - w) * (ST::scaled ? a.scale : 1.0f));
+    put<S, false>(p, (buf[idx] - w) * (ST::scaled ? a.scale : 1.0f));
   }
 }
 
@@ -637,9 +667,7 @@ __global__ __launch_bounds__(256) void conservation_kernel(LBArgs a, const void 
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
        idx += (int64_t)gridDim.x * blockDim.x) {
     if (a.solid != nullptr && a.solid[idx]) continue;
-    int x, y, z;
-    cell_xyz(a, idx, x, y, z);
-    const int64_t e0 = felem(a.nxb, a.ny, 0, x, y, z);
+    const int64_t e0 = felem(0, idx);
     double cm = 0, cx = 0, cy = 0, cz = 0;
 #pragma unroll
     for (int d = 0; d < Q; ++d) {
@@ -674,6 +702,17 @@ __global__ __launch_bounds__(256) void conservation_kernel(LBArgs a, const void 
 
 /* ---------------- host launchers ---------------- */
 
+/* Both copies of the populations, in bytes. */
+static int64_t lb_bytes(const pfg_handle *h) {
+  return 2 * (h->inst.back().fblk0 + h->inst.back().nfblk) * Q * XBLOCK * (int64_t)h->esize;
+}
+
+static bool lb_cached(const pfg_handle *h) { return lb_bytes(h) <= LB_CACHED_MAX_BYTES; }
+
+int lb_default_xcd_rows(const pfg_handle *h) {
+  return lb_bytes(h) <= LB_XCD_MAX_BYTES || (h->K == 1 && h->N >= LB_LARGE_CELLS) ? 1 : 0;
+}
+
 /* Arguments of lattice k of the handle, starting from copy `cur` of f. */
 void make_lb_args(const pfg_handle *h, int k, int cur, LBArgs *a) {
   const Inst &L = h->inst[(size_t)k];
@@ -693,7 +732,10 @@ void make_lb_args(const pfg_handle *h, int k, int cur, LBArgs *a) {
   a->nx = p.nx;
   a->ny = p.ny;
   a->nz = p.nz;
-  a->nxb = L.nxb;
+  a->block_kind = h->block_kind ? h->block_kind + L.fblk0 : nullptr;
+  a->ncell = (uint32_t)L.N;
+  a->inv_nx = 1.0f / (float)p.nx;
+  a->inv_ny = 1.0f / (float)p.ny;
   a->block0 = L.lb_block0;
   a->tnx = L.tnx;
   a->tny = L.tny;
@@ -737,44 +779,51 @@ void make_lb_args(const pfg_handle *h, int k, int cur, LBArgs *a) {
   }
 }
 
-template <int S, int CPT, int MODE>
-static void launch_fused(const LBArgs &a, dim3 grid, float *rho, float *ux, float *uy,
-                         float *uz, hipStream_t st) {
+template <int S, int CPT, int MODE, int WAVES>
+static hipError_t launch_fused(const LBArgs &a, float *rho, float *ux, float *uy, float *uz,
+                               hipStream_t st) {
+  constexpr int PER = 4 * XBLOCK * CPT; /* cells per workgroup */
+  const dim3 grid((unsigned)(((int64_t)a.ncell + PER - 1) / PER));
   if (a.zvel)
-    hipLaunchKernelGGL((lb_fused_kernel<S, CPT, MODE | LB_ZVEL>), grid, dim3(256), 0, st, a,
+    hipLaunchKernelGGL((lb_fused_kernel<S, CPT, MODE | LB_ZVEL, WAVES>), grid, dim3(256), 0, st, a,
                        rho, ux, uy, uz);
   else
-    hipLaunchKernelGGL((lb_fused_kernel<S, CPT, MODE>), grid, dim3(256), 0, st, a, rho, ux,
+    hipLaunchKernelGGL((lb_fused_kernel<S, CPT, MODE, WAVES>), grid, dim3(256), 0, st, a, rho, ux,
                        uy, uz);
-}
-
-template <int S, int CPT>
-static hipError_t launch_lb_t(pfg_handle *h, const LBArgs &a, int mode, float *rho,
-                              float *ux, float *uy, float *uz, hipStream_t st) {
-  const int64_t waves = (int64_t)a.nxb * a.ny * ((a.nz + CPT - 1) / CPT);
-  const dim3 grid((unsigned)((waves + 3) / 4));
-  if (mode == LB_MODE_STEP)
-    launch_fused<S, CPT, LB_MODE_STEP>(a, grid, nullptr, nullptr, nullptr, nullptr, st);
-  else if (mode == LB_MODE_FIELDS)
-    launch_fused<S, CPT, LB_MODE_FIELDS>(a, grid, rho, ux, uy, uz, st);
-  else if (CPT != 1)
-    return hipErrorInvalidValue;
-  else if (mode == LB_MODE_BULK)
-    launch_fused<S, 1, LB_MODE_BULK>(a, grid, nullptr, nullptr, nullptr, nullptr, st);
-  else
-    launch_fused<S, 1, LB_MODE_REGION>(a, grid, nullptr, nullptr, nullptr, nullptr, st);
   return hipGetLastError();
 }
 
+/* Which variant a step takes (LB-only launches, us, on the same box):
+ * - Both copies within LB_CACHED_MAX_BYTES: stores through the caches, the
+ *   next step then reads from the 256 MB cache in front of HBM.  Streamed /
+ *   cached: 201x99x75 FP32 (226 MB) 43 / 34, 128^3 FP16 (160 MB) 30.6 / 26,
+ *   128^3 FP32 and 256x128x128 FP16 (319 MB) 56 / 52 and 55.7 / 54, but
+ *   160x128x128 FP32 (398 MB) 70 / 72, 200^3 FP16 (608 MB) 102 / 107.
+ * - XCD order (lb_default_xcd_rows) where they fit that cache, each XCD's
+ *   range then mostly its own L2's: hardware / XCD order 201x99x75 FP32
+ *   34 / 30, 150x75x67 19.3 / 17.2, but 256x128x128 108 / 114; and from
+ *   LB_LARGE_CELLS up, where the order keeps the reads of neighbouring planes
+ *   in one L2: 1024x512x512 FP32 7350 / 6720, FP16 3370 / 3330.
+ * - Wavefronts per SIMD: fewer resident wavefronts walk fewer DRAM pages at
+ *   once.  8 / 6 / 4: FP32 512x256x256 896 / 890 / 868, its tube 630 / 631 /
+ *   587; 1024x512x512 FP32 7150 / 6700 / 6690, FP16 3510 / 3330 / 3560,
+ *   FP16 512x256x256 427 / 415 / 431. */
 template <int S>
-static hipError_t launch_lb_s(pfg_handle *h, const LBArgs &a, int mode, float *rho, float *ux,
-                              float *uy, float *uz, hipStream_t st) {
-  const int cpt = mode >= LB_MODE_BULK ? 1 : h->lb_cpt;
-  switch (cpt) {
-    case 2: return launch_lb_t<S, 2>(h, a, mode, rho, ux, uy, uz, st);
-    case 4: return launch_lb_t<S, 4>(h, a, mode, rho, ux, uy, uz, st);
-    default: return launch_lb_t<S, 1>(h, a, mode, rho, ux, uy, uz, st);
+static hipError_t launch_lb_s(const pfg_handle *h, const LBArgs &a, int mode, float *rho,
+                              float *ux, float *uy, float *uz, hipStream_t st) {
+  switch (mode) {
+    case LB_MODE_FIELDS: return launch_fused<S, 1, LB_MODE_FIELDS, 6>(a, rho, ux, uy, uz, st);
+    case LB_MODE_BULK: return launch_fused<S, 1, LB_MODE_BULK, 6>(a, rho, ux, uy, uz, st);
+    case LB_MODE_REGION: return launch_fused<S, 1, LB_MODE_REGION, 6>(a, rho, ux, uy, uz, st);
   }
+  if (h->lb_cpt == 2) return launch_fused<S, 2, LB_MODE_STEP, 6>(a, rho, ux, uy, uz, st);
+  if (h->lb_cpt == 4) return launch_fused<S, 4, LB_MODE_STEP, 6>(a, rho, ux, uy, uz, st);
+  if (lb_cached(h))
+    return launch_fused<S, 1, LB_MODE_STEP | LB_CACHED, 6>(a, rho, ux, uy, uz, st);
+  if constexpr (S == PFG_STORE_F32)
+    if (a.ncell < LB_LARGE_CELLS)
+      return launch_fused<S, 1, LB_MODE_STEP, 4>(a, rho, ux, uy, uz, st);
+  return launch_fused<S, 1, LB_MODE_STEP, 6>(a, rho, ux, uy, uz, st);
 }
 
 static hipError_t dispatch_lb(pfg_handle *h, int k, int mode, float *rho, float *ux, float *uy,
@@ -806,39 +855,41 @@ static unsigned queue_grid(pfg_handle *h, KER kernel) {
 
 template <int S, int CPT, int MODE>
 static void launch_batch(pfg_handle *h, hipStream_t st) {
-  const dim3 grid((unsigned)h->lb_blocks), block(256);
+  const uint32_t ntasks = (uint32_t)h->lb_blocks;
+  const dim3 grid((ntasks + CPT - 1) / CPT), block(256);
   const LBArgs *args = h->d_lbargs[h->cur];
-  if (h->lb_persistent && MODE == LB_MODE_STEP && h->lb_queue) {
-    if (h->p.wall[2] == PFG_WALL_VELOCITY) {
-      auto k = lb_batch_queue_kernel<S, CPT, MODE | LB_ZVEL>;
-      hipLaunchKernelGGL(k, dim3(queue_grid(h, k)), block, 0, st, args, h->lb_block_inst,
-                         (uint32_t)h->lb_blocks, h->lb_queue);
+  const bool zvel = h->p.wall[2] == PFG_WALL_VELOCITY; /* the lattices of a batch share the walls */
+  if (CPT == 1 && h->lb_persistent && MODE == LB_MODE_STEP && h->lb_queue) {
+    if (zvel) {
+      auto k = lb_batch_queue_kernel<S, MODE | LB_ZVEL>;
+      hipLaunchKernelGGL(k, dim3(queue_grid(h, k)), block, 0, st, args, h->lb_block_inst, ntasks,
+                         h->lb_queue);
     } else {
-      auto k = lb_batch_queue_kernel<S, CPT, MODE>;
-      hipLaunchKernelGGL(k, dim3(queue_grid(h, k)), block, 0, st, args, h->lb_block_inst,
-                         (uint32_t)h->lb_blocks, h->lb_queue);
+      auto k = lb_batch_queue_kernel<S, MODE>;
+      hipLaunchKernelGGL(k, dim3(queue_grid(h, k)), block, 0, st, args, h->lb_block_inst, ntasks,
+                         h->lb_queue);
     }
     return;
   }
   const int xcd = h->lb_xcd_rows;
-  if (h->p.wall[2] == PFG_WALL_VELOCITY) /* the lattices of a batch share the walls */
+  if (CPT == 1 && MODE == LB_MODE_STEP && !zvel && lb_cached(h))
+    hipLaunchKernelGGL((lb_batch_kernel<S, 1, LB_MODE_STEP | LB_CACHED>), grid, block, 0, st, args,
+                       h->lb_block_inst, ntasks, xcd);
+  else if (zvel)
     hipLaunchKernelGGL((lb_batch_kernel<S, CPT, MODE | LB_ZVEL>), grid, block, 0, st, args,
-                       h->lb_block_inst, xcd);
+                       h->lb_block_inst, ntasks, xcd);
   else
     hipLaunchKernelGGL((lb_batch_kernel<S, CPT, MODE>), grid, block, 0, st, args,
-                       h->lb_block_inst, xcd);
+                       h->lb_block_inst, ntasks, xcd);
 }
 
-/* The workgroup table follows h->lb_cpt; the row-split passes take one
- * z-row per wavefront. */
 template <int S>
 static hipError_t launch_lb_batch_s(pfg_handle *h, int mode, hipStream_t st) {
-  if (mode != LB_MODE_STEP && h->lb_cpt != 1) return hipErrorInvalidValue;
   switch (mode) {
     case LB_MODE_BULK: launch_batch<S, 1, LB_MODE_BULK>(h, st); break;
     case LB_MODE_REGION: launch_batch<S, 1, LB_MODE_REGION>(h, st); break;
-    default:
-      switch (h->lb_cpt) {
+    default: /* the persistent launch takes its blocks one at a time */
+      switch (h->lb_persistent ? 1 : h->lb_cpt) {
         case 2: launch_batch<S, 2, LB_MODE_STEP>(h, st); break;
         case 4: launch_batch<S, 4, LB_MODE_STEP>(h, st); break;
         default: launch_batch<S, 1, LB_MODE_STEP>(h, st);
@@ -847,7 +898,7 @@ static hipError_t launch_lb_batch_s(pfg_handle *h, int mode, hipStream_t st) {
   return hipGetLastError();
 }
 
-/* All lattices of a batch in one launch (one z-cell per lane). */
+/* All lattices of a batch in one launch. */
 static hipError_t launch_lb_batch(pfg_handle *h, int mode, hipStream_t st) {
   switch (h->p.store) {
     case PFG_STORE_F16: return launch_lb_batch_s<PFG_STORE_F16>(h, mode, st);
@@ -884,6 +935,8 @@ hipError_t launch_bbmask(pfg_handle *h, int k) {
   const Inst &L = h->inst[(size_t)k];
   hipLaunchKernelGGL(bbmask_kernel, dim3((unsigned)((L.N + 255) / 256)), dim3(256), 0,
                      h->stream, a, a.solid, h->bbmask + L.cell0);
+  hipLaunchKernelGGL(block_kind_kernel, dim3((unsigned)((L.N + 255) / 256)), dim3(256), 0,
+                     h->stream, h->bbmask + L.cell0, a.ncell, h->block_kind + L.fblk0);
   return hipGetLastError();
 }
 

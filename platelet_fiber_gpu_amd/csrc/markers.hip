@@ -440,12 +440,15 @@ __global__ __launch_bounds__(256) void begin_kernel(MArgs a) {
       for (int ky = 0; ky < 4; ++ky) {
         const int y = axis_index(oy + ky, L.ny, L.periodic[1]);
         if (y < 0) continue;
-        int last = -1;
+        const int64_t row = y + (int64_t)L.ny * z;
+        int64_t last = -1;
         for (int kx = 0; kx < 4; ++kx) {
           const int x = axis_index(ox + kx, L.nx, L.periodic[0]);
-          if (x < 0 || (x >> 6) == last) continue;
-          last = x >> 6;
-          L.row_stamp[last + (int64_t)L.nxb * (y + (int64_t)L.ny * z)] = step;
+          if (x < 0) continue;
+          const int64_t blk = (x + L.nx * row) >> 6;
+          if (blk == last) continue;
+          last = blk;
+          L.row_stamp[blk] = step;
         }
       }
     }
@@ -3504,7 +3507,6 @@ void fill_mlat(const pfg_handle *h, int k, MLat *L) {
   L->bin0 = (int)I.bin0;
   L->binc0 = (int)I.binc0;
   L->tile0 = I.tile0;
-  L->nxb = I.nxb;
   L->row_stamp = h->row_stamp ? h->row_stamp + I.fblk0 : nullptr;
   L->seed = I.p.seed;
   L->rec0 = I.rec0;

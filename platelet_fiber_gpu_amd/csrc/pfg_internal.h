@@ -66,10 +66,16 @@ constexpr int RESOLVE_IN_GATHER_MAX = 2048;
  * (above it the counting wavefronts meet on few spans and a reduction
  * launch is cheaper). */
 constexpr int SPAN_COUNT_MAX = 32768;
-/* Lattice cells from which a single-lattice LB launch gives each XCD a
- * contiguous range of rows by default (faster at 268 M cells, slower at
- * 4 M; the autotuner tries both). */
-constexpr int64_t XCD_ROWS_MIN_CELLS = (int64_t)1 << 27;
+/* Both copies of the populations together, up to which the LB update stores
+ * through the caches, and up to which each XCD takes a contiguous range of
+ * blocks by default (so do single lattices from LB_LARGE_CELLS up); the
+ * figures are at the launcher in lb.hip. */
+constexpr int64_t LB_CACHED_MAX_BYTES = (int64_t)320 << 20;
+constexpr int64_t LB_XCD_MAX_BYTES = (int64_t)256 << 20;
+constexpr int64_t LB_LARGE_CELLS = (int64_t)1 << 27;
+/* Kind of a block of 64 cells: no solid cell and no solid upstream
+ * neighbour, some, or solid cells only. */
+constexpr int BLOCK_FLUID = 0, BLOCK_MIXED = 1, BLOCK_SOLID = 2;
 /* Device counters of a handle (Markers::counters). */
 constexpr int N_COUNTERS = 16;
 /* Morse pairs whose distance lies within this of the cutoff are counted: a
@@ -87,13 +93,16 @@ struct LBArgs {
   const uint8_t *solid;   /* nullptr when there are no solid cells          */
   const uint32_t *bbmask; /* per cell: bit d = upstream of d is solid,
                              bit 31 = cell is solid; nullptr without flags  */
+  const int32_t *block_kind; /* per block of 64 cells: BLOCK_FLUID, ...;
+                             nullptr without flags                          */
   const int64_t *halt;    /* nonzero *halt: leave the lattice unchanged
                              (run halted at detach); nullptr: never          */
-  const int32_t *row_stamp; /* per x-block row: the last step whose IB
-                             stencils touch the row                          */
+  const int32_t *row_stamp; /* per block of 64 cells: the last step whose IB
+                             stencils touch the block                        */
   const int64_t *step;    /* the current step (device counter)              */
   int nx, ny, nz;
-  int nxb;                /* x-blocks of XBLOCK cells per row                 */
+  uint32_t ncell;         /* cells of the lattice                             */
+  float inv_nx, inv_ny;   /* 1 / nx, 1 / ny                                   */
   int64_t block0;         /* first workgroup of this lattice in a batched
                              launch                                          */
   int tnx, tny;           /* tiles per axis                                   */
@@ -129,8 +138,7 @@ struct MLat {
   int nbc[3];             /* coarse bins per axis (lists without elements)    */
   int binc0;              /* first global coarse bin of the lattice           */
   int64_t tile0;          /* first global tile of the lattice                 */
-  int nxb;                /* x-blocks per row                                 */
-  int32_t *row_stamp;     /* the lattice's x-block rows (nullptr: unused)     */
+  int32_t *row_stamp;     /* the lattice's blocks of 64 cells (nullptr: unused) */
   /* counter-RNG key of the lattice's own draws (bonds, noise): its seed and
    * lattice-local receptor and marker indices, so that a lattice of a batch
    * draws what it draws in a handle of its own */
@@ -298,8 +306,8 @@ struct Inst {
   pfg_params p{};          /* lattice and fluid fields apply per lattice     */
   int64_t N = 0;           /* cells                                          */
   int64_t cell0 = 0;       /* first cell in the concatenated cell fields     */
-  int nxb = 0;
-  int64_t fblk0 = 0;       /* first x-block in the population arrays          */
+  int64_t fblk0 = 0;       /* first block in the population arrays            */
+  int64_t nfblk = 0;       /* its blocks of 64 cells                          */
   int tnx = 0, tny = 0, tnz = 0;
   int64_t ntiles = 0, tile0 = 0;
   int nb[3] = {1, 1, 1};
@@ -317,10 +325,9 @@ struct pfg_handle {
   int device = 0;
   hipStream_t stream = nullptr;
   int64_t N = 0, plane = 0;
-  int nxb = 0;                 /* x-blocks per row in the population layout */
   int esize = 4;
-  /* populations, blocked: element (d,x,y,z) at
-   * ((x/64 + nxb*(y + ny*z))*19 + d)*64 + x%64 */
+  /* populations, blocked: direction d of cell i = x + nx*(y + ny*z) at
+   * ((i/64)*19 + d)*64 + i%64 */
   void *f[2] = {nullptr, nullptr};
   int cur = 0;
   /* IB coupling fields: spreading adds the force of a step into aux and
@@ -337,9 +344,10 @@ struct pfg_handle {
   int64_t ntiles = 0;
   uint8_t *solid = nullptr;
   uint32_t *bbmask = nullptr;  /* per-cell bounce mask built from solid        */
+  int32_t *block_kind = nullptr; /* per block of 64 cells, from the masks      */
   double *red = nullptr;       /* reduction partials                        */
   int64_t red_blocks = 0;
-  int lb_cpt = 1;              /* LB launch: z-cells per lane               */
+  int lb_cpt = 1;              /* LB launch: cells (blocks in a row) per lane */
   int lb_xcd_rows = 0;         /* LB launch: contiguous rows per XCD        */
   pfg::Markers m;
   bool model_loaded = false;
@@ -381,9 +389,11 @@ namespace pfg {
 
 /* lb.hip; k selects a lattice of the handle */
 void make_lb_args(const pfg_handle *h, int k, int cur, LBArgs *a);
+/* the block order a handle starts with (pfg_set_lb_xcd_rows) */
+int lb_default_xcd_rows(const pfg_handle *h);
 hipError_t launch_lb(pfg_handle *h);
-/* part 1: rows no IB stencil touches this step (on stream s); part 2: the
- * rows they touch, with the IB force (then the copies of f alternate) */
+/* part 1: blocks no IB stencil touches this step (on stream s); part 2: the
+ * blocks they touch, with the IB force (then the copies of f alternate) */
 hipError_t launch_lb_part(pfg_handle *h, int part, hipStream_t s);
 hipError_t launch_bbmask(pfg_handle *h, int k);
 hipError_t launch_lb_fields(pfg_handle *h, int k, float *rho, float *ux, float *uy,
