@@ -230,13 +230,23 @@ __device__ inline bool ib_coupled(int kind, int fiber_move) {
   return kind == PFG_MARKER_ELEMENT || (kind == PFG_MARKER_FIBER && fiber_move == PFG_FIBER_IB);
 }
 
+/* A coordinate in the periodic cell [0, n]; one that is not a number, or too
+ * large for the remainder to mean anything, lands on its boundary. */
 __device__ inline float wrap_coord(float v, int n, int periodic) {
   if (!periodic) return v;
   const float fn = (float)n;
   float w = v - fn * floorf(v / fn);
   if (w >= fn) w -= fn;
   if (w < 0.f) w += fn;
-  return w;
+  return fminf(fmaxf(w, 0.f), fn);
+}
+
+/* floor(W) as an index, any W: far outside the lattice (or not a number) it
+ * stops eight nodes outside, where no node of a stencil is inside.  The
+ * unlimited conversion overflowed when a node's offset was added, and the
+ * range checks, compiled under the promise that it does not, let it through. */
+__device__ inline int floor_index(float W, int n) {
+  return (int)fminf(fmaxf(floorf(W), -8.0f), (float)n + 8.0f);
 }
 
 /* Lattice index along an axis, or -1 when outside a wall-bounded axis.
@@ -290,7 +300,7 @@ __device__ inline float stencil_weight(float W, int k) {
  * (or -1) and weight phi(X - i). */
 __device__ inline int stencil_node(float X, int k, int n, int periodic, float *w) {
   *w = stencil_weight(X, k);
-  return axis_index((int)floorf(X) - 1 + k, n, periodic);
+  return axis_index(floor_index(X, n) - 1 + k, n, periodic);
 }
 
 /* ---------------- K1: tile clear + bin counting ---------------- */
@@ -431,9 +441,9 @@ __global__ __launch_bounds__(256) void begin_kernel(MArgs a) {
      * interpolation use), so that the LB update of every other row may run
      * before the spreading */
     const int step = (int)*a.m.d_step;
-    const int ox = (int)floorf(wrap_coord(a.m.x[i], L.nx, L.periodic[0])) - 1;
-    const int oy = (int)floorf(wrap_coord(a.m.y[i], L.ny, L.periodic[1])) - 1;
-    const int oz = (int)floorf(wrap_coord(a.m.z[i], L.nz, L.periodic[2])) - 1;
+    const int ox = floor_index(wrap_coord(a.m.x[i], L.nx, L.periodic[0]), L.nx) - 1;
+    const int oy = floor_index(wrap_coord(a.m.y[i], L.ny, L.periodic[1]), L.ny) - 1;
+    const int oz = floor_index(wrap_coord(a.m.z[i], L.nz, L.periodic[2]), L.nz) - 1;
     for (int kz = 0; kz < 4; ++kz) {
       const int z = axis_index(oz + kz, L.nz, L.periodic[2]);
       if (z < 0) continue;
@@ -1797,7 +1807,7 @@ __global__ __launch_bounds__(BODY_THREADS) void forces_body_build_kernel(MArgs a
   int d[3] = {1, 1, 1};
   if (rebuild) {
     cs = fmaxf(R, 1e-3f);
-    for (;;) {
+    for (int doubled = 0;; ++doubled) {
       int64_t nb = 1;
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
@@ -1805,6 +1815,10 @@ __global__ __launch_bounds__(BODY_THREADS) void forces_body_build_kernel(MArgs a
         nb *= d[k];
       }
       if (nb <= FB_BINS) break;
+      if (doubled == 200) { /* an extent that is not finite: one cell */
+        d[0] = d[1] = d[2] = 1;
+        break;
+      }
       cs *= 2.0f;
     }
     inv = 1.0f / cs;
@@ -2160,7 +2174,7 @@ __device__ inline void stencil_origin(const MLat &L, const float v[3], const flo
   for (int k = 0; k < 3; ++k) {
     W[k] = wrap_coord(v[k], n[k], L.periodic[k]);
     const int img = L.periodic[k] ? -(int)rintf((W[k] - ref[k]) / (float)n[k]) * n[k] : 0;
-    o[k] = (int)floorf(W[k]) - 1 + img;
+    o[k] = floor_index(W[k], n[k]) - 1 + img;
   }
 }
 
@@ -2881,8 +2895,8 @@ __global__ __launch_bounds__(256) void spread_prep_kernel(MArgs a) {
       const float W[3] = {wrap_coord(a.m.x[i], L.nx, L.periodic[0]),
                           wrap_coord(a.m.y[i], L.ny, L.periodic[1]),
                           wrap_coord(a.m.z[i], L.nz, L.periodic[2])};
-      const int ox = (int)floorf(W[0]) - 1, oy = (int)floorf(W[1]) - 1,
-                oz = (int)floorf(W[2]) - 1;
+      const int ox = floor_index(W[0], L.nx) - 1, oy = floor_index(W[1], L.ny) - 1,
+                oz = floor_index(W[2], L.nz) - 1;
       r.o = make_int4(ox, oy, oz, 1);
       float w4[4];
       stencil_weights(W[0], w4);
@@ -3131,7 +3145,7 @@ __device__ void interp_marker(const MArgs &a, int i, int j, float *v) {
     const float wxy = wx * wy;
     float wz4[4];
     stencil_weights(Z, wz4);
-    const int oz = (int)floorf(Z) - 1;
+    const int oz = floor_index(Z, L.nz) - 1;
 #pragma unroll
     for (int kz = 0; kz < 4; ++kz) {
       const int iz = axis_index(oz + kz, L.nz, L.periodic[2]);

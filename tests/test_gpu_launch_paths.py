@@ -102,3 +102,30 @@ def test_overlap_equals_serial_on_rows_that_share_blocks(gpu, nx):
     assert np.abs(res[0][0] - res[1][0]).max() < 1e-6
     for k in ("x", "y", "z", "vx", "vy", "vz"):
         assert np.abs(res[0][1][k] - res[1][1][k]).max() < 1e-5, k
+
+
+@pytest.mark.parametrize("by_body", [1, 2])
+@pytest.mark.parametrize("staging", [1, 2, 3, 4])
+def test_markers_that_left_every_range(gpu, staging, by_body):
+    """A run that has diverged ends in numbers, not in a fault: elements far below a
+    wall (beyond the range of int), far along a periodic axis, infinite or not a
+    number.  The stencil index of such a coordinate used to overflow past its range
+    check.  The fluid around the lost elements is lost with them; a platelet far
+    from them steps on."""
+    pfg = gpu
+    sc = pfg.Scene(pfg.SCENE_LARGE, nx=128, ny=64, nz=64, n_platelets=3, elements=200,
+                   receptors=16, ligands=256, fibrin_nodes=64, fibrin_links=80)
+    x, y, z = sc.x.copy(), sc.y.copy(), sc.z.copy()
+    first, lost, healthy = (np.flatnonzero(sc.body == b) for b in range(3))
+    z[first] = -3e9
+    x[lost[0]], y[lost[1]], x[lost[2]], z[lost[3]] = 1e30, np.inf, np.nan, 3e38
+    with pfg.Solver(sc.params) as s:
+        s.load(sc)
+        s.set_ib_staging(staging)
+        s.set_forces_by_body(by_body)
+        s.set_forces_lanes(4 if by_body == 1 else 0)
+        s.set_markers(x, y, z)
+        s.step(2)
+        m = s.markers()
+    assert all(np.isfinite(m[k][healthy]).all() for k in ("x", "y", "z", "fx", "fy", "fz"))
+    assert (m["z"][first] < -2e9).all()
