@@ -326,6 +326,24 @@ hipError_t upload_batch_args(pfg_handle *h) {
   return hipSuccess;
 }
 
+/* Arrays to the host, through pinned memory where it can be had.  A null
+ * destination is skipped. */
+hipError_t download_all(pfg_handle *h, Piece *pieces, int n) {
+  for (int k = 0; k < n; ++k)
+    if (!pieces[k].dst) pieces[k].bytes = 0;
+  hipError_t e = hipErrorOutOfMemory;
+  try {
+    e = fetch_pieces(h, pieces, n);
+  } catch (const std::bad_alloc &) {
+  }
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  e = hipSuccess;
+  for (int k = 0; k < n && e == hipSuccess; ++k)
+    e = download(h, (char *)pieces[k].dst, (const char *)pieces[k].src, pieces[k].bytes);
+  return e;
+}
+
 /* One or K lattices; shared fields (storage, markers, bonds, fibrin) come
  * from ps[0], lattice and fluid fields from each ps[k]. */
 pfg_status create_impl(const pfg_params *ps, int K, int device, pfg_handle **out) {
@@ -363,6 +381,7 @@ pfg_status create_impl(const pfg_params *ps, int K, int device, pfg_handle **out
 
   pfg_handle *h = new (std::nothrow) pfg_handle();
   if (!h) return PFG_ERR_ALLOC;
+  frames_ref();
   h->p = p;
   h->device = device;
   h->K = K;
@@ -548,21 +567,21 @@ pfg_status upload_flags_impl(pfg_handle *h, int k, const uint8_t *flags) {
 
 pfg_status fields_impl(pfg_handle *h, int k, float *rho, float *ux, float *uy, float *uz) {
   hipSetDevice(h->device);
+  float *host[4] = {rho, ux, uy, uz};
+  hipError_t e = hipErrorOutOfMemory;
+  try {
+    e = fetch_fields(h, k, host);
+  } catch (const std::bad_alloc &) {
+  }
+  if (e != hipErrorOutOfMemory) return from_hip(e);
+  (void)hipGetLastError();
+  /* without pinned memory: through device arrays */
   const int64_t n = h->inst[(size_t)k].N;
   float *dev[4] = {nullptr, nullptr, nullptr, nullptr};
-  float *host[4] = {rho, ux, uy, uz};
   pfg_status st = PFG_OK;
-  for (int c = 0; c < 4; ++c) {
-    if (!host[c]) continue;
-    if (hipMalloc(&dev[c], sizeof(float) * n) != hipSuccess) {
-      st = PFG_ERR_ALLOC;
-      break;
-    }
-    /* solid cells are not written by the fields pass: they read 0 */
-    st = from_hip(hipMemsetAsync(dev[c], 0, sizeof(float) * n, h->stream));
-    if (st != PFG_OK) break;
-  }
-  if (st == PFG_OK) st = from_hip(launch_lb_fields(h, k, dev[0], dev[1], dev[2], dev[3]));
+  for (int c = 0; c < 4 && st == PFG_OK; ++c)
+    if (host[c] && hipMalloc(&dev[c], sizeof(float) * n) != hipSuccess) st = PFG_ERR_ALLOC;
+  if (st == PFG_OK) st = from_hip(launch_lb_fields_window(h, k, 0, (uint32_t)n, dev));
   for (int c = 0; c < 4 && st == PFG_OK; ++c)
     if (host[c]) st = from_hip(download(h, host[c], dev[c], (size_t)n));
   for (int c = 0; c < 4; ++c)
@@ -610,6 +629,7 @@ pfg_status pfg_destroy(pfg_handle *h) {
   if (h->stream2) hipStreamDestroy(h->stream2);
   if (h->stream) hipStreamDestroy(h->stream);
   delete h;
+  frames_unref();
   return PFG_OK;
 }
 
@@ -1469,23 +1489,24 @@ pfg_status pfg_upload_markers(pfg_handle *h, const float *x, const float *y,
   return PFG_OK;
 }
 
+static pfg_status download_markers(pfg_handle *h, size_t m0, size_t n, float *x, float *y,
+                                   float *z, float *vx, float *vy, float *vz, float *fx,
+                                   float *fy, float *fz) {
+  const Markers &m = h->m;
+  float *dst[9] = {x, y, z, vx, vy, vz, fx, fy, fz};
+  const float *src[9] = {m.x, m.y, m.z, m.vx, m.vy, m.vz, m.fx, m.fy, m.fz};
+  Piece p[9];
+  for (int k = 0; k < 9; ++k) p[k] = {dst[k], src[k] + m0, sizeof(float) * n};
+  return from_hip(download_all(h, p, 9));
+}
+
 pfg_status pfg_download_markers(pfg_handle *h, float *x, float *y, float *z,
                                 float *vx, float *vy, float *vz, float *fx,
                                 float *fy, float *fz) {
   if (!h) return PFG_ERR_ARG;
   if (!h->model_loaded) return PFG_ERR_STATE;
   hipSetDevice(h->device);
-  const size_t n = (size_t)h->m.n;
-  PFG_TRY(download(h, x, h->m.x, n));
-  PFG_TRY(download(h, y, h->m.y, n));
-  PFG_TRY(download(h, z, h->m.z, n));
-  PFG_TRY(download(h, vx, h->m.vx, n));
-  PFG_TRY(download(h, vy, h->m.vy, n));
-  PFG_TRY(download(h, vz, h->m.vz, n));
-  PFG_TRY(download(h, fx, h->m.fx, n));
-  PFG_TRY(download(h, fy, h->m.fy, n));
-  PFG_TRY(download(h, fz, h->m.fz, n));
-  return PFG_OK;
+  return download_markers(h, 0, (size_t)h->m.n, x, y, z, vx, vy, vz, fx, fy, fz);
 }
 
 pfg_status pfg_batch_download_markers(pfg_handle *h, int k, float *x, float *y, float *z,
@@ -1496,16 +1517,7 @@ pfg_status pfg_batch_download_markers(pfg_handle *h, int k, float *x, float *y, 
   hipSetDevice(h->device);
   const size_t m0 = (size_t)h->marker0[(size_t)k];
   const size_t n = (size_t)h->marker0[(size_t)k + 1] - m0;
-  PFG_TRY(download(h, x, h->m.x + m0, n));
-  PFG_TRY(download(h, y, h->m.y + m0, n));
-  PFG_TRY(download(h, z, h->m.z + m0, n));
-  PFG_TRY(download(h, vx, h->m.vx + m0, n));
-  PFG_TRY(download(h, vy, h->m.vy + m0, n));
-  PFG_TRY(download(h, vz, h->m.vz + m0, n));
-  PFG_TRY(download(h, fx, h->m.fx + m0, n));
-  PFG_TRY(download(h, fy, h->m.fy + m0, n));
-  PFG_TRY(download(h, fz, h->m.fz + m0, n));
-  return PFG_OK;
+  return download_markers(h, m0, n, x, y, z, vx, vy, vz, fx, fy, fz);
 }
 
 pfg_status pfg_upload_marker_forces(pfg_handle *h, const float *fx,
@@ -1537,10 +1549,10 @@ pfg_status pfg_download_membrane(pfg_handle *h, double *S_all, double *V,
   if (!h) return PFG_ERR_ARG;
   if (!h->model_loaded) return PFG_ERR_STATE;
   hipSetDevice(h->device);
-  PFG_TRY(download(h, S_all, h->m.plt_S, (size_t)h->m.n_plt));
-  PFG_TRY(download(h, V, h->m.plt_V, (size_t)h->m.n_plt));
-  PFG_TRY(download(h, tri_S, h->m.tri_S, (size_t)h->m.n_tri));
-  return PFG_OK;
+  Piece p[3] = {{S_all, h->m.plt_S, sizeof(double) * (size_t)h->m.n_plt},
+                {V, h->m.plt_V, sizeof(double) * (size_t)h->m.n_plt},
+                {tri_S, h->m.tri_S, sizeof(double) * (size_t)h->m.n_tri}};
+  return from_hip(download_all(h, p, 3));
 }
 
 pfg_status pfg_download_bonds(pfg_handle *h, int32_t *rec_bond, int32_t *lig_owner,
@@ -1548,10 +1560,10 @@ pfg_status pfg_download_bonds(pfg_handle *h, int32_t *rec_bond, int32_t *lig_own
   if (!h) return PFG_ERR_ARG;
   if (!h->model_loaded) return PFG_ERR_STATE;
   hipSetDevice(h->device);
-  PFG_TRY(download(h, rec_bond, h->m.rec_bond, (size_t)h->m.n_rec));
-  PFG_TRY(download(h, lig_owner, h->m.lig_owner, (size_t)h->m.n_lig));
-  PFG_TRY(download(h, rec_force, h->m.rec_force, 3 * (size_t)h->m.n_rec));
-  return PFG_OK;
+  Piece p[3] = {{rec_bond, h->m.rec_bond, sizeof(int32_t) * (size_t)h->m.n_rec},
+                {lig_owner, h->m.lig_owner, sizeof(int32_t) * (size_t)h->m.n_lig},
+                {rec_force, h->m.rec_force, sizeof(float) * 3 * (size_t)h->m.n_rec}};
+  return from_hip(download_all(h, p, 3));
 }
 
 pfg_status pfg_upload_bonds(pfg_handle *h, const int32_t *rec_bond) {
@@ -1590,9 +1602,9 @@ pfg_status pfg_download_cells(pfg_handle *h, int32_t *bin_start, int32_t *bin_it
   if (!h->model_loaded) return PFG_ERR_STATE;
   hipSetDevice(h->device);
   const int64_t nb = bin_elements(h) ? h->m.nbins : h->m.nbinsc;
-  PFG_TRY(download(h, bin_start, h->m.bin_start, (size_t)nb + 1));
-  PFG_TRY(download(h, bin_items, h->m.bin_items, (size_t)h->m.n));
-  return PFG_OK;
+  Piece p[2] = {{bin_start, h->m.bin_start, sizeof(int32_t) * ((size_t)nb + 1)},
+                {bin_items, h->m.bin_items, sizeof(int32_t) * (size_t)h->m.n}};
+  return from_hip(download_all(h, p, 2));
 }
 
 pfg_status pfg_download_aux(pfg_handle *h, float *a3n) {
@@ -1714,21 +1726,15 @@ static hipError_t build_graphs(pfg_handle *h) {
   return e;
 }
 
-static pfg_status fill_info(pfg_handle *h, pfg_step_info *info) {
-  if (!info) return PFG_OK;
-  int64_t c[N_COUNTERS] = {};
-  int64_t ds = -1;
-  PFG_TRY(download(h, c, h->m.counters, N_COUNTERS));
-  PFG_TRY(download(h, &ds, h->m.detach_step, 1));
-  info->step = h->h_step;
-  info->total_bonds = (int32_t)c[0];
-  info->detached = (int32_t)c[1];
-  info->detach_step = ds;
-  info->near_threshold = c[2];
-  info->bond_events = c[4];
-  info->near_cutoff = c[8];
-  info->contact_overflow = c[9];
-  return PFG_OK;
+/* The counters, detach step and step index after all enqueued work. */
+static hipError_t read_report(pfg_handle *h, int64_t r[N_COUNTERS + 2]) {
+  hipError_t e = fetch_report(h, r);
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  e = download(h, r, h->m.counters, N_COUNTERS);
+  if (e == hipSuccess) e = download(h, r + N_COUNTERS, h->m.detach_step, 1);
+  if (e == hipSuccess) e = download(h, r + N_COUNTERS + 1, h->m.d_step, 1);
+  return e;
 }
 
 pfg_status pfg_step(pfg_handle *h, int nsteps, pfg_step_info *info) {
@@ -1751,19 +1757,32 @@ pfg_status pfg_step(pfg_handle *h, int nsteps, pfg_step_info *info) {
     }
     h->h_step++;
   }
-  PFG_TRY(hipStreamSynchronize(h->stream));
-  if (h->halt_on_detach && h->model_loaded && !h->fluid_only) {
+  const bool halts = h->halt_on_detach && h->model_loaded && !h->fluid_only;
+  if (!info && !halts) {
+    PFG_TRY(hipStreamSynchronize(h->stream));
+    return PFG_OK;
+  }
+  int64_t r[N_COUNTERS + 2];
+  PFG_TRY(read_report(h, r));
+  const int64_t done = r[N_COUNTERS + 1];
+  if (halts && h->h_step > done) {
     /* steps launched after the detach test fired left the lattice in place
      * while the host alternated the copies: realign the current copy with
      * the steps that actually ran */
-    int64_t done = 0;
-    PFG_TRY(download(h, &done, h->m.d_step, 1));
-    if (h->h_step > done) {
-      if ((h->h_step - done) & 1) h->cur = 1 - h->cur;
-      h->h_step = done;
-    }
+    if ((h->h_step - done) & 1) h->cur = 1 - h->cur;
+    h->h_step = done;
   }
-  return fill_info(h, info);
+  if (info) {
+    info->step = h->h_step;
+    info->total_bonds = (int32_t)r[0];
+    info->detached = (int32_t)r[1];
+    info->detach_step = r[N_COUNTERS];
+    info->near_threshold = r[2];
+    info->bond_events = r[4];
+    info->near_cutoff = r[8];
+    info->contact_overflow = r[9];
+  }
+  return PFG_OK;
 }
 
 pfg_status pfg_set_overlap(pfg_handle *h, int enable) {

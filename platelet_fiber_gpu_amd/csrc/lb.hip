@@ -295,14 +295,22 @@ __device__ __forceinline__ void lb_update(const LBArgs &a, uint32_t blk, float *
     if (touched != (M == LB_MODE_REGION)) return;
   }
   const int kind = a.block_kind != nullptr ? a.block_kind[task] : BLOCK_FLUID;
-  if (kind == BLOCK_SOLID) return;
+  if (M != LB_MODE_FIELDS && kind == BLOCK_SOLID) return;
   const uint32_t lane = threadIdx.x & (XBLOCK - 1);
   const uint32_t i = i0 + lane;
   if (i < lo || i >= hi || i >= a.ncell) return;
   uint32_t mask = 0;
-  if (kind == BLOCK_MIXED) {
+  if (kind != BLOCK_FLUID) {
     mask = a.bbmask[i];
-    if (mask >> 31) return; /* solid cell */
+    if (mask >> 31) { /* solid cell: its fields read 0 */
+      if (M == LB_MODE_FIELDS) {
+        if (orho) orho[i] = 0.f;
+        if (oux) oux[i] = 0.f;
+        if (ouy) ouy[i] = 0.f;
+        if (ouz) ouz[i] = 0.f;
+      }
+      return;
+    }
   }
   const uint32_t nx = (uint32_t)a.nx, ny = (uint32_t)a.ny, nxy = nx * ny;
   const uint32_t wz = i0 / nxy, wr = i0 - wz * nxy, wy = wr / nx, wx = wr - wy * nx;
@@ -394,9 +402,10 @@ __device__ inline uint32_t launch_block(int xcd_rows) {
  * wavefronts a SIMD holds at most. */
 template <int S, int CPT, int MODE, int WAVES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void
-lb_fused_kernel(LBArgs a, float *orho, float *oux, float *ouy, float *ouz) {
+lb_fused_kernel(LBArgs a) {
   const uint32_t blk = launch_block(a.xcd_rows) * CPT;
-  for (uint32_t c = 0; c < CPT; ++c) lb_update<S, MODE>(a, blk + c, orho, oux, ouy, ouz);
+  for (uint32_t c = 0; c < CPT; ++c)
+    lb_update<S, MODE>(a, blk + c, nullptr, nullptr, nullptr, nullptr);
 }
 
 /* A batch of lattices in one launch: workgroup task -> lattice through a
@@ -468,10 +477,10 @@ __global__ __launch_bounds__(256) void lb_batch_queue_kernel(const LBArgs *args,
  * process ends; calls on one device share it. */
 static __device__ __align__(256) float scratch[FIELDS_SCRATCH_FLOATS];
 
-/* The fields pass over the blocks [t0, t1) that hold the cells [lo, hi) of
- * z-planes [z0, z1), one wavefront per block; o* point at cell 0 of the window's first
- * plane minus z0 planes, so that each cell lands at its offset in the window. */
-template <int S>
+/* The fields pass over the blocks [t0, t1) that hold the cells [lo, hi), one
+ * wavefront per block; o* point lo cells before the window, so that each cell
+ * lands at its offset in it. */
+template <int S, int MODE>
 __global__ __launch_bounds__(256) void lb_fields_window_kernel(LBArgs a, uint32_t blk0,
                                                                uint32_t t0, uint32_t t1,
                                                                uint32_t lo, uint32_t hi,
@@ -480,12 +489,7 @@ __global__ __launch_bounds__(256) void lb_fields_window_kernel(LBArgs a, uint32_
   const uint32_t blk = blk0 + blockIdx.x;
   const uint32_t task = blk * 4u + (threadIdx.x >> 6);
   if (task < t0 || task >= t1) return;
-  lb_update<S, LB_MODE_FIELDS>(a, blk, orho, oux, ouy, ouz, -1, lo, hi);
-}
-
-__global__ __launch_bounds__(256) void fill_zero_kernel(float *p, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] = 0.f;
+  lb_update<S, MODE>(a, blk, orho, oux, ouy, ouz, -1, lo, hi);
 }
 
 /* Device address of `scratch` per device, looked up once with the device
@@ -513,48 +517,51 @@ hipError_t fields_scratch_setup(int device, float **out) {
 }
 
 template <int S>
-static hipError_t fields_window_s(pfg_handle *h, const LBArgs &a, int z0, int z1,
+static hipError_t fields_window_s(pfg_handle *h, const LBArgs &a, uint32_t lo, uint32_t hi,
                                   float *const win[4]) {
-  const int64_t plane = (int64_t)a.nx * a.ny;
-  const uint32_t lo = (uint32_t)(plane * z0), hi = (uint32_t)(plane * z1);
   const uint32_t t0 = lo / XBLOCK, t1 = (hi + XBLOCK - 1u) / XBLOCK;
   const uint32_t blk0 = t0 / 4u, blk1 = (t1 + 3u) / 4u;
   float *o[4];
-  for (int c = 0; c < 4; ++c) o[c] = win[c] ? win[c] - (int64_t)z0 * plane : nullptr;
-  hipLaunchKernelGGL(lb_fields_window_kernel<S>, dim3(blk1 - blk0), dim3(256), 0, h->stream, a,
-                     blk0, t0, t1, lo, hi, o[0], o[1], o[2], o[3]);
+  for (int c = 0; c < 4; ++c) o[c] = win[c] ? win[c] - (int64_t)lo : nullptr;
+  if (a.zvel)
+    hipLaunchKernelGGL((lb_fields_window_kernel<S, LB_MODE_FIELDS | LB_ZVEL>), dim3(blk1 - blk0),
+                       dim3(256), 0, h->stream, a, blk0, t0, t1, lo, hi, o[0], o[1], o[2], o[3]);
+  else
+    hipLaunchKernelGGL((lb_fields_window_kernel<S, LB_MODE_FIELDS>), dim3(blk1 - blk0), dim3(256),
+                       0, h->stream, a, blk0, t0, t1, lo, hi, o[0], o[1], o[2], o[3]);
   return hipGetLastError();
+}
+
+hipError_t launch_lb_fields_window(pfg_handle *h, int k, uint32_t lo, uint32_t hi,
+                                   float *const win[4]) {
+  LBArgs a;
+  make_lb_args(h, k, h->cur, &a);
+  switch (h->p.store) {
+    case PFG_STORE_F16: return fields_window_s<PFG_STORE_F16>(h, a, lo, hi, win);
+    case PFG_STORE_BF16: return fields_window_s<PFG_STORE_BF16>(h, a, lo, hi, win);
+    default: return fields_window_s<PFG_STORE_F32>(h, a, lo, hi, win);
+  }
 }
 
 hipError_t download_fields_noalloc(pfg_handle *h, float *const host[4]) {
   float *base = nullptr;
   hipError_t e = fields_scratch_setup(h->device, &base);
   if (e != hipSuccess) return e;
-  LBArgs a;
-  make_lb_args(h, 0, h->cur, &a);
   int nf = 0;
   for (int c = 0; c < 4; ++c) nf += host[c] != nullptr;
   if (nf == 0) return hipSuccess;
-  const int64_t plane = (int64_t)a.nx * a.ny;
+  const int nz = h->p.nz;
+  const int64_t plane = (int64_t)h->p.nx * h->p.ny;
   const int64_t zmax = FIELDS_SCRATCH_FLOATS / (plane * nf); /* planes per window */
   if (zmax < 1) return hipErrorInvalidValue;
-  for (int z0 = 0; z0 < a.nz && e == hipSuccess; z0 += (int)zmax) {
-    const int z1 = (int)std::min<int64_t>(a.nz, z0 + zmax);
+  for (int z0 = 0; z0 < nz && e == hipSuccess; z0 += (int)zmax) {
+    const int z1 = (int)std::min<int64_t>(nz, z0 + zmax);
     const int64_t n = plane * (z1 - z0);
     float *win[4] = {nullptr, nullptr, nullptr, nullptr};
     int slot = 0;
     for (int c = 0; c < 4; ++c)
       if (host[c]) win[c] = base + n * slot++;
-    /* solid cells are not written by the pass: they read 0 */
-    hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((n * nf + 255) / 256)), dim3(256), 0,
-                       h->stream, base, n * nf);
-    e = hipGetLastError();
-    if (e != hipSuccess) break;
-    switch (h->p.store) {
-      case PFG_STORE_F16: e = fields_window_s<PFG_STORE_F16>(h, a, z0, z1, win); break;
-      case PFG_STORE_BF16: e = fields_window_s<PFG_STORE_BF16>(h, a, z0, z1, win); break;
-      default: e = fields_window_s<PFG_STORE_F32>(h, a, z0, z1, win);
-    }
+    e = launch_lb_fields_window(h, 0, (uint32_t)(plane * z0), (uint32_t)(plane * z1), win);
     for (int c = 0; c < 4 && e == hipSuccess; ++c)
       if (host[c])
         e = hipMemcpyAsync(host[c] + (int64_t)z0 * plane, win[c], sizeof(float) * n,
@@ -780,16 +787,13 @@ void make_lb_args(const pfg_handle *h, int k, int cur, LBArgs *a) {
 }
 
 template <int S, int CPT, int MODE, int WAVES>
-static hipError_t launch_fused(const LBArgs &a, float *rho, float *ux, float *uy, float *uz,
-                               hipStream_t st) {
+static hipError_t launch_fused(const LBArgs &a, hipStream_t st) {
   constexpr int PER = 4 * XBLOCK * CPT; /* cells per workgroup */
   const dim3 grid((unsigned)(((int64_t)a.ncell + PER - 1) / PER));
   if (a.zvel)
-    hipLaunchKernelGGL((lb_fused_kernel<S, CPT, MODE | LB_ZVEL, WAVES>), grid, dim3(256), 0, st, a,
-                       rho, ux, uy, uz);
+    hipLaunchKernelGGL((lb_fused_kernel<S, CPT, MODE | LB_ZVEL, WAVES>), grid, dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((lb_fused_kernel<S, CPT, MODE, WAVES>), grid, dim3(256), 0, st, a, rho, ux,
-                       uy, uz);
+    hipLaunchKernelGGL((lb_fused_kernel<S, CPT, MODE, WAVES>), grid, dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
@@ -809,31 +813,28 @@ static hipError_t launch_fused(const LBArgs &a, float *rho, float *ux, float *uy
  *   587; 1024x512x512 FP32 7150 / 6700 / 6690, FP16 3510 / 3330 / 3560,
  *   FP16 512x256x256 427 / 415 / 431. */
 template <int S>
-static hipError_t launch_lb_s(const pfg_handle *h, const LBArgs &a, int mode, float *rho,
-                              float *ux, float *uy, float *uz, hipStream_t st) {
+static hipError_t launch_lb_s(const pfg_handle *h, const LBArgs &a, int mode, hipStream_t st) {
   switch (mode) {
-    case LB_MODE_FIELDS: return launch_fused<S, 1, LB_MODE_FIELDS, 6>(a, rho, ux, uy, uz, st);
-    case LB_MODE_BULK: return launch_fused<S, 1, LB_MODE_BULK, 6>(a, rho, ux, uy, uz, st);
-    case LB_MODE_REGION: return launch_fused<S, 1, LB_MODE_REGION, 6>(a, rho, ux, uy, uz, st);
+    case LB_MODE_BULK: return launch_fused<S, 1, LB_MODE_BULK, 6>(a, st);
+    case LB_MODE_REGION: return launch_fused<S, 1, LB_MODE_REGION, 6>(a, st);
   }
-  if (h->lb_cpt == 2) return launch_fused<S, 2, LB_MODE_STEP, 6>(a, rho, ux, uy, uz, st);
-  if (h->lb_cpt == 4) return launch_fused<S, 4, LB_MODE_STEP, 6>(a, rho, ux, uy, uz, st);
+  if (h->lb_cpt == 2) return launch_fused<S, 2, LB_MODE_STEP, 6>(a, st);
+  if (h->lb_cpt == 4) return launch_fused<S, 4, LB_MODE_STEP, 6>(a, st);
   if (lb_cached(h))
-    return launch_fused<S, 1, LB_MODE_STEP | LB_CACHED, 6>(a, rho, ux, uy, uz, st);
+    return launch_fused<S, 1, LB_MODE_STEP | LB_CACHED, 6>(a, st);
   if constexpr (S == PFG_STORE_F32)
     if (a.ncell < LB_LARGE_CELLS)
-      return launch_fused<S, 1, LB_MODE_STEP, 4>(a, rho, ux, uy, uz, st);
-  return launch_fused<S, 1, LB_MODE_STEP, 6>(a, rho, ux, uy, uz, st);
+      return launch_fused<S, 1, LB_MODE_STEP, 4>(a, st);
+  return launch_fused<S, 1, LB_MODE_STEP, 6>(a, st);
 }
 
-static hipError_t dispatch_lb(pfg_handle *h, int k, int mode, float *rho, float *ux, float *uy,
-                              float *uz, hipStream_t st) {
+static hipError_t dispatch_lb(pfg_handle *h, int mode, hipStream_t st) {
   LBArgs a;
-  make_lb_args(h, k, h->cur, &a);
+  make_lb_args(h, 0, h->cur, &a);
   switch (h->p.store) {
-    case PFG_STORE_F16: return launch_lb_s<PFG_STORE_F16>(h, a, mode, rho, ux, uy, uz, st);
-    case PFG_STORE_BF16: return launch_lb_s<PFG_STORE_BF16>(h, a, mode, rho, ux, uy, uz, st);
-    default: return launch_lb_s<PFG_STORE_F32>(h, a, mode, rho, ux, uy, uz, st);
+    case PFG_STORE_F16: return launch_lb_s<PFG_STORE_F16>(h, a, mode, st);
+    case PFG_STORE_BF16: return launch_lb_s<PFG_STORE_BF16>(h, a, mode, st);
+    default: return launch_lb_s<PFG_STORE_F32>(h, a, mode, st);
   }
 }
 
@@ -909,8 +910,7 @@ static hipError_t launch_lb_batch(pfg_handle *h, int mode, hipStream_t st) {
 
 hipError_t launch_lb(pfg_handle *h) {
   hipError_t e = h->K > 1 ? launch_lb_batch(h, LB_MODE_STEP, h->stream)
-                          : dispatch_lb(h, 0, LB_MODE_STEP, nullptr, nullptr, nullptr, nullptr,
-                                        h->stream);
+                          : dispatch_lb(h, LB_MODE_STEP, h->stream);
   if (e == hipSuccess) h->cur = 1 - h->cur;
   return e;
 }
@@ -919,13 +919,9 @@ hipError_t launch_lb_part(pfg_handle *h, int part, hipStream_t st) {
   if (!h->row_stamp) return hipErrorInvalidValue;
   const int mode = part == 1 ? LB_MODE_BULK : LB_MODE_REGION;
   hipError_t e = h->K > 1 ? launch_lb_batch(h, mode, st)
-                          : dispatch_lb(h, 0, mode, nullptr, nullptr, nullptr, nullptr, st);
+                          : dispatch_lb(h, mode, st);
   if (e == hipSuccess && part == 2) h->cur = 1 - h->cur;
   return e;
-}
-
-hipError_t launch_lb_fields(pfg_handle *h, int k, float *rho, float *ux, float *uy, float *uz) {
-  return dispatch_lb(h, k, LB_MODE_FIELDS, rho, ux, uy, uz, h->stream);
 }
 
 hipError_t launch_bbmask(pfg_handle *h, int k) {

@@ -396,8 +396,6 @@ hipError_t launch_lb(pfg_handle *h);
  * blocks they touch, with the IB force (then the copies of f alternate) */
 hipError_t launch_lb_part(pfg_handle *h, int part, hipStream_t s);
 hipError_t launch_bbmask(pfg_handle *h, int k);
-hipError_t launch_lb_fields(pfg_handle *h, int k, float *rho, float *ux, float *uy,
-                            float *uz);
 /* per_z: the inputs hold one value per z-plane of lattice k */
 hipError_t launch_init_eq(pfg_handle *h, int k, const float *rho, const float *ux,
                           const float *uy, const float *uz, bool per_z = false);
@@ -417,6 +415,27 @@ hipError_t fields_scratch_setup(int device, float **out_or_null);
 /* rho, ux, uy, uz of a single lattice to host (any may be NULL), window of
  * whole z-planes at a time through the fixed array */
 hipError_t download_fields_noalloc(pfg_handle *h, float *const host[4]);
+
+/* rho, ux, uy, uz of the cells [lo, hi) of lattice k, into windows of hi - lo
+ * values (nullptr: not wanted); solid cells read 0 */
+hipError_t launch_lb_fields_window(pfg_handle *h, int k, uint32_t lo, uint32_t hi,
+                                   float *const win[4]);
+
+/* frames.hip: to host arrays through pinned memory.  hipErrorOutOfMemory: no
+ * pinned buffer could be had, nothing was written. */
+struct Piece {
+  void *dst;        /* host                  */
+  const void *src;  /* device                */
+  size_t bytes;     /* a multiple of 4; 0: skipped */
+};
+hipError_t fetch_pieces(pfg_handle *h, const Piece *pieces, int n);
+hipError_t fetch_fields(pfg_handle *h, int k, float *const host[4]);
+/* the counters, the detach step and the step index, after the work enqueued
+ * so far */
+hipError_t fetch_report(pfg_handle *h, int64_t out[N_COUNTERS + 2]);
+/* every handle holds a reference; the last one frees the pinned buffers */
+void frames_ref();
+void frames_unref();
 
 /* markers.hip: fused marker-side launches, each with the roles it runs */
 void fill_mlat(const pfg_handle *h, int k, MLat *L);

@@ -104,6 +104,88 @@ def test_overlap_equals_serial_on_rows_that_share_blocks(gpu, nx):
         assert np.abs(res[0][1][k] - res[1][1][k]).max() < 1e-5, k
 
 
+def fibrin_cloud(pfg, n, nx=48):
+    """n free fibrin nodes without links on a small lattice."""
+    rng = np.random.default_rng(n)
+    P = (rng.random((3, n)) * nx).astype(np.float32)
+    p = pfg.default_params(nx=nx, ny=nx, nz=nx)
+    ma = ModelArrays(*P, kind=np.full(n, pfg.MARKER_FIBER), body=np.full(n, -1))
+    s = pfg.Solver(p)
+    s.load(ma.model)
+    s._keep = ma
+    return s, P
+
+
+@pytest.mark.parametrize("n", [1, 3, 29127, 29128, 233017, 300001])
+def test_frames_of_any_size(gpu, n):
+    """A frame of nine arrays goes through one small pinned buffer (up to 29127
+    markers: 1 MiB), one half of a large one (up to 233016: 8 MiB) or several, with
+    array and batch boundaries apart: every value arrives, exactly."""
+    pfg = gpu
+    s, P = fibrin_cloud(pfg, n)
+    with s:
+        rng = np.random.default_rng(1)
+        F, V = (rng.standard_normal((3, n)).astype(np.float32) for _ in range(2))
+        s.set_marker_forces(*F)
+        s.set_marker_velocities(*V)
+        for _ in range(2):
+            m = s.markers()
+            for names, want in (("xyz", P), (("vx", "vy", "vz"), V), (("fx", "fy", "fz"), F)):
+                for k, a in zip(names, want):
+                    assert np.array_equal(m[k], a), k
+
+
+def test_frames_from_several_threads(gpu):
+    """Handles in threads of their own download at once (buffers are shared by the
+    process, a call holds one): the same values as one after the other."""
+    import threading
+    pfg = gpu
+    solvers = []
+    for k in range(4):
+        p = pfg.default_params(nx=96 + 7 * k, ny=90, nz=80, store=k % 3)
+        p.body_force[0] = 1e-5
+        p.wall[1] = pfg.WALL_BOUNCE
+        s = pfg.Solver(p)
+        s.step(3 + k)
+        solvers.append(s)
+    want = [s.fields() for s in solvers]
+    bad = []
+
+    def work(k):
+        for _ in range(5):
+            got = solvers[k].fields()
+            if not all(np.array_equal(a, b) for a, b in zip(got, want[k])):
+                bad.append(k)
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for s in solvers:
+        s.close()
+    assert not bad
+
+
+def test_noalloc_fields_with_velocity_faces(gpu):
+    """Both field downloads impose the velocity faces: equal bit for bit."""
+    import ctypes as C
+    pfg = gpu
+    p = pfg.default_params(nx=40, ny=30, nz=20)
+    p.wall[0] = p.wall[1] = pfg.WALL_BOUNCE
+    p.wall[2] = pfg.WALL_VELOCITY
+    p.wall_u_lo[2][2] = p.wall_u_hi[2][2] = 0.04
+    with pfg.Solver(p) as s:
+        s.step(7)
+        want = s.fields()
+        got = [np.empty(s.N, np.float32) for _ in range(4)]
+        st = pfg.lib().pfg_download_fields_noalloc(
+            C.c_void_p(s._h.value), *[a.ctypes.data_as(C.POINTER(C.c_float)) for a in got])
+        assert st == 0
+        for a, b in zip(got, want):
+            assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("by_body", [1, 2])
 @pytest.mark.parametrize("staging", [1, 2, 3, 4])
 def test_markers_that_left_every_range(gpu, staging, by_body):
