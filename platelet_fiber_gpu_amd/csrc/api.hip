@@ -107,6 +107,7 @@ void free_markers(Markers &m) {
   dfree(m.tile_list); dfree(m.tile_count); dfree(m.spread_rec);
   dfree(m.body_range); dfree(m.rchunk_start); dfree(m.rchunk_items); dfree(m.tile_owner);
   dfree(m.body_spread); dfree(m.body_fallback); dfree(m.chunk_body); dfree(m.chunk_sum);
+  dfree(m.run_range); dfree(m.run_lo); dfree(m.run_hi); dfree(m.marker_runs);
   dfree(m.fbody_range); dfree(m.frest_items); dfree(m.fb_ref); dfree(m.fb_nlen); dfree(m.fb_nbr);
   dfree(m.fb_done);
   dfree(m.chunk_info);
@@ -952,6 +953,33 @@ pfg_status load_impl(pfg_handle *h, const pfg_model &M, const int32_t *minst,
         if (!in_body[(size_t)i]) frest_items.push_back(i);
       }
   }
+  /* runs of MORSE_RUN elements for the force pass with a wavefront per marker,
+   * when every platelet's elements are one run of indices */
+  std::vector<int32_t> run_range;
+  std::vector<int2> marker_runs((size_t)n, make_int2(0, 0));
+  {
+    std::set<std::pair<int, int>> seen;
+    bool ok = true;
+    for (int g0 = 0; g0 < n && ok;) {
+      int g1 = g0 + 1;
+      while (g1 < n && M.body[g1] == M.body[g0] && !(minst && minst[g1] != minst[g0])) ++g1;
+      bool elements = false;
+      for (int i = g0; i < g1; ++i) elements = elements || M.kind[i] == PFG_MARKER_ELEMENT;
+      if (elements) {
+        const int runs = (g1 - g0 + MORSE_RUN - 1) / MORSE_RUN, r0 = (int)run_range.size() / 2;
+        ok = M.body[g0] >= 0 && runs <= MORSE_RUNS_MAX &&
+             seen.insert({minst ? minst[g0] : 0, M.body[g0]}).second;
+        for (int i = g0; i < g1; ++i) marker_runs[(size_t)i] = make_int2(r0, runs);
+        for (int i = g0; i < g1; i += MORSE_RUN) {
+          run_range.push_back(i);
+          run_range.push_back(std::min(g1, i + MORSE_RUN));
+        }
+      }
+      g0 = g1;
+    }
+    if (!ok) run_range.clear();
+  }
+  m.n_runs = (int)run_range.size() / 2;
   m.n_fbodies = (int)(fbody_range.size() / 2);
   m.n_frest = (int)frest_items.size();
   m.fb_all_elements = m.n_fbodies > 0;
@@ -1250,6 +1278,12 @@ pfg_status load_impl(pfg_handle *h, const pfg_model &M, const int32_t *minst,
   ALLOC_FILL(m.tile_owner, ~(uint64_t)0, h->ntiles > 0 ? h->ntiles : 1);
   ALLOC_FILL(m.body_spread, (int32_t)-1, m.n_bodies > 0 ? m.n_bodies : 1);
   ALLOC_FILL(m.body_fallback, (int32_t)-1, m.n_bodies > 0 ? m.n_bodies : 1);
+  if (m.n_runs > 0) {
+    ALLOC_UP(m.run_range, run_range.data(), run_range.size());
+    ALLOC_UP(m.marker_runs, marker_runs.data(), marker_runs.size());
+    ALLOC_FILL(m.run_lo, make_float4(0.f, 0.f, 0.f, 0.f), m.n_runs);
+    ALLOC_FILL(m.run_hi, make_float4(0.f, 0.f, 0.f, 0.f), m.n_runs);
+  }
   if (minst) ALLOC_UP(m.minst, minst, n);
   ALLOC_FILL(m.bin_scatter, 0, n);
   ALLOC_FILL(m.sorted_pos, make_float4(0.f, 0.f, 0.f, 0.f), n);
@@ -1282,6 +1316,7 @@ pfg_status load_impl(pfg_handle *h, const pfg_model &M, const int32_t *minst,
     PFG_TRY(upload(h, h->d_lats, lats.data(), lats.size()));
   }
   h->h_step = 0;
+  h->cells_stale = false;
   h->model_loaded = true;
   return PFG_OK;
 }
@@ -1601,6 +1636,10 @@ pfg_status pfg_download_cells(pfg_handle *h, int32_t *bin_start, int32_t *bin_it
   if (!h) return PFG_ERR_ARG;
   if (!h->model_loaded) return PFG_ERR_STATE;
   hipSetDevice(h->device);
+  if (h->cells_stale) { /* the step needed other lists, or none */
+    PFG_TRY(launch_cells_again(h));
+    h->cells_stale = false;
+  }
   const int64_t nb = bin_elements(h) ? h->m.nbins : h->m.nbinsc;
   Piece p[2] = {{bin_start, h->m.bin_start, sizeof(int32_t) * ((size_t)nb + 1)},
                 {bin_items, h->m.bin_items, sizeof(int32_t) * (size_t)h->m.n}};
@@ -1622,6 +1661,7 @@ static hipError_t run_stage(pfg_handle *h, int s) {
   hipError_t e = hipSuccess;
   switch (s) {
     case PFG_STAGE_CELLS:
+      h->cells_stale = false;
       e = launch_begin(h, false, true);
       if (e == hipSuccess) e = launch_scan(h);
       if (e == hipSuccess) e = launch_place(h, true, false);
@@ -1660,26 +1700,32 @@ static hipError_t run_stage(pfg_handle *h, int s) {
  * lb0/lb1), one LB launch follows the spreading. */
 static hipError_t enqueue_step(pfg_handle *h, hipEvent_t lb0, hipEvent_t lb1) {
   hipError_t e = hipSuccess;
+  h->in_step = true;
   const bool markers = h->model_loaded && h->m.n > 0 && !h->fluid_only;
   const bool overlap = markers && h->overlap && h->row_stamp && !lb0 && !lb1;
   if (markers) {
-    e = launch_begin(h, false, true);
+    const bool lists = step_lists(h), sums = !sums_with_forces(h);
+    e = launch_begin(h, false, true, !lists);
     if (overlap) {
       if (e == hipSuccess) e = hipEventRecord(h->ev_fork, h->stream);
       if (e == hipSuccess) e = hipStreamWaitEvent(h->stream2, h->ev_fork, 0);
       if (e == hipSuccess) e = launch_lb_part(h, 1, h->stream2);
       if (e == hipSuccess) e = hipEventRecord(h->ev_join, h->stream2);
     }
-    if (e == hipSuccess) e = launch_scan(h);
-    if (e == hipSuccess) e = launch_place(h, true, true);
+    if (lists) {
+      if (e == hipSuccess) e = launch_scan(h);
+      if (e == hipSuccess) e = launch_place(h, true, true);
+    } else if (e == hipSuccess) {
+      e = launch_bend(h);
+    }
     bool resolved = false;
     /* the bin-sorted order serves the Morse gathers, the contact search and
      * the tile gather, none of which runs when the lists leave the elements
      * out */
-    if (e == hipSuccess) e = launch_gather(h, bin_elements(h), true, true, &resolved);
+    if (e == hipSuccess) e = launch_gather(h, step_bin_elements(h), sums, true, &resolved);
     if (e == hipSuccess && !resolved) e = launch_resolve(h);
     const bool fused = forces_can_spread(h);
-    if (e == hipSuccess) e = launch_forces(h, fused);
+    if (e == hipSuccess) e = launch_forces(h, fused, !sums);
     if (e == hipSuccess && !fused) e = launch_spread(h);
   }
   if (overlap) {
@@ -1691,6 +1737,7 @@ static hipError_t enqueue_step(pfg_handle *h, hipEvent_t lb0, hipEvent_t lb1) {
     if (e == hipSuccess && lb1) e = hipEventRecord(lb1, h->stream);
   }
   if (markers && e == hipSuccess) e = launch_move(h, true, true);
+  h->in_step = false;
   return e;
 }
 
@@ -1737,10 +1784,17 @@ static hipError_t read_report(pfg_handle *h, int64_t r[N_COUNTERS + 2]) {
   return e;
 }
 
+/* Whether pfg_download_cells has to bin again after these steps. */
+static void note_step_lists(pfg_handle *h, int nsteps) {
+  if (nsteps > 0 && h->model_loaded && h->m.n > 0 && !h->fluid_only)
+    h->cells_stale = !step_lists(h) || step_bin_elements(h) != bin_elements(h);
+}
+
 pfg_status pfg_step(pfg_handle *h, int nsteps, pfg_step_info *info) {
   if (!h || nsteps < 0) return PFG_ERR_ARG;
   hipSetDevice(h->device);
   if (h->use_graph && nsteps > 0 && !h->graph_valid) PFG_TRY(build_graphs(h));
+  note_step_lists(h, nsteps);
   int s = 0;
   if (h->use_graph) {
     for (; s + GRAPH_CHUNK <= nsteps; s += GRAPH_CHUNK) {
@@ -1886,6 +1940,7 @@ pfg_status pfg_profile(pfg_handle *h, int nsteps, double *ms_total, double *ms_l
   hipError_t e = hipEventCreate(&t0);
   if (e == hipSuccess) e = hipEventCreate(&t1);
   for (size_t k = 0; k < ev.size() && e == hipSuccess; ++k) e = hipEventCreate(&ev[k]);
+  note_step_lists(h, nsteps);
   if (e == hipSuccess) e = hipEventRecord(t0, h->stream);
   for (int s = 0; s < nsteps && e == hipSuccess; ++s) {
     e = enqueue_step(h, ev[2 * (size_t)s], ev[2 * (size_t)s + 1]);

@@ -84,6 +84,9 @@ struct MArgs {
   int bin_elements; /* 0: the cell lists hold the markers other than elements
                        (every element's Morse partners come from its
                        platelet's own lists and nothing else reads them) */
+  int by_runs;      /* 1: Morse candidates from the platelet's runs              */
+  int lists;        /* 1: the counting launch bins the markers                   */
+  int again;        /* 1: bin the positions the step started from (pos4)         */
   int spread_scratch; /* 1: the chunks of bodies write scratch boxes (form 4) */
   const int32_t *force_list; /* force_count >= 0: the force pass takes these */
   int force_count;           /* markers only; -1: every marker                */
@@ -108,7 +111,8 @@ constexpr float BOND_EPS_R = 1e-4f; /* |r - reach| below this: near-threshold  *
  * launch, so every lane reads the same value). */
 __device__ inline bool halted(const MArgs &a) { return a.halt && a.m.counters[1] != 0; }
 
-__device__ void spread_direct(const MArgs &a, int i, int lane, float Fx, float Fy, float Fz);
+__device__ void spread_direct(const MArgs &a, int i, int lane, int kind, float4 p, float Fx,
+                              float Fy, float Fz);
 /* body spreading's tile claims: workgroup `block` of the claim blocks the
  * force launch appends (blocks1 bodies, then blocks2 of 256 other markers) */
 __device__ void claim_role(const MArgs &a, int block);
@@ -374,45 +378,10 @@ __device__ inline float morse_tag(const MArgs &a, int j) {
   return __int_as_float(a.m.kind[j] == PFG_MARKER_ELEMENT ? a.m.body[j] : -1);
 }
 
-/* roles: A = clear this step's force tiles (blocks0 blocks, the CLEAR stage
- * only), B = count bins and pack each marker's position with its Morse tag
- * (blocks1), C = receptor positions (blocks2) */
-__global__ __launch_bounds__(256) void begin_kernel(MArgs a) {
-  int blk = blockIdx.x;
-  if (a.roles & ROLE_A) {
-    if (blk < a.blocks0) {
-      clear_tiles(a, blk);
-      return;
-    }
-    blk -= a.blocks0;
-  }
-  if (a.roles & ROLE_C) {
-    if (!(a.roles & ROLE_B) || blk >= a.blocks1) {
-      const int r = (blk - ((a.roles & ROLE_B) ? a.blocks1 : 0)) * 256 + threadIdx.x;
-      if (r < a.m.n_rec) {
-        float rp[3];
-        int nodes[3];
-        receptor_pos(a, r, rp, nodes);
-        const int lat = a.lats ? a.m.minst[nodes[0]] : 0;
-        a.m.rec_pos[r] = make_float4(rp[0], rp[1], rp[2], __int_as_float(lat));
-      }
-      return;
-    }
-  }
-  if (!(a.roles & ROLE_B)) return;
-  const int i = blk * 256 + threadIdx.x;
-  if (i == 0) {
-    a.m.counters[0] = 0;          /* bonds held, counted again this step      */
-    a.m.counters[6] = *a.m.d_step; /* this step's index, for the later launches
-                                     (the last one advances d_step)            */
-    a.m.counters[7] = 0;          /* platelet pairs in contact, found again    */
-  }
-  if (i >= a.m.n) return;
-  const MLat L = lat_of(a, i);
-  const int kind_i = a.m.kind[i];
-  const float4 p = make_float4(a.m.x[i], a.m.y[i], a.m.z[i],
-                               __int_as_float(kind_i == PFG_MARKER_ELEMENT ? a.m.body[i] : -1));
-  a.m.pos4[i] = p;
+__device__ void triangle_geometry(const MArgs &a, int t);
+
+/* Count marker i (position p) in its bin. */
+__device__ inline void bin_marker(const MArgs &a, int i, const MLat &L, int kind_i, float4 p) {
   const bool binned = a.bin_elements || kind_i != PFG_MARKER_ELEMENT;
   const MLat G = a.bin_elements ? L : coarse_grid(L); /* the lists' grid */
   int b3[3];
@@ -436,6 +405,88 @@ __global__ __launch_bounds__(256) void begin_kernel(MArgs a) {
       todo &= ~same;
     }
   }
+}
+
+/* Bounding box of run r: a wavefront, a lane per element. */
+__device__ void run_box(const MArgs &a, int r) {
+  const int lane = threadIdx.x & 63;
+  const int i = a.m.run_range[2 * r] + lane;
+  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  if (i < a.m.run_range[2 * r + 1]) {
+    lo[0] = hi[0] = a.m.x[i];
+    lo[1] = hi[1] = a.m.y[i];
+    lo[2] = hi[2] = a.m.z[i];
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      lo[k] = fminf(lo[k], __shfl_xor(lo[k], o, 64));
+      hi[k] = fmaxf(hi[k], __shfl_xor(hi[k], o, 64));
+    }
+  }
+  if (lane == 0) {
+    a.m.run_lo[r] = make_float4(lo[0], lo[1], lo[2], 0.f);
+    a.m.run_hi[r] = make_float4(hi[0], hi[1], hi[2], 0.f);
+  }
+}
+
+/* roles: A = clear this step's force tiles (blocks0 blocks, the CLEAR stage
+ * only), B = count bins and pack each marker's position with its Morse tag
+ * (blocks1), C = receptor positions (blocks2), D = bounding boxes of the
+ * runs, four per block, then triangle terms (blocks3, then the rest) */
+__global__ __launch_bounds__(256) void begin_kernel(MArgs a) {
+  int blk = blockIdx.x;
+  if (a.roles & ROLE_D) { /* the last blocks */
+    const int b = blk - (a.blocks0 + a.blocks1 + a.blocks2);
+    if (b >= 0) {
+      if (b < a.blocks3) {
+        const int r = b * 4 + (threadIdx.x >> 6);
+        if (r < a.m.n_runs) run_box(a, r);
+      } else {
+        const int t = (b - a.blocks3) * 256 + threadIdx.x;
+        if (t < a.m.n_tri) triangle_geometry(a, t);
+      }
+      return;
+    }
+  }
+  if (a.roles & ROLE_A) {
+    if (blk < a.blocks0) {
+      clear_tiles(a, blk);
+      return;
+    }
+    blk -= a.blocks0;
+  }
+  if (a.roles & ROLE_C) {
+    if (!(a.roles & ROLE_B) || blk >= a.blocks1) {
+      const int r = (blk - ((a.roles & ROLE_B) ? a.blocks1 : 0)) * 256 + threadIdx.x;
+      if (r < a.m.n_rec) {
+        float rp[3];
+        int nodes[3];
+        receptor_pos(a, r, rp, nodes);
+        const int lat = a.lats ? a.m.minst[nodes[0]] : 0;
+        a.m.rec_pos[r] = make_float4(rp[0], rp[1], rp[2], __int_as_float(lat));
+      }
+      return;
+    }
+  }
+  if (!(a.roles & ROLE_B)) return;
+  const int i = blk * 256 + threadIdx.x;
+  if (i == 0 && !a.again) {
+    a.m.counters[0] = 0;          /* bonds held, counted again this step      */
+    a.m.counters[6] = *a.m.d_step; /* this step's index, for the later launches
+                                     (the last one advances d_step)            */
+    a.m.counters[7] = 0;          /* platelet pairs in contact, found again    */
+  }
+  if (i >= a.m.n) return;
+  const MLat L = lat_of(a, i);
+  const int kind_i = a.m.kind[i];
+  const float4 p = a.again ? a.m.pos4[i]
+                           : make_float4(a.m.x[i], a.m.y[i], a.m.z[i],
+                                         __int_as_float(kind_i == PFG_MARKER_ELEMENT ? a.m.body[i]
+                                                                                     : -1));
+  if (!a.again) a.m.pos4[i] = p;
+  if (a.lists) bin_marker(a, i, L, kind_i, p);
   if (a.mark_rows && ib_coupled(a.m.kind[i], a.fiber_move) && !halted(a)) {
     /* stamp the rows of this step's 4x4x4 stencil (the nodes spreading and
      * interpolation use), so that the LB update of every other row may run
@@ -1570,9 +1621,45 @@ __device__ inline void element_terms(const MArgs &a, int i, int lane, float xi, 
   }
 }
 
+/* Morse force on marker i from the runs of its platelet whose boxes (run_box)
+ * come within the cutoff: lane r tests run r, then the wavefront takes two
+ * runs at a time, a lane per element.  The box distance is built from the
+ * differences and in the order of the pair distance, so no pair within the
+ * cutoff (or its counted vicinity) is left out by rounding.  Elements of one
+ * platelet lie along its surface in index order, so a marker meets a few of
+ * its runs: about the candidates the cell lists gave, without a count, a scan
+ * and a scatter in front of the force launch. */
+__device__ inline void morse_runs(const MArgs &a, int i, float4 pi, int lane, float &fx,
+                                  float &fy, float &fz) {
+  const int2 runs = a.m.marker_runs[i];
+  bool near = false;
+  if (lane < runs.y) {
+    const float4 lo = a.m.run_lo[runs.x + lane], hi = a.m.run_hi[runs.x + lane];
+    const float dx = fmaxf(fmaxf(lo.x - pi.x, pi.x - hi.x), 0.f);
+    const float dy = fmaxf(fmaxf(lo.y - pi.y, pi.y - hi.y), 0.f);
+    const float dz = fmaxf(fmaxf(lo.z - pi.z, pi.z - hi.z), 0.f);
+    near = fmaf(dz, dz, fmaf(dy, dy, dx * dx)) < a.morse_cut2 + a.morse_eps2;
+  }
+  const int m0 = a.m.run_range[2 * runs.x];
+  const int m1 = a.m.run_range[2 * (runs.x + runs.y - 1) + 1];
+  for (uint64_t todo = __ballot(near); todo != 0;) {
+    const int j0 = m0 + MORSE_RUN * (__ffsll((unsigned long long)todo) - 1) + lane;
+    todo &= todo - 1;
+    const bool two = todo != 0;
+    const int j1 = two ? m0 + MORSE_RUN * (__ffsll((unsigned long long)todo) - 1) + lane : 0;
+    todo &= todo - 1; /* zero stays zero */
+    const bool in0 = j0 < m1, in1 = two && j1 < m1;
+    float4 p0 = pi, p1 = pi;
+    if (in0) p0 = a.m.pos4[j0];
+    if (in1) p1 = a.m.pos4[j1];
+    if (in0) morse_pair(a, p0, pi.w, pi.x, pi.y, pi.z, fx, fy, fz);
+    if (in1) morse_pair(a, p1, pi.w, pi.x, pi.y, pi.z, fx, fy, fz);
+  }
+}
+
 /* A group of G lanes per marker (G = 64: one wavefront, markers in index
  * order, the Morse candidates of all neighbour ranges flattened over the
- * lanes; G < 64: markers in bin-sorted order, so that the groups of a
+ * lanes, or the runs of the platelet; G < 64: markers in bin-sorted order, so that the groups of a
  * wavefront mostly share their neighbour bins and read the same packed
  * positions, each group striding through the ranges).  The lanes of a group
  * then stride over the marker's CSR lists (triangles, edges, receptor
@@ -1580,8 +1667,10 @@ __device__ inline void element_terms(const MArgs &a, int i, int lane, float xi, 
 template <int G, bool SPREAD = false>
 __global__ __launch_bounds__(256) void forces_kernel(MArgs a) {
   static_assert(!SPREAD || G == 64, "spreading takes a lane per stencil node");
-  if ((int)blockIdx.x >= a.blocks0 && a.blocks1 + a.blocks2 > 0) { /* whole workgroups */
-    claim_role(a, (int)blockIdx.x - a.blocks0);
+  if ((int)blockIdx.x >= a.blocks0 && a.blocks1 + a.blocks2 + a.blocks3 > 0) {
+    const int b = (int)blockIdx.x - a.blocks0; /* whole workgroups */
+    if (b < a.blocks3) platelet_sums(a, b);
+    else claim_role(a, b - a.blocks3);
     return;
   }
   const int lane = threadIdx.x & (G - 1);
@@ -1607,7 +1696,9 @@ __global__ __launch_bounds__(256) void forces_kernel(MArgs a) {
   float fx = 0.f, fy = 0.f, fz = 0.f;
   if (kind == PFG_MARKER_ELEMENT) {
     const int body = a.m.body[i];
-    if (a.morse_u0 != 0.f) {
+    if (G == 64 && a.by_runs) {
+      if (a.morse_u0 != 0.f) morse_runs(a, i, pi, lane, fx, fy, fz);
+    } else if (a.morse_u0 != 0.f) {
       const MLat L = lat_of(a, i);
       const int b = a.m.marker_bin[i] - L.bin0;
       const int b3[3] = {b % L.nb[0], (b / L.nb[0]) % L.nb[1], b / (L.nb[0] * L.nb[1])};
@@ -1666,7 +1757,7 @@ __global__ __launch_bounds__(256) void forces_kernel(MArgs a) {
   }
   /* the wavefront holds the marker's whole force: spread it at once, a
    * lane per stencil node (the direct form, without another launch) */
-  if constexpr (SPREAD) spread_direct(a, i, lane, fx, fy, fz);
+  if constexpr (SPREAD) spread_direct(a, i, lane, kind, pi, fx, fy, fz);
 }
 
 /* Force pass by body: a workgroup of BODY_THREADS lanes per body (a
@@ -2132,12 +2223,13 @@ __device__ inline void stamp_stencil_tile(const MLat &L, int kx, int ky, int kz,
 
 /* Direct spreading of marker i: lane = stencil node (consecutive lanes take
  * consecutive x, so one atomic instruction covers 16 runs of 4 nodes). */
-__device__ void spread_direct(const MArgs &a, int i, int lane, float Fx, float Fy, float Fz) {
-  if (!ib_coupled(a.m.kind[i], a.fiber_move)) return;
+__device__ void spread_direct(const MArgs &a, int i, int lane, int kind, float4 p, float Fx,
+                              float Fy, float Fz) {
+  if (!ib_coupled(kind, a.fiber_move)) return;
   const MLat L = lat_of(a, i);
-  const float X = wrap_coord(a.m.x[i], L.nx, L.periodic[0]);
-  const float Y = wrap_coord(a.m.y[i], L.ny, L.periodic[1]);
-  const float Z = wrap_coord(a.m.z[i], L.nz, L.periodic[2]);
+  const float X = wrap_coord(p.x, L.nx, L.periodic[0]);
+  const float Y = wrap_coord(p.y, L.ny, L.periodic[1]);
+  const float Z = wrap_coord(p.z, L.nz, L.periodic[2]);
   float wx, wy, wz;
   const int ix = stencil_node(X, lane & 3, L.nx, L.periodic[0], &wx);
   const int iy = stencil_node(Y, (lane >> 2) & 3, L.ny, L.periodic[1], &wy);
@@ -2153,7 +2245,8 @@ __device__ void spread_direct(const MArgs &a, int i, int lane, float Fx, float F
 }
 
 __device__ inline void spread_direct(const MArgs &a, int i, int lane) {
-  spread_direct(a, i, lane, a.m.fx[i], a.m.fy[i], a.m.fz[i]);
+  spread_direct(a, i, lane, a.m.kind[i], make_float4(a.m.x[i], a.m.y[i], a.m.z[i], 0.f),
+                a.m.fx[i], a.m.fy[i], a.m.fz[i]);
 }
 
 /* One wavefront per marker. */
@@ -3527,6 +3620,8 @@ void fill_mlat(const pfg_handle *h, int k, MLat *L) {
   L->marker0 = I.marker0;
 }
 
+static bool by_runs(const pfg_handle *h);
+
 static void make_margs(const pfg_handle *h, MArgs *a) {
   const pfg_params &p = h->p;
   a->m = h->m;
@@ -3584,7 +3679,10 @@ static void make_margs(const pfg_handle *h, MArgs *a) {
   a->resolve_last = 0;
   a->count_spans = 0;
   a->spread_scratch = 0;
-  a->bin_elements = bin_elements(h) ? 1 : 0;
+  a->bin_elements = (h->in_step ? step_bin_elements(h) : bin_elements(h)) ? 1 : 0;
+  a->lists = 1;
+  a->again = 0;
+  a->by_runs = by_runs(h) ? 1 : 0;
   a->force_list = nullptr;
   a->force_count = -1;
   a->move_list = nullptr;
@@ -3599,26 +3697,50 @@ static inline int blocks_for(int64_t n, int per_block) {
 /* Few markers: the counting launch adds the span totals itself. */
 static bool count_spans(const pfg_handle *h) { return h->m.n < SPAN_COUNT_MAX; }
 
-hipError_t launch_begin(pfg_handle *h, bool clear, bool count) {
+hipError_t launch_begin(pfg_handle *h, bool clear, bool count, bool geometry) {
   MArgs a;
   make_margs(h, &a);
   const bool recs = count && h->m.n_rec > 0;
   count = count && h->m.n > 0;
-  a.count_spans = count && count_spans(h);
-  a.roles = (clear ? ROLE_A : 0) | (count ? ROLE_B : 0) | (recs ? ROLE_C : 0);
+  geometry = geometry && h->m.n_tri > 0;
+  a.lists = !h->in_step || step_lists(h);
+  a.count_spans = count && a.lists && count_spans(h);
+  const bool boxes = count && a.by_runs;
+  a.roles = (clear ? ROLE_A : 0) | (count ? ROLE_B : 0) | (recs ? ROLE_C : 0) |
+            (boxes || geometry ? ROLE_D : 0);
   a.blocks0 = clear ? blocks_for(h->ntiles, 256) : 0;
   a.blocks1 = count ? blocks_for(h->m.n, 256) : 0;
   a.blocks2 = recs ? blocks_for(h->m.n_rec, 256) : 0;
-  const int grid = a.blocks0 + a.blocks1 + a.blocks2;
+  a.blocks3 = boxes ? blocks_for(h->m.n_runs, 4) : 0;
+  const int grid = a.blocks0 + a.blocks1 + a.blocks2 + a.blocks3 +
+                   (geometry ? blocks_for(h->m.n_tri, 256) : 0);
   if (grid == 0) return hipSuccess;
   hipLaunchKernelGGL(begin_kernel, dim3(grid), dim3(256), 0, h->stream, a);
   return hipGetLastError();
 }
 
+hipError_t launch_cells_again(pfg_handle *h) {
+  if (h->m.n == 0) return hipSuccess;
+  MArgs a;
+  make_margs(h, &a);
+  a.again = 1;
+  a.count_spans = count_spans(h);
+  a.roles = ROLE_B;
+  a.blocks1 = blocks_for(h->m.n, 256);
+  a.mark_rows = 0;
+  hipLaunchKernelGGL(begin_kernel, dim3(a.blocks1), dim3(256), 0, h->stream, a);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = launch_scan(h);
+  if (e == hipSuccess) e = launch_place(h, true, false);
+  if (e == hipSuccess) e = launch_gather(h, true, false, false);
+  return e;
+}
+
 hipError_t launch_scan(pfg_handle *h) {
   const Markers &m = h->m;
   if (m.n == 0) return hipSuccess;
-  const bool full = bin_elements(h); /* else the coarse grid */
+  /* else the coarse grid */
+  const bool full = h->in_step ? step_bin_elements(h) : bin_elements(h);
   const int64_t blocks = full ? m.scan_blocks : m.scan_blocks_c;
   if (!count_spans(h))
     hipLaunchKernelGGL(scan_reduce_kernel, dim3((unsigned)blocks), dim3(256), 0, h->stream,
@@ -3639,12 +3761,19 @@ hipError_t launch_place(pfg_handle *h, bool scatter, bool geometry) {
   const int grid = a.blocks0 + a.blocks1;
   if (grid == 0) return hipSuccess;
   hipLaunchKernelGGL(place_kernel, dim3(grid), dim3(256), 0, h->stream, a);
-  if (geometry && h->m.bend) { /* node normals, then the mean curvature */
-    a.blocks0 = blocks_for((int64_t)h->m.n * BEND_LANES, 256);
-    hipLaunchKernelGGL(bend_normal_kernel, dim3(a.blocks0 + blocks_for(h->m.n_tedges, 256)),
-                       dim3(256), 0, h->stream, a);
-    hipLaunchKernelGGL(bend_km_kernel, dim3(a.blocks0), dim3(256), 0, h->stream, a);
-  }
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess && geometry ? launch_bend(h) : e;
+}
+
+/* node normals, then the mean curvature */
+hipError_t launch_bend(pfg_handle *h) {
+  if (!h->m.bend) return hipSuccess;
+  MArgs a;
+  make_margs(h, &a);
+  a.blocks0 = blocks_for((int64_t)h->m.n * BEND_LANES, 256);
+  hipLaunchKernelGGL(bend_normal_kernel, dim3(a.blocks0 + blocks_for(h->m.n_tedges, 256)),
+                     dim3(256), 0, h->stream, a);
+  hipLaunchKernelGGL(bend_km_kernel, dim3(a.blocks0), dim3(256), 0, h->stream, a);
   return hipGetLastError();
 }
 
@@ -3703,6 +3832,26 @@ static bool contact_on(const pfg_handle *h) {
   return h->m.contact_slot && h->p.contact_a != 0.f && h->m.n_plt >= 2;
 }
 
+/* A wavefront per marker takes its Morse candidates from its platelet's runs. */
+static bool by_runs(const pfg_handle *h) {
+  return h->m.n_runs > 0 && forces_lanes(h) == 64 &&
+         !(forces_by_body(h) && !forces_can_spread(h));
+}
+
+bool step_bin_elements(const pfg_handle *h) {
+  return contact_on(h) || spread_form(h) == 3 || (bin_elements(h) && !by_runs(h));
+}
+
+bool step_lists(const pfg_handle *h) {
+  return step_bin_elements(h) || (h->m.fibrin_lig && h->m.n_rec > 0);
+}
+
+/* The force launch reads the platelet sums for the area and volume forces and
+ * the lowest element for the wall repulsion only. */
+bool sums_with_forces(const pfg_handle *h) {
+  return h->m.n_rec == 0 && h->p.ks == 0.f && h->p.kv == 0.f && h->p.wall_rep_a == 0.f;
+}
+
 /* Whether the cell lists hold the elements: not when the step's force pass
  * takes every element's Morse partners from its platelet's own lists (the
  * pass by body, which the step runs unless the force pass spreads too) and
@@ -3721,7 +3870,7 @@ bool forces_can_spread(const pfg_handle *h) {
          !contact_on(h) && !h->halt_on_detach;
 }
 
-hipError_t launch_forces(pfg_handle *h, bool spread) {
+hipError_t launch_forces(pfg_handle *h, bool spread, bool sums) {
   if (h->m.n == 0) return hipSuccess;
   MArgs a;
   make_margs(h, &a);
@@ -3734,9 +3883,13 @@ hipError_t launch_forces(pfg_handle *h, bool spread) {
   /* at least one workgroup: the first one makes the detach test */
   unsigned grid = (unsigned)std::max(
       1, blocks_for((int64_t)(by_body ? h->m.n_frest : h->m.n) * G, 256));
+  a.blocks0 = (int)grid;
+  if (sums) { /* the platelet sums, which nothing in this launch reads */
+    a.blocks3 = h->m.n_plt;
+    grid += (unsigned)a.blocks3;
+  }
   if (!spread && spread_form(h) == 4) {
-    /* the body spreading's tile claims, in workgroups after the markers' */
-    a.blocks0 = (int)grid;
+    /* the body spreading's tile claims, in the last workgroups */
     a.blocks1 = h->m.n_bodies;
     a.blocks2 = blocks_for(h->m.n_ritems, 256);
     grid += (unsigned)(a.blocks1 + a.blocks2);

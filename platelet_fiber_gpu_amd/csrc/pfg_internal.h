@@ -52,6 +52,11 @@ constexpr int FB_BINS = 2048;
  * cutoff plus a skin of FB_SKIN cutoffs */
 constexpr int FB_NBR_MAX = 64;
 constexpr float FB_SKIN = 0.25f;
+/* Force pass with a wavefront per marker: its platelet's elements are taken
+ * 64 at a time (a run of the index order), and runs whose bounding box is
+ * beyond the Morse cutoff are skipped; a lane tests a box, so a platelet has
+ * at most 64 runs */
+constexpr int MORSE_RUN = 64, MORSE_RUNS_MAX = 64;
 /* lanes of the per-body workgroups (force pass, second spreading pass) */
 constexpr int BODY_THREADS = 1024;
 /* Marker count from which spreading is staged through LDS by default. */
@@ -283,6 +288,15 @@ struct Markers {
   int16_t *fb_nbr = nullptr;
   int32_t *fb_done = nullptr;    /* per body: the step whose forces the build
                                     kernel summed (its lists overflowed)     */
+  /* runs of MORSE_RUN elements of a platelet: per run its markers
+   * [run_range[2r], run_range[2r+1]) and this step's bounding box; per marker
+   * the first run of its platelet and their number (0: not an element).
+   * n_runs = 0 when some platelet's elements are no single run of indices,
+   * or too many */
+  int n_runs = 0;
+  int32_t *run_range = nullptr;
+  float4 *run_lo = nullptr, *run_hi = nullptr;
+  int2 *marker_runs = nullptr;
   SpreadRec *spread_rec = nullptr; /* per cell-list slot: the marker's record */
   int tile_gather_ok = 0;
   /* platelet-platelet contact: per platelet pair (lo * n_plt + hi) the best
@@ -351,6 +365,9 @@ struct pfg_handle {
   int lb_xcd_rows = 0;         /* LB launch: contiguous rows per XCD        */
   pfg::Markers m;
   bool model_loaded = false;
+  bool in_step = false;        /* launches of a whole step (not of a stage)     */
+  bool cells_stale = false;    /* the last step kept other cell lists than
+                                  pfg_download_cells gives, or none             */
   bool fluid_only = false;
   bool halt_on_detach = false; /* steps after the detach test fired change nothing */
   int ib_staging = 0;          /* spreading: 0 auto, 1 LDS-staged chunks, 2 direct */
@@ -439,7 +456,11 @@ void frames_unref();
 
 /* markers.hip: fused marker-side launches, each with the roles it runs */
 void fill_mlat(const pfg_handle *h, int k, MLat *L);
-hipError_t launch_begin(pfg_handle *h, bool clear, bool count);
+hipError_t launch_begin(pfg_handle *h, bool clear, bool count, bool geometry = false);
+/* the cell lists of the positions the last step started from */
+hipError_t launch_cells_again(pfg_handle *h);
+/* the bending chain's normals and curvature, after the triangle terms */
+hipError_t launch_bend(pfg_handle *h);
 hipError_t launch_scan(pfg_handle *h);
 hipError_t launch_place(pfg_handle *h, bool scatter, bool geometry);
 /* resolved != nullptr: resolve the bonds in the same launch when there are
@@ -448,10 +469,15 @@ hipError_t launch_gather(pfg_handle *h, bool sort, bool sums, bool decide,
                          bool *resolved = nullptr);
 hipError_t launch_resolve(pfg_handle *h);
 /* spread = true: the force pass also spreads (only when forces_can_spread) */
-hipError_t launch_forces(pfg_handle *h, bool spread = false);
-/* whether the step's cell lists hold the elements (else only the other
- * markers, and the step needs no bin-sorted order) */
+hipError_t launch_forces(pfg_handle *h, bool spread = false, bool sums = false);
+/* whether the cell lists that pfg_download_cells gives hold the elements (else
+ * only the other markers) */
 bool bin_elements(const pfg_handle *h);
+/* whether a step's own lists do, whether a step needs lists at all, and
+ * whether its platelet sums can go with the force launch */
+bool step_bin_elements(const pfg_handle *h);
+bool step_lists(const pfg_handle *h);
+bool sums_with_forces(const pfg_handle *h);
 bool forces_can_spread(const pfg_handle *h);
 hipError_t launch_spread(pfg_handle *h);
 hipError_t launch_move(pfg_handle *h, bool interp, bool update);
