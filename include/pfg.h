@@ -395,8 +395,9 @@ pfg_status pfg_set_fluid_only(pfg_handle *h, int fluid_only);
  * reports the steps that ran.  Default 0: stepping continues after detach. */
 pfg_status pfg_set_halt_on_detach(pfg_handle *h, int enable);
 /* IB spreading form (LB_kernel.cu:1419-1520 restated four ways): 0 automatic
- * (4 from 32768 markers up when the model has compact platelets, else 1
- * there; 2 below), 1 always staged (a workgroup per run
+ * (4 from 2^20 markers up when the model has compact platelets; else 1 from
+ * 2560 markers up, or from 1280 where the force pass cannot spread itself; 2
+ * below), 1 always staged (a workgroup per run
  * of up to 128 markers of one platelet accumulates them in LDS first),
  * 2 always direct (FP32 atomics per marker and node), 3 tile gather (a
  * wavefront per 4x4x4 tile that this step's stencils meet sums the
@@ -415,13 +416,14 @@ pfg_status pfg_set_halt_on_detach(pfg_handle *h, int enable);
 pfg_status pfg_set_ib_staging(pfg_handle *h, int mode);
 /* Lanes per marker in the SEM/fibrin force pass (sem_Force_kernel,
  * sem_kernel.cu:320-513, with the Morse pairs over the cell lists): 0
- * automatic (64 below 32768 markers, else 4), or 1, 2, 4, 8, 16, 32 or 64.  With
+ * automatic (64 below 65536 markers, else 4), or 1, 2, 4, 8, 16, 32 or 64.  With
  * fewer than 64 the markers are taken in cell-list order.  Same result up
  * to FP32 summation order. */
 pfg_status pfg_set_forces_lanes(pfg_handle *h, int lanes);
 /* Force pass by body (sem_Force_kernel's Morse term, sem_kernel.cu:320-513,
- * acts between the elements of one platelet): 0 automatic (on from 32768
- * markers), 1 on, 2 off.  On: a workgroup per platelet of at most 2048
+ * acts between the elements of one platelet): 0 automatic (on from 65536
+ * markers, and from 32768 where fewer than 64 lanes per marker are set), 1
+ * on, 2 off.  On: a workgroup per platelet of at most 2048
  * elements sorts its positions into a cell list of its own in LDS and sums
  * each element's Morse pairs there, then its other terms; the other
  * markers take the per-marker pass (pfg_set_forces_lanes).  It applies

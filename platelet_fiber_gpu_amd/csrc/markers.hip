@@ -3805,31 +3805,48 @@ hipError_t launch_resolve(pfg_handle *h) {
   return hipGetLastError();
 }
 
-/* spreading form: 1 staged chunks, 2 direct, 3 tile gather, 4 by body */
-static int spread_form(const pfg_handle *h) {
-  if (h->ib_staging == 3 && !h->m.tile_gather_ok) return 1;
-  if (h->ib_staging == 4 && h->m.n_bodies == 0) return 1;
-  if (h->ib_staging) return h->ib_staging;
-  return h->m.n >= IB_STAGED_MIN ? (h->m.n_bodies > 0 ? 4 : 1) : 2;
-}
-
-static bool staged_spreading(const pfg_handle *h) { return spread_form(h) != 2; }
-
 static int forces_lanes(const pfg_handle *h) {
   /* few markers: a wavefront each, for parallelism; many: 4 lanes each in
    * bin order, for fewer instructions per marker */
   return h->forces_lanes ? h->forces_lanes : (h->m.n >= FORCES_SORTED_MIN ? 4 : 64);
 }
 
+static bool contact_on(const pfg_handle *h) {
+  return h->m.contact_slot && h->p.contact_a != 0.f && h->m.n_plt >= 2;
+}
+
+/* The force pass could spread direct stencils itself: it has a wavefront per
+ * marker, no later pass adds to the forces (bending, contact) and no detach
+ * halt can stop the step midway. */
+static bool spread_rides_along(const pfg_handle *h) {
+  return h->m.n > 0 && forces_lanes(h) == 64 && !h->m.bend && !contact_on(h) &&
+         !h->halt_on_detach;
+}
+
+/* spreading form: 1 staged chunks, 2 direct, 3 tile gather, 4 by body */
+static int spread_form(const pfg_handle *h) {
+  if (h->ib_staging == 3 && !h->m.tile_gather_ok) return 1;
+  if (h->ib_staging == 4 && h->m.n_bodies == 0) return 1;
+  if (h->ib_staging) return h->ib_staging;
+  /* staged rather than by body: 500 platelets in the tube 1056 against 1080 us
+   * per step, a batch of 256 lattices 2076 against 2112.  From SPREAD_BODY_MIN
+   * markers by body, whose sums have a fixed order where a platelet meets a
+   * tile alone, so that runs in 16-bit storage repeat closely, for 0.7 % of a
+   * step: 2000 platelets in 1024x512x512 5201 against 5165 us. */
+  if (h->m.n >= SPREAD_BODY_MIN && h->m.n_bodies > 0) return 4;
+  return h->m.n >= (spread_rides_along(h) ? IB_STAGED_MIN : IB_STAGED_MIN_ALONE) ? 1 : 2;
+}
+
+static bool staged_spreading(const pfg_handle *h) { return spread_form(h) != 2; }
+
 /* the force pass by body: automatic with many markers, when the model has
  * such bodies */
 static bool forces_by_body(const pfg_handle *h) {
   if (h->m.n_fbodies == 0 || h->forces_body == 2) return false;
-  return h->forces_body == 1 || h->m.n >= FORCES_SORTED_MIN;
-}
-
-static bool contact_on(const pfg_handle *h) {
-  return h->m.contact_slot && h->p.contact_a != 0.f && h->m.n_plt >= 2;
+  if (h->forces_body == 1) return true;
+  /* a wavefront per marker by choice of the library comes first */
+  const bool runs = h->forces_lanes == 0 && h->m.n < FORCES_SORTED_MIN && h->m.n_runs > 0;
+  return h->m.n >= BY_BODY_MIN && !runs;
 }
 
 /* A wavefront per marker takes its Morse candidates from its platelet's runs. */
@@ -3839,7 +3856,8 @@ static bool by_runs(const pfg_handle *h) {
 }
 
 bool step_bin_elements(const pfg_handle *h) {
-  return contact_on(h) || spread_form(h) == 3 || (bin_elements(h) && !by_runs(h));
+  const bool body_pass = forces_by_body(h) && !forces_can_spread(h) && h->m.fb_all_elements;
+  return contact_on(h) || spread_form(h) == 3 || !(by_runs(h) || body_pass);
 }
 
 bool step_lists(const pfg_handle *h) {
@@ -3854,20 +3872,18 @@ bool sums_with_forces(const pfg_handle *h) {
 
 /* Whether the cell lists hold the elements: not when the step's force pass
  * takes every element's Morse partners from its platelet's own lists (the
- * pass by body, which the step runs unless the force pass spreads too) and
- * no contact search or tile gather reads the lists (then only the fibrin
- * ligand search does). */
+ * pass by body, where the force pass does not spread too, or at its sizes the
+ * runs) and no contact search or tile gather reads the lists (then only the
+ * fibrin ligand search does). */
 bool bin_elements(const pfg_handle *h) {
-  const bool body_pass = forces_by_body(h) && !forces_can_spread(h);
+  const bool body_pass = h->m.n_fbodies > 0 && h->forces_body != 2 &&
+                         (h->forces_body == 1 || h->m.n >= BY_BODY_MIN) &&
+                         !forces_can_spread(h);
   return !(body_pass && h->m.fb_all_elements && !contact_on(h) && spread_form(h) != 3);
 }
 
-/* The force pass can spread each marker's force itself when it has a
- * wavefront per marker, spreading is direct, no later pass adds to the
- * forces (bending, contact) and no detach halt can stop the step midway. */
 bool forces_can_spread(const pfg_handle *h) {
-  return h->m.n > 0 && forces_lanes(h) == 64 && !staged_spreading(h) && !h->m.bend &&
-         !contact_on(h) && !h->halt_on_detach;
+  return spread_rides_along(h) && !staged_spreading(h);
 }
 
 hipError_t launch_forces(pfg_handle *h, bool spread, bool sums) {

@@ -59,11 +59,23 @@ constexpr float FB_SKIN = 0.25f;
 constexpr int MORSE_RUN = 64, MORSE_RUNS_MAX = 64;
 /* lanes of the per-body workgroups (force pass, second spreading pass) */
 constexpr int BODY_THREADS = 1024;
-/* Marker count from which spreading is staged through LDS by default. */
-constexpr int IB_STAGED_MIN = 32768;
-/* Marker count from which the forces take 4 lanes per marker in bin order
- * (below it, a wavefront per marker). */
-constexpr int FORCES_SORTED_MIN = 32768;
+/* Marker counts from which spreading is staged through LDS by default: when
+ * the force launch could spread as well, and when spreading is a launch of its
+ * own anyway.  us per step, direct / staged, on 160x96x96 FP32: fused 1536
+ * markers 60.5 / 62.8, 2048 62.0 / 64.4, 3000 66.9 / 62.6, 6000 77 / 66; own
+ * launch 1024 62.0 / 62.7, 1536 65.2 / 63.6, 2048 67.7 / 65.3. */
+constexpr int IB_STAGED_MIN = 2560, IB_STAGED_MIN_ALONE = 1280;
+/* ... and from which it goes by body when the model has compact platelets. */
+constexpr int SPREAD_BODY_MIN = 1 << 20;
+/* Marker count from which the forces take 4 lanes per marker in bin order, or
+ * the pass by body where it applies (below it, a wavefront per marker).  us
+ * per step, wavefront / by body: 31 200 markers 187 / 224, 46 800 246 / 259,
+ * 83 200 442 / 441, 156 000 497 / 477. */
+constexpr int FORCES_SORTED_MIN = 65536;
+/* Marker count from which the force pass by body is taken without being asked
+ * for (where the library does not take a wavefront per marker), and
+ * pfg_download_cells leaves the elements of such models out. */
+constexpr int BY_BODY_MIN = 32768;
 /* Receptor count up to which the cell-list/bond launch resolves the bonds
  * itself (its last workgroup takes them all). */
 constexpr int RESOLVE_IN_GATHER_MAX = 2048;

@@ -211,3 +211,74 @@ def test_markers_that_left_every_range(gpu, staging, by_body):
         m = s.markers()
     assert all(np.isfinite(m[k][healthy]).all() for k in ("x", "y", "z", "fx", "fy", "fz"))
     assert (m["z"][first] < -2e9).all()
+
+
+def cloud_model(sizes, nx=48):
+    """Platelets of `sizes` elements as random clouds, about 20 Morse partners each."""
+    rng = np.random.default_rng(sum(sizes))
+    P, body = [], []
+    for b, n in enumerate(sizes):
+        side = 0.72 * n ** (1 / 3)
+        P.append(rng.random((n, 3)) * side + rng.random(3) * (nx - 1))
+        body += [b] * n
+    P, body = np.concatenate(P), np.array(body)
+    start = np.concatenate([[0], np.cumsum(sizes)])
+    return ModelArrays(*P.T, body=body, plt_elem_start=start,
+                       plt_tri_start=np.zeros(len(sizes) + 1), tri_S0=[],
+                       plt_S0=np.ones(len(sizes)), plt_V0=np.ones(len(sizes)))
+
+
+@pytest.mark.parametrize("sizes", [(1, 2), (63, 64, 65), (127, 1, 128, 129), (4096,), (4097, 70)])
+def test_morse_from_runs_of_the_platelet(gpu, sizes):
+    """A wavefront per marker takes its Morse candidates from runs of 64 elements
+    (part runs, several platelets in turn, the longest platelet that has a lane per
+    run), or from the cell lists where a platelet is longer: the forces of the 4-lane
+    pass over the cell lists, to the rounding of sums of some 20 terms of up to 80."""
+    pfg = gpu
+    ma = cloud_model(sizes)
+    p = pfg.default_params(nx=48, ny=48, nz=48, bin_cells=2)
+    p.morse_u0, p.morse_cutoff = 1.0, 1.2
+    p.wall[2] = pfg.WALL_BOUNCE
+    F = []
+    for lanes in (64, 4):
+        with pfg.Solver(p) as s:
+            s.load(ma.model)
+            s.set_forces_by_body(2)
+            s.set_forces_lanes(lanes)
+            for st in (pfg.STAGE_CELLS, pfg.STAGE_MEMBRANE, pfg.STAGE_FORCES):
+                s.stage(st)
+            m = s.markers()
+            F.append(np.stack([m["fx"], m["fy"], m["fz"]]))
+    assert np.abs(F[0] - F[1]).max() <= 1e-5 * max(1.0, np.abs(F[1]).max())
+    assert sum(sizes) < 4 or np.abs(F[1]).max() > 0
+
+
+@pytest.mark.parametrize("by_body", [0, 1])
+def test_cell_lists_after_steps_without_them(gpu, by_body):
+    """Steps that need no cell lists keep none; asked for afterwards, they are those
+    of the positions the last step started from, as the CELLS stage gives them."""
+    pfg = gpu
+    sc = pfg.Scene(pfg.SCENE_LARGE, nx=96, ny=64, nz=64, n_platelets=3, elements=200,
+                   receptors=-1, ligands=-1, fibrin_nodes=128, fibrin_links=150)
+    with pfg.Solver(sc.params) as s:
+        s.load(sc)
+        s.set_forces_by_body(by_body)
+        s.set_forces_lanes(4 if by_body else 0)  # 0: a wavefront each, which spreads too
+        s.step(3)
+        m = s.markers()
+        s.step(1)
+        got = s.cells()
+    with pfg.Solver(sc.params) as s:
+        s.load(sc)
+        s.set_forces_by_body(by_body)
+        s.set_forces_lanes(4 if by_body else 0)
+        s.set_markers(m["x"], m["y"], m["z"])
+        s.stage(pfg.STAGE_CELLS)
+        want = s.cells()
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    n = want[1][-1]
+    assert n == (128 if by_body else s.n_markers)
+    if not by_body:
+        assert np.array_equal(got[2][:n], want[2][:n])
+    else:
+        assert np.array_equal(np.sort(got[2][:n]), np.sort(want[2][:n]))
