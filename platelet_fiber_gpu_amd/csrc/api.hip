@@ -797,10 +797,11 @@ pfg_status load_impl(pfg_handle *h, const pfg_model &M, const int32_t *minst,
    * membrane (or a cluster of fibrin nodes) and its stencils a small box.
    * Chunks whose box already exceeds IB_BOX_CELLS nodes at load (markers
    * far apart, as sparse fibrin nodes are) are listed for direct spreading
-   * instead.  The chunk length (16..IB_CHUNK, a power of two) aims at ~2048
-   * chunks so that a single platelet still spreads over many workgroups ---- */
+   * instead.  The chunk length (16..IB_CHUNK, a power of two) aims at
+   * IB_CHUNKS_MIN chunks, so that a single platelet still spreads over many
+   * workgroups ---- */
   int chunk_len = 16;
-  while (chunk_len < IB_CHUNK && (int64_t)chunk_len * 2 * 2048 <= n) chunk_len *= 2;
+  while (chunk_len < IB_CHUNK && (int64_t)chunk_len * 2 * IB_CHUNKS_MIN <= n) chunk_len *= 2;
   std::vector<int32_t> chunk_start, chunk_items, direct_items;
   /* body spreading: the groups that are compact platelets (elements only, at
    * most BODY_MAX_MARKERS, stencils spanning at most BODY_BOX_DIM nodes

@@ -88,10 +88,9 @@ struct MArgs {
   int lists;        /* 1: the counting launch bins the markers                   */
   int again;        /* 1: bin the positions the step started from (pos4)         */
   int spread_scratch; /* 1: the chunks of bodies write scratch boxes (form 4) */
+  int direct_span;    /* listed markers per workgroup of the spreading launch */
   const int32_t *force_list; /* force_count >= 0: the force pass takes these */
   int force_count;           /* markers only; -1: every marker                */
-  const int32_t *move_list;  /* move_count >= 0: move_kernel takes these       */
-  int move_count;            /* markers only (and leaves the step counter)    */
   int blocks0, blocks1, blocks2, blocks3; /* blocks of role ranges 0..3 */
 };
 
@@ -2288,7 +2287,7 @@ __device__ inline void stencil_origin(const MLat &L, const float v[3], const flo
  * alone, marker after marker, in the two boxes' memory taken as one.  A
  * scattered chunk (fibrin nodes far apart) adds each marker's 64 nodes with
  * device-wide atomics, as the direct form does; so do the markers listed
- * for direct spreading, IB_CHUNK per workgroup before the chunks', staged
+ * for direct spreading, direct_span per workgroup before the chunks', staged
  * the same way (each with its own lattice).  Contributions are the direct form's bit for bit; only the
  * order in which they are added differs. */
 __global__ __launch_bounds__(128) void spread_chunk_kernel(MArgs a) {
@@ -2308,17 +2307,17 @@ __global__ __launch_bounds__(128) void spread_chunk_kernel(MArgs a) {
    * run beside the chunks' summation instead of after it (spreading them
    * evenly among the chunks' workgroups measured no faster: the atomics and
    * the chunks' summation do not overlap either way) */
-  const int ndirect = (a.m.n_direct + IB_CHUNK - 1) / IB_CHUNK;
+  const int span = a.direct_span, ndirect = (a.m.n_direct + span - 1) / span;
   const bool chunk = (int)blockIdx.x >= ndirect;
   const int cid = (int)blockIdx.x - ndirect; /* the chunk */
   int c0, cnt;
   if (chunk) {
     c0 = a.m.chunk_start[cid];
     cnt = a.m.chunk_start[cid + 1] - c0;
-  } else { /* IB_CHUNK markers of the direct list (of any lattices) */
-    const int k0 = IB_CHUNK * (int)blockIdx.x;
+  } else { /* markers of the direct list (of any lattices) */
+    const int k0 = span * (int)blockIdx.x;
     c0 = a.m.chunk_start[a.m.n_chunks] + k0;
-    cnt = min(IB_CHUNK, a.m.n_direct - k0);
+    cnt = min(span, a.m.n_direct - k0);
   }
   if (cnt <= 0) return;
   const int *items = a.m.chunk_items + c0;
@@ -3365,15 +3364,11 @@ __device__ inline void finish_marker(const MArgs &a, int i, int lane, int kind, 
 /* roles: A = interpolate V at the markers, B = move the markers and advance
  * the step counter.  Four markers per wavefront, 16 lanes each. */
 __global__ __launch_bounds__(256) void move_kernel(MArgs a) {
-  const int k = (blockIdx.x * 256 + threadIdx.x) >> 4;
+  const int i = (blockIdx.x * 256 + threadIdx.x) >> 4;
   const int lane = threadIdx.x & 15;
   if (halted(a)) return;
-  /* every marker, advancing the step counter, or the markers of a list
-   * (the chunk launch of the same step advances it) */
-  if ((a.roles & ROLE_B) && a.move_count < 0 && blockIdx.x == 0 && threadIdx.x == 0)
-    *a.m.d_step += 1;
-  if (k >= (a.move_count < 0 ? a.m.n : a.move_count)) return;
-  const int i = a.move_count < 0 ? k : a.move_list[k];
+  if ((a.roles & ROLE_B) && blockIdx.x == 0 && threadIdx.x == 0) *a.m.d_step += 1;
+  if (i >= a.m.n) return;
   const int kind = a.m.kind[i];
   float v[3] = {0.f, 0.f, 0.f};
   if ((a.roles & ROLE_A) && ib_coupled(kind, a.fiber_move)) interp_marker(a, i, lane, v);
@@ -3412,7 +3407,7 @@ __device__ inline void interp_staged(const MLat &L, int4 o, const float *w, int 
 }
 
 /* Chunk-staged interpolation (ROLE_A, always) and move (ROLE_B): a
- * workgroup of MC_THREADS lanes per IB chunk, then one per IB_CHUNK markers
+ * workgroup of MC_THREADS lanes per IB chunk, then one per IB_DIRECT markers
  * listed for direct spreading (the first IB_CHUNK lanes stage the markers;
  * every lane loads the velocity box and interpolates, a marker per group of
  * 16 lanes).  Every global read of a marker (index, kind,
@@ -3449,10 +3444,10 @@ __global__ __launch_bounds__(MC_THREADS, 4) void move_chunk_kernel(MArgs a) {
   if (chunk) {
     c0 = a.m.chunk_start[blockIdx.x];
     cnt = a.m.chunk_start[blockIdx.x + 1] - c0;
-  } else { /* IB_CHUNK markers of the direct list (of any lattices) */
-    const int k0 = IB_CHUNK * ((int)blockIdx.x - a.m.n_chunks);
+  } else { /* IB_DIRECT markers of the direct list (of any lattices) */
+    const int k0 = IB_DIRECT * ((int)blockIdx.x - a.m.n_chunks);
     c0 = a.m.chunk_start[a.m.n_chunks] + k0;
-    cnt = min(IB_CHUNK, a.m.n_direct - k0);
+    cnt = min(IB_DIRECT, a.m.n_direct - k0);
   }
   if (cnt <= 0) return;
   const int *items = a.m.chunk_items + c0;
@@ -3626,6 +3621,9 @@ static void make_margs(const pfg_handle *h, MArgs *a) {
   const pfg_params &p = h->p;
   a->m = h->m;
   fill_mlat(h, 0, &a->lat);
+  a->direct_span = IB_DIRECT;
+  while (a->direct_span < IB_CHUNK && h->m.n_direct > a->direct_span * IB_DIRECT_GROUPS)
+    a->direct_span *= 2;
   a->lats = h->K > 1 ? h->d_lats : nullptr;
   a->tile0s = h->K > 1 ? h->d_tile0 : nullptr;
   a->K = h->K;
@@ -3685,8 +3683,6 @@ static void make_margs(const pfg_handle *h, MArgs *a) {
   a->by_runs = by_runs(h) ? 1 : 0;
   a->force_list = nullptr;
   a->force_count = -1;
-  a->move_list = nullptr;
-  a->move_count = -1;
   a->blocks0 = a->blocks1 = a->blocks2 = a->blocks3 = 0;
 }
 
@@ -3964,7 +3960,7 @@ hipError_t launch_spread(pfg_handle *h) {
      * marker as in form 1), then a workgroup per body adds its boxes */
     a.spread_scratch = 1;
     hipLaunchKernelGGL(spread_chunk_kernel,
-                       dim3(h->m.n_chunks + (h->m.n_direct + IB_CHUNK - 1) / IB_CHUNK),
+                       dim3(h->m.n_chunks + blocks_for(h->m.n_direct, a.direct_span)),
                        dim3(128), 0, h->stream, a);
     hipLaunchKernelGGL(spread_body_kernel, dim3(h->m.n_bodies), dim3(256), 0, h->stream, a);
     return hipGetLastError();
@@ -3972,7 +3968,7 @@ hipError_t launch_spread(pfg_handle *h) {
   /* one workgroup per IB_CHUNK markers listed for direct spreading, then
    * one per chunk, in a single launch */
   hipLaunchKernelGGL(spread_chunk_kernel,
-                     dim3(h->m.n_chunks + (h->m.n_direct + IB_CHUNK - 1) / IB_CHUNK),
+                     dim3(h->m.n_chunks + blocks_for(h->m.n_direct, a.direct_span)),
                      dim3(128), 0, h->stream, a);
   return hipGetLastError();
 }
@@ -3983,21 +3979,14 @@ hipError_t launch_move(pfg_handle *h, bool interp, bool update) {
   make_margs(h, &a);
   a.roles = (interp ? ROLE_A : 0) | (update ? ROLE_B : 0);
   if (interp && staged_spreading(h) && h->m.n_chunks > 0) {
-    /* interpolation staged by chunk, as the spreading is (this launch
-     * advances the step counter); the markers listed for direct spreading,
-     * scattered, take a group of lanes each in a launch of their own, where
-     * the many groups hide their loads' latency */
-    const dim3 grid(h->m.n_chunks);
+    /* interpolation staged by chunk, as the spreading is; the markers listed
+     * for direct spreading, scattered, follow in the same launch, one per
+     * group of 16 lanes */
+    const dim3 grid(h->m.n_chunks + blocks_for(h->m.n_direct, IB_DIRECT));
     if (h->p.sem_integrator != PFG_SEM_BBK && h->p.fiber_move != PFG_FIBER_KICK)
       hipLaunchKernelGGL(move_chunk_kernel<true>, grid, dim3(MC_THREADS), 0, h->stream, a);
     else
       hipLaunchKernelGGL(move_chunk_kernel<false>, grid, dim3(MC_THREADS), 0, h->stream, a);
-    if (h->m.n_direct > 0) {
-      a.move_list = h->m.chunk_items + h->m.n_chunk_items;
-      a.move_count = h->m.n_direct;
-      hipLaunchKernelGGL(move_kernel, dim3(blocks_for(h->m.n_direct, 16)), dim3(256), 0,
-                         h->stream, a);
-    }
     return hipGetLastError();
   }
   hipLaunchKernelGGL(move_kernel, dim3(blocks_for(h->m.n, 16)), dim3(256), 0, h->stream, a);

@@ -29,10 +29,23 @@ constexpr int SCAN_SPAN = 8192; /* bins per block of the bin-count scan */
  * axis: a scan over 64 times fewer bins for a few more candidates. */
 constexpr int COARSE_BINS = 4;
 constexpr int IB_CHUNK = 128;
+/* Chunks to have before they are made longer: two per CU.  A longer chunk
+ * adds fewer of its nodes to the lattice twice; us per step with 2048 and
+ * 512: 16625 markers 82 and 77, 31200 148 and 137, 62400 211 and 187, 25344 in
+ * 24 lattices 186 and 175 (256 chunks: within 3 us of 512). */
+constexpr int IB_CHUNKS_MIN = 512;
 /* workgroups of the tile-gather spreading launch (each takes listed tiles in
  * turn) */
 constexpr int SPREAD_TILE_GRID = 4096;
 constexpr int IB_BOX_CELLS = 1024;
+/* Markers listed for direct spreading per workgroup: their atomics follow
+ * one another in two wavefronts, so that few markers go IB_DIRECT at a time
+ * (625 scattered fibrin nodes among 1009 chunks: the launch takes 24 us, 60
+ * with IB_CHUNK, whose five workgroups were the last to end); many fill
+ * IB_DIRECT_GROUPS workgroups first, up to IB_CHUNK each (20000 nodes: 157 us
+ * with IB_CHUNK, 167 with 16, whose idle lanes and staging cost more than
+ * the shorter chain gives). */
+constexpr int IB_DIRECT = 16, IB_DIRECT_GROUPS = 128;
 /* Body spreading (spreading form 4): the chunks of a compact body (a
  * platelet of at most BODY_MAX_MARKERS markers, its stencils at most
  * BODY_BOX_DIM nodes along each axis) write their LDS sums to a scratch box

@@ -282,3 +282,38 @@ def test_cell_lists_after_steps_without_them(gpu, by_body):
         assert np.array_equal(got[2][:n], want[2][:n])
     else:
         assert np.array_equal(np.sort(got[2][:n]), np.sort(want[2][:n]))
+
+
+@pytest.mark.parametrize("kick", [False, True])
+@pytest.mark.parametrize("fibrin", [16, 17, 2049])
+def test_scattered_markers_beside_chunks(gpu, fibrin, kick):
+    """Scattered fibrin nodes share the launches of the platelets' chunks, 16 or more
+    per workgroup by their number: the force field, velocities and moves of the form
+    without chunks (sums of FP32 terms in another order)."""
+    pfg = gpu
+    sc = pfg.Scene(pfg.SCENE_LARGE, nx=128, ny=96, nz=96, n_platelets=4, elements=300,
+                   receptors=-1, ligands=-1, fibrin_nodes=fibrin, fibrin_links=8)
+    p = sc.params
+    if kick:
+        p.fiber_move = pfg.FIBER_KICK
+    f = np.random.default_rng(2).standard_normal((3, sc.n_markers)).astype(np.float32) * 1e-3
+    out = []
+    for form in (1, 2):
+        with pfg.Solver(p) as s:
+            s.load(sc)
+            s.set_ib_staging(form)
+            s.set_marker_forces(*f)
+            s.stage(pfg.STAGE_SPREAD)
+            F = s.aux()
+            s.stage(pfg.STAGE_LB)
+            s.stage(pfg.STAGE_INTERP)
+            s.stage(pfg.STAGE_UPDATE)
+            m = s.markers()
+            out.append([F] + [m[k] for k in ("vx", "vy", "vz", "x", "y", "z")])
+    scale = np.abs(out[1][0]).max()
+    assert scale > 0
+    assert np.abs(out[0][0] - out[1][0]).max() <= 2e-6 * scale
+    for a, b in zip(out[0][1:4], out[1][1:4]):
+        assert np.abs(a - b).max() <= 2e-6 * max(np.abs(b).max(), 1.0)
+    for a, b in zip(out[0][4:], out[1][4:]):
+        assert np.abs(a - b).max() <= 1e-5 * 128
