@@ -496,7 +496,7 @@ class Batch(Solver):
 
     def set_lb_persistent(self, on):
         """One persistent launch of resident workgroups taking every lattice's
-        x-block rows from a device work queue (pfg_set_lb_persistent)."""
+        blocks of cells from a device work queue (pfg_set_lb_persistent)."""
         self._c("pfg_set_lb_persistent", int(bool(on)))
 
     def init_lattice(self, k, rho=None, ux=None, uy=None, uz=None):
