@@ -358,9 +358,6 @@ __device__ __forceinline__ void lb_update(const LBArgs &a, uint32_t blk, float *
       ax = a.aux[i];
       ay = a.aux[a.plane + i];
       az = a.aux[2 * a.plane + i];
-      a.aux[i] = 0.f;
-      a.aux[a.plane + i] = 0.f;
-      a.aux[2 * a.plane + i] = 0.f;
     }
   }
   /* edge pass: upstream cell outside a wall or solid: halfway bounce-back,
@@ -383,6 +380,17 @@ __device__ __forceinline__ void lb_update(const LBArgs &a, uint32_t blk, float *
   }
   lb_cell<S, MODE>(a, dev, x, y, zlo, zhi, i, flagged, ax, ay, az, fout + own, orho, oux, ouy,
                    ouz);
+  /* zeros only where a marker added: many cells of a stamped tile hold none
+   * (all of the tile's: 5161 against 5098 us per step with 2000 platelets in
+   * 1024x512x512 FP16, 1026 against 1015 with 500 in a tube, 2100 against 2055
+   * for 256 lattices) */
+  if (M == LB_MODE_STEP || M == LB_MODE_REGION) {
+    if ((__float_as_uint(ax) | __float_as_uint(ay) | __float_as_uint(az)) != 0u) {
+      a.aux[i] = 0.f;
+      a.aux[a.plane + i] = 0.f;
+      a.aux[2 * a.plane + i] = 0.f;
+    }
+  }
 }
 
 /* Workgroups are dealt round-robin to the 8 XCDs.  With xcd_rows each XCD

@@ -317,3 +317,23 @@ def test_scattered_markers_beside_chunks(gpu, fibrin, kick):
         assert np.abs(a - b).max() <= 2e-6 * max(np.abs(b).max(), 1.0)
     for a, b in zip(out[0][4:], out[1][4:]):
         assert np.abs(a - b).max() <= 1e-5 * 128
+
+
+@pytest.mark.parametrize("store", [0, 1])
+@pytest.mark.parametrize("force", [(1e-3, 0, 0), (0, 0, -1e-30), (0, float("nan"), 0)])
+def test_force_field_is_empty_after_the_lb_update(gpu, store, force):
+    """The LB update consumes the spread force: every cell that holds one, in any one
+    component, however small, holds zero afterwards."""
+    pfg = gpu
+    sc = pfg.Scene(pfg.SCENE_SHEAR, nx=50, ny=33, nz=35, n_platelets=1, elements=200,
+                   receptors=-1, ligands=-1, fibrin_nodes=-1)
+    p = sc.params
+    p.store = store
+    f = np.repeat(np.asarray(force, np.float32)[:, None], sc.n_markers, axis=1)
+    with pfg.Solver(p) as s:
+        s.load(sc)
+        s.set_marker_forces(*f)
+        s.stage(pfg.STAGE_SPREAD)
+        assert (s.aux() != 0).any()
+        s.stage(pfg.STAGE_LB)
+        assert (s.aux() == 0).all()
