@@ -805,7 +805,7 @@ static hipError_t launch_fused(const LBArgs &a, hipStream_t st) {
   return hipGetLastError();
 }
 
-/* Which variant a step takes (LB-only launches, us, on the same box):
+/* Which variant a step takes (LB-only launches, us, on one card):
  * - Both copies within LB_CACHED_MAX_BYTES: stores through the caches, the
  *   next step then reads from the 256 MB cache in front of HBM.  Streamed /
  *   cached: 201x99x75 FP32 (226 MB) 43 / 34, 128^3 FP16 (160 MB) 30.6 / 26,
