@@ -3701,7 +3701,9 @@ hipError_t launch_begin(pfg_handle *h, bool clear, bool count, bool geometry) {
   geometry = geometry && h->m.n_tri > 0;
   a.lists = !h->in_step || step_lists(h);
   a.count_spans = count && a.lists && count_spans(h);
-  const bool boxes = count && a.by_runs;
+  /* outside a step the settings may change before the force pass: the boxes
+   * go with the lists, whichever of them that pass will read */
+  const bool boxes = count && h->m.n_runs > 0 && (a.by_runs || !h->in_step);
   a.roles = (clear ? ROLE_A : 0) | (count ? ROLE_B : 0) | (recs ? ROLE_C : 0) |
             (boxes || geometry ? ROLE_D : 0);
   a.blocks0 = clear ? blocks_for(h->ntiles, 256) : 0;

@@ -253,6 +253,32 @@ def test_morse_from_runs_of_the_platelet(gpu, sizes):
     assert sum(sizes) < 4 or np.abs(F[1]).max() > 0
 
 
+@pytest.mark.parametrize("setting, values", [("set_forces_lanes", (4, 64)),
+                                             ("set_forces_by_body", (1, 2))])
+def test_settings_between_the_cells_and_the_forces(gpu, setting, values):
+    """What CELLS leaves serves the force pass of any later setting: the forces of a
+    handle that had the setting from the start, in both directions of the change."""
+    pfg = gpu
+    ma = cloud_model((200, 300))
+    p = pfg.default_params(nx=48, ny=48, nz=48, bin_cells=2)
+    p.morse_u0, p.morse_cutoff = 1.0, 1.2
+    for first, then in (values, values[::-1]):
+        F = []
+        for before in (first, then):
+            with pfg.Solver(p) as s:
+                s.load(ma.model)
+                s.set_ib_staging(1)
+                getattr(s, setting)(before)
+                for st in (pfg.STAGE_CELLS, pfg.STAGE_MEMBRANE):
+                    s.stage(st)
+                getattr(s, setting)(then)
+                s.stage(pfg.STAGE_FORCES)
+                m = s.markers()
+                F.append(np.stack([m["fx"], m["fy"], m["fz"]]))
+        assert np.abs(F[1]).max() > 0
+        assert np.abs(F[0] - F[1]).max() <= 1e-5 * np.abs(F[1]).max()
+
+
 @pytest.mark.parametrize("by_body", [0, 1])
 def test_cell_lists_after_steps_without_them(gpu, by_body):
     """Steps that need no cell lists keep none; asked for afterwards, they are those
