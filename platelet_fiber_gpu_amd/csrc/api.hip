@@ -1317,7 +1317,8 @@ pfg_status load_impl(pfg_handle *h, const pfg_model &M, const int32_t *minst,
     PFG_TRY(upload(h, h->d_lats, lats.data(), lats.size()));
   }
   h->h_step = 0;
-  h->cells_stale = false;
+  h->lists_kept = LISTS_AS_LOADED;
+  h->boxes_kept = false;
   h->model_loaded = true;
   return PFG_OK;
 }
@@ -1633,14 +1634,25 @@ pfg_status pfg_cell_grid(const pfg_handle *h, int32_t dims[3]) {
   return PFG_OK;
 }
 
+/* The lists and boxes that the stages and pfg_download_cells read under the
+ * present settings, where the last steps or a CELLS stage under others left
+ * different ones: made again from the positions they started from. */
+static hipError_t current_lists(pfg_handle *h) {
+  const int want = bin_elements(h) ? LISTS_FULL : LISTS_COARSE;
+  if (h->lists_kept == LISTS_AS_LOADED ||
+      (h->lists_kept == want && (h->boxes_kept || h->m.n_runs == 0)))
+    return hipSuccess;
+  const hipError_t e = launch_cells_again(h);
+  h->lists_kept = e == hipSuccess ? want : LISTS_NONE;
+  h->boxes_kept = e == hipSuccess;
+  return e;
+}
+
 pfg_status pfg_download_cells(pfg_handle *h, int32_t *bin_start, int32_t *bin_items) {
   if (!h) return PFG_ERR_ARG;
   if (!h->model_loaded) return PFG_ERR_STATE;
   hipSetDevice(h->device);
-  if (h->cells_stale) { /* the step needed other lists, or none */
-    PFG_TRY(launch_cells_again(h));
-    h->cells_stale = false;
-  }
+  PFG_TRY(current_lists(h));
   const int64_t nb = bin_elements(h) ? h->m.nbins : h->m.nbinsc;
   Piece p[2] = {{bin_start, h->m.bin_start, sizeof(int32_t) * ((size_t)nb + 1)},
                 {bin_items, h->m.bin_items, sizeof(int32_t) * (size_t)h->m.n}};
@@ -1659,10 +1671,12 @@ pfg_status pfg_download_aux(pfg_handle *h, float *a3n) {
 /* ---------------- stepping ---------------- */
 
 static hipError_t run_stage(pfg_handle *h, int s) {
-  hipError_t e = hipSuccess;
+  hipError_t e = stage_reads_lists(h, s) ? current_lists(h) : hipSuccess;
+  if (e != hipSuccess) return e;
   switch (s) {
     case PFG_STAGE_CELLS:
-      h->cells_stale = false;
+      h->lists_kept = bin_elements(h) ? LISTS_FULL : LISTS_COARSE;
+      h->boxes_kept = true;
       e = launch_begin(h, false, true);
       if (e == hipSuccess) e = launch_scan(h);
       if (e == hipSuccess) e = launch_place(h, true, false);
@@ -1785,10 +1799,12 @@ static hipError_t read_report(pfg_handle *h, int64_t r[N_COUNTERS + 2]) {
   return e;
 }
 
-/* Whether pfg_download_cells has to bin again after these steps. */
+/* What these steps leave of the lists and boxes. */
 static void note_step_lists(pfg_handle *h, int nsteps) {
-  if (nsteps > 0 && h->model_loaded && h->m.n > 0 && !h->fluid_only)
-    h->cells_stale = !step_lists(h) || step_bin_elements(h) != bin_elements(h);
+  if (nsteps == 0 || !h->model_loaded || h->m.n == 0 || h->fluid_only) return;
+  h->lists_kept = !step_lists(h) ? LISTS_NONE
+                  : step_bin_elements(h) ? LISTS_FULL : LISTS_COARSE;
+  h->boxes_kept = by_runs(h);
 }
 
 pfg_status pfg_step(pfg_handle *h, int nsteps, pfg_step_info *info) {

@@ -412,9 +412,11 @@ __device__ void run_box(const MArgs &a, int r) {
   const int i = a.m.run_range[2 * r] + lane;
   float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   if (i < a.m.run_range[2 * r + 1]) {
-    lo[0] = hi[0] = a.m.x[i];
-    lo[1] = hi[1] = a.m.y[i];
-    lo[2] = hi[2] = a.m.z[i];
+    /* pos4 is being written beside this, unless it is binned again */
+    const float4 p = a.again ? a.m.pos4[i] : make_float4(a.m.x[i], a.m.y[i], a.m.z[i], 0.f);
+    lo[0] = hi[0] = p.x;
+    lo[1] = hi[1] = p.y;
+    lo[2] = hi[2] = p.z;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
@@ -3615,8 +3617,6 @@ void fill_mlat(const pfg_handle *h, int k, MLat *L) {
   L->marker0 = I.marker0;
 }
 
-static bool by_runs(const pfg_handle *h);
-
 static void make_margs(const pfg_handle *h, MArgs *a) {
   const pfg_params &p = h->p;
   a->m = h->m;
@@ -3723,10 +3723,11 @@ hipError_t launch_cells_again(pfg_handle *h) {
   make_margs(h, &a);
   a.again = 1;
   a.count_spans = count_spans(h);
-  a.roles = ROLE_B;
+  a.roles = ROLE_B | (h->m.n_runs > 0 ? ROLE_D : 0);
   a.blocks1 = blocks_for(h->m.n, 256);
+  a.blocks3 = blocks_for(h->m.n_runs, 4);
   a.mark_rows = 0;
-  hipLaunchKernelGGL(begin_kernel, dim3(a.blocks1), dim3(256), 0, h->stream, a);
+  hipLaunchKernelGGL(begin_kernel, dim3(a.blocks1 + a.blocks3), dim3(256), 0, h->stream, a);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = launch_scan(h);
   if (e == hipSuccess) e = launch_place(h, true, false);
@@ -3848,7 +3849,7 @@ static bool forces_by_body(const pfg_handle *h) {
 }
 
 /* A wavefront per marker takes its Morse candidates from its platelet's runs. */
-static bool by_runs(const pfg_handle *h) {
+bool by_runs(const pfg_handle *h) {
   return h->m.n_runs > 0 && forces_lanes(h) == 64 &&
          !(forces_by_body(h) && !forces_can_spread(h));
 }
@@ -3860,6 +3861,11 @@ bool step_bin_elements(const pfg_handle *h) {
 
 bool step_lists(const pfg_handle *h) {
   return step_bin_elements(h) || (h->m.fibrin_lig && h->m.n_rec > 0);
+}
+
+bool stage_reads_lists(const pfg_handle *h, int s) {
+  return s == PFG_STAGE_FORCES || (s == PFG_STAGE_BONDS && h->m.fibrin_lig) ||
+         (s == PFG_STAGE_SPREAD && spread_form(h) == 3);
 }
 
 /* The force launch reads the platelet sums for the area and volume forces and

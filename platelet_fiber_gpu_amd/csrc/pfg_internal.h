@@ -106,6 +106,10 @@ constexpr int64_t LB_LARGE_CELLS = (int64_t)1 << 27;
 /* Kind of a block of 64 cells: no solid cell and no solid upstream
  * neighbour, some, or solid cells only. */
 constexpr int BLOCK_FLUID = 0, BLOCK_MIXED = 1, BLOCK_SOLID = 2;
+/* Cell lists a handle holds: the empty ones of the load, none (a step that
+ * reads no list keeps none), those of the markers other than elements on the
+ * coarse grid, those of every marker. */
+enum { LISTS_AS_LOADED, LISTS_NONE, LISTS_COARSE, LISTS_FULL };
 /* Device counters of a handle (Markers::counters). */
 constexpr int N_COUNTERS = 16;
 /* Morse pairs whose distance lies within this of the cutoff are counted: a
@@ -391,8 +395,10 @@ struct pfg_handle {
   pfg::Markers m;
   bool model_loaded = false;
   bool in_step = false;        /* launches of a whole step (not of a stage)     */
-  bool cells_stale = false;    /* the last step kept other cell lists than
-                                  pfg_download_cells gives, or none             */
+  /* what the last steps or CELLS stage left of the positions in pos4: which
+   * cell lists, and whether the runs' boxes */
+  int lists_kept = pfg::LISTS_AS_LOADED;
+  bool boxes_kept = false;
   bool fluid_only = false;
   bool halt_on_detach = false; /* steps after the detach test fired change nothing */
   int ib_staging = 0;          /* spreading: 0 auto, 1 LDS-staged chunks, 2 direct */
@@ -482,7 +488,7 @@ void frames_unref();
 /* markers.hip: fused marker-side launches, each with the roles it runs */
 void fill_mlat(const pfg_handle *h, int k, MLat *L);
 hipError_t launch_begin(pfg_handle *h, bool clear, bool count, bool geometry = false);
-/* the cell lists of the positions the last step started from */
+/* the cell lists and run boxes of the positions the last step started from */
 hipError_t launch_cells_again(pfg_handle *h);
 /* the bending chain's normals and curvature, after the triangle terms */
 hipError_t launch_bend(pfg_handle *h);
@@ -502,6 +508,10 @@ bool bin_elements(const pfg_handle *h);
  * whether its platelet sums can go with the force launch */
 bool step_bin_elements(const pfg_handle *h);
 bool step_lists(const pfg_handle *h);
+/* whether stage s reads cell lists or run boxes */
+bool stage_reads_lists(const pfg_handle *h, int s);
+/* whether a step writes the runs' boxes */
+bool by_runs(const pfg_handle *h);
 bool sums_with_forces(const pfg_handle *h);
 bool forces_can_spread(const pfg_handle *h);
 hipError_t launch_spread(pfg_handle *h);

@@ -279,6 +279,48 @@ def test_settings_between_the_cells_and_the_forces(gpu, setting, values):
         assert np.abs(F[0] - F[1]).max() <= 1e-5 * np.abs(F[1]).max()
 
 
+DEFAULT, LISTS, BODY = (0, 0, 0), (4, 2, 1), (4, 1, 1)  # lanes, by body, staging
+
+
+@pytest.mark.parametrize("fibrin_ligands", [0, 1])
+@pytest.mark.parametrize("stage, stepped, then", [
+    ("FORCES", DEFAULT, LISTS), ("FORCES", LISTS, DEFAULT), ("FORCES", BODY, LISTS),
+    ("BONDS", DEFAULT, DEFAULT), ("BONDS", BODY, LISTS), ("SPREAD", DEFAULT, (0, 0, 3))])
+def test_stages_after_a_step_that_kept_other_lists(gpu, stage, stepped, then, fibrin_ligands):
+    """A step keeps the lists it needs itself; a stage called afterwards gives what it
+    gives after a step that keeps the lists of every marker (one step, so that both
+    start from the same positions): the bonds exactly, forces to their rounding."""
+    pfg = gpu
+    sc = pfg.Scene(pfg.SCENE_LARGE, nx=64, ny=48, nz=48, n_platelets=2, elements=300,
+                   receptors=64, ligands=256, fibrin_nodes=2000, fibrin_links=2000)
+    sc.fibrin_ligands = fibrin_ligands
+    m = sc.model()
+    p = sc.params
+    p.k_on, p.bond_reach, p.detach_rate = 0.5, 2.0, 0.0
+    out = []
+
+    def apply(s, lanes, by_body, staging):
+        s.set_forces_lanes(lanes)
+        s.set_forces_by_body(by_body)
+        s.set_ib_staging(staging)
+
+    for first, second in ((LISTS, LISTS if stage == "FORCES" else then), (stepped, then)):
+        with pfg.Solver(p) as s:
+            s.load(m)
+            apply(s, *first)
+            s.step(1)
+            apply(s, *second)
+            s.stage(getattr(pfg, "STAGE_" + stage))
+            mk = s.markers()
+            out.append((np.stack([mk["fx"], mk["fy"], mk["fz"]]), s.bonds()[0], s.aux()))
+    (F0, bonds0, aux0), (F1, bonds1, aux1) = out
+    assert np.array_equal(bonds0, bonds1)
+    assert stage != "BONDS" or not fibrin_ligands or (bonds0 >= m.n_wall_ligands).any()
+    assert np.abs(F0).max() > 0 and (stage != "SPREAD" or np.abs(aux0).max() > 0)
+    assert np.abs(F0 - F1).max() <= 1e-5 * np.abs(F0).max()
+    assert np.abs(aux0 - aux1).max() <= 1e-5 * np.abs(aux0).max()
+
+
 @pytest.mark.parametrize("by_body", [0, 1])
 def test_cell_lists_after_steps_without_them(gpu, by_body):
     """Steps that need no cell lists keep none; asked for afterwards, they are those
