@@ -18,13 +18,11 @@
 #include <sched.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cstring>
 #include <mutex>
-#include <system_error>
-#include <thread>
 #include <vector>
 
+#include "frame_copy.h"
 #include "pfg_internal.h"
 
 namespace pfg {
@@ -38,22 +36,19 @@ namespace {
  * one buffer; at most KEEP of a size stay allocated between calls, and none
  * once the last handle is destroyed. */
 constexpr size_t SMALL_BYTES = (size_t)1 << 20, HALF_BYTES = (size_t)8 << 20;
-constexpr size_t KEEP = 4;
+constexpr int KEEP = 4;
 
 std::mutex g_mu;
 int g_handles = 0;
-std::vector<void *> g_free[2]; /* 0: small, 1: large */
+void *g_free[2][KEEP]; /* 0: small, 1: large */
+int g_nfree[2];
 
 size_t size_of(int kind) { return kind == 0 ? SMALL_BYTES : 2 * HALF_BYTES; }
 
 void *take_buffer(int kind) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (!g_free[kind].empty()) {
-      void *p = g_free[kind].back();
-      g_free[kind].pop_back();
-      return p;
-    }
+    if (g_nfree[kind] > 0) return g_free[kind][--g_nfree[kind]];
   }
   void *p = nullptr;
   return hipHostMalloc(&p, size_of(kind), hipHostMallocPortable) == hipSuccess ? p : nullptr;
@@ -62,8 +57,8 @@ void *take_buffer(int kind) {
 void give_buffer(int kind, void *p) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if (g_handles > 0 && g_free[kind].size() < KEEP) {
-      g_free[kind].push_back(p); /* capacity reserved by frames_ref */
+    if (g_handles > 0 && g_nfree[kind] < KEEP) {
+      g_free[kind][g_nfree[kind]++] = p;
       return;
     }
   }
@@ -81,82 +76,30 @@ struct Buffer {
   Buffer &operator=(const Buffer &) = delete;
 };
 
-/* ---------------- host threads ---------------- */
-
-struct Segment { /* bytes of a half buffer and where they go */
-  char *dst;
-  const char *src;
-  size_t bytes;
-};
-
-/* Copies lists of segments with a few threads that live for one call. */
-class Copiers {
- public:
-  explicit Copiers(int n) {
-    for (int t = 1; t < n; ++t) {
-      try {
-        threads_.emplace_back([this, t] { work(t); });
-      } catch (const std::system_error &) {
-        break; /* fewer threads do it as well */
-      }
-    }
-    n_ = 1 + (int)threads_.size();
-    sized_.store(true, std::memory_order_release);
-  }
-  ~Copiers() {
-    stop_.store(true, std::memory_order_release);
-    for (std::thread &t : threads_) t.join();
-  }
-  void copy(const std::vector<Segment> &list) {
-    list_ = &list;
-    left_.store(n_ - 1, std::memory_order_relaxed);
-    epoch_.fetch_add(1, std::memory_order_release);
-    share(0);
-    while (left_.load(std::memory_order_acquire) > 0) sched_yield();
-  }
-
- private:
-  void work(int t) {
-    int seen = 0;
-    while (!sized_.load(std::memory_order_acquire)) sched_yield();
-    for (;;) {
-      while (epoch_.load(std::memory_order_acquire) == seen) {
-        if (stop_.load(std::memory_order_acquire)) return;
-        sched_yield();
-      }
-      ++seen;
-      share(t);
-      left_.fetch_sub(1, std::memory_order_release);
-    }
-  }
-  /* the t-th of n_ equal shares of the list's bytes */
-  void share(int t) const {
-    size_t total = 0;
-    for (const Segment &s : *list_) total += s.bytes;
-    size_t lo = total / n_ * t, hi = t == n_ - 1 ? total : total / n_ * (t + 1), at = 0;
-    for (const Segment &s : *list_) {
-      const size_t a = std::max(lo, at), b = std::min(hi, at + s.bytes);
-      if (a < b) std::memcpy(s.dst + (a - at), s.src + (a - at), b - a);
-      at += s.bytes;
-    }
-  }
-  std::vector<std::thread> threads_;
-  const std::vector<Segment> *list_ = nullptr;
-  int n_ = 1;
-  std::atomic<int> epoch_{0}, left_{0};
-  std::atomic<bool> stop_{false}, sized_{false};
-};
-
-/* One thread per 2 MiB, at most 8 and half of the CPUs the process may use. */
+/* One thread per 2 MiB, at most COPIERS_MAX and half of the CPUs the process may use. */
 int copier_count(size_t bytes) {
   cpu_set_t set;
   int cpus = 2;
   if (sched_getaffinity(0, sizeof(set), &set) == 0) cpus = CPU_COUNT(&set);
-  const size_t n = std::min<size_t>({bytes / ((size_t)2 << 20), 8, (size_t)cpus / 2});
+  const size_t n = std::min<size_t>({bytes / ((size_t)2 << 20), COPIERS_MAX, (size_t)cpus / 2});
   return (int)std::max<size_t>(n, 1);
 }
 
 /* ---------------- the pipeline ---------------- */
+
+struct Events {
+  hipEvent_t e[2] = {nullptr, nullptr};
+  hipError_t create() {
+    hipError_t r = hipSuccess;
+    for (int k = 0; k < 2 && r == hipSuccess; ++k)
+      r = hipEventCreateWithFlags(&e[k], hipEventDisableTiming);
+    return r;
+  }
+  ~Events() {
+    for (hipEvent_t x : e)
+      if (x) hipEventDestroy(x);
+  }
+};
 
 /* Writes batches 0 .. nb-1 into the buffer's halves in turn (fill(b, device
  * pointer) enqueues the kernel) and copies each out (list(b, host pointer,
@@ -169,44 +112,34 @@ hipError_t run_batches(pfg_handle *h, size_t total, int nb, Fill fill, List list
   void *dev = nullptr;
   hipError_t e = hipHostGetDevicePointer(&dev, buf.host, 0);
   if (e != hipSuccess) return e;
-  std::vector<Segment> segs;
   if (nb == 1) {
     e = fill(0, (char *)dev);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    const hipError_t e2 = hipStreamSynchronize(h->stream);
+    if (e == hipSuccess) e = e2;
     if (e != hipSuccess) return e;
+    SegmentList segs;
     list(0, (const char *)buf.host, segs);
     Copiers(copier_count(total)).copy(segs);
     return hipSuccess;
   }
-  hipEvent_t ev[2] = {nullptr, nullptr};
-  for (int k = 0; k < 2 && e == hipSuccess; ++k)
-    e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
-  {
-    Copiers copiers(copier_count(total));
-    auto start = [&](int b) {
-      hipError_t r = fill(b, (char *)dev + (size_t)(b & 1) * HALF_BYTES);
-      return r == hipSuccess ? hipEventRecord(ev[b & 1], h->stream) : r;
-    };
-    if (e == hipSuccess) e = start(0);
-    for (int b = 0; b < nb && e == hipSuccess; ++b) {
-      if (b + 1 < nb) e = start(b + 1);
-      if (e == hipSuccess) e = hipEventSynchronize(ev[b & 1]);
-      if (e != hipSuccess) break;
-      segs.clear();
-      list(b, (const char *)buf.host + (size_t)(b & 1) * HALF_BYTES, segs);
-      copiers.copy(segs);
-    }
-  }
-  /* no kernel writes the buffer once it is given back */
-  const hipError_t e2 = hipStreamSynchronize(h->stream);
-  for (hipEvent_t x : ev)
-    if (x) hipEventDestroy(x);
-  return e == hipSuccess ? e2 : e;
+  Events ev;
+  e = ev.create();
+  if (e != hipSuccess) return e;
+  Copiers copiers(copier_count(total));
+  return copy_halves<hipError_t>(
+      nb, copiers,
+      [&](int b) {
+        const hipError_t r = fill(b, (char *)dev + (size_t)(b & 1) * HALF_BYTES);
+        return r == hipSuccess ? hipEventRecord(ev.e[b & 1], h->stream) : r;
+      },
+      [&](int b) { return hipEventSynchronize(ev.e[b & 1]); },
+      [&](int b, SegmentList &out) {
+        list(b, (const char *)buf.host + (size_t)(b & 1) * HALF_BYTES, out);
+      },
+      [&] { return hipStreamSynchronize(h->stream); });
 }
 
 /* ---------------- kernels ---------------- */
-
-constexpr int PACK_MAX = 12; /* arrays per launch */
 
 struct PackArgs {
   const uint32_t *src[PACK_MAX];
@@ -235,20 +168,18 @@ __global__ void report_kernel(const int64_t *counters, const int64_t *detach_ste
 void frames_ref() {
   std::lock_guard<std::mutex> lk(g_mu);
   ++g_handles;
-  for (auto &f : g_free) f.reserve(KEEP);
 }
 
 void frames_unref() {
-  std::vector<void *> drop;
+  void *drop[2 * KEEP];
+  int n = 0;
   {
     std::lock_guard<std::mutex> lk(g_mu);
     if (--g_handles > 0) return;
-    for (auto &f : g_free) {
-      drop.insert(drop.end(), f.begin(), f.end());
-      f.clear();
-    }
+    for (int kind = 0; kind < 2; ++kind)
+      while (g_nfree[kind] > 0) drop[n++] = g_free[kind][--g_nfree[kind]];
   }
-  for (void *p : drop) hipHostFree(p);
+  for (int k = 0; k < n; ++k) hipHostFree(drop[k]);
 }
 
 hipError_t fetch_pieces(pfg_handle *h, const Piece *pieces, int n) {
@@ -262,7 +193,7 @@ hipError_t fetch_pieces(pfg_handle *h, const Piece *pieces, int n) {
   for (int k = 0; k < n; ++k) {
     if (pieces[k].bytes % 4 != 0) return hipErrorInvalidValue;
     for (size_t off = 0; off < pieces[k].bytes;) {
-      if (room == 0 || batches.back().size() == PACK_MAX) {
+      if (room == 0 || batches.back().size() == (size_t)PACK_MAX) {
         batches.emplace_back();
         room = HALF_BYTES;
       }
@@ -289,9 +220,9 @@ hipError_t fetch_pieces(pfg_handle *h, const Piece *pieces, int n) {
     hipLaunchKernelGGL(pack_kernel, dim3(gx, (unsigned)parts.size()), dim3(256), 0, h->stream, a);
     return hipGetLastError();
   };
-  auto list = [&](int b, const char *host, std::vector<Segment> &out) {
+  auto list = [&](int b, const char *host, SegmentList &out) {
     for (const Part &q : batches[(size_t)b]) {
-      out.push_back({(char *)pieces[q.piece].dst + q.off, host, q.bytes});
+      out.add((char *)pieces[q.piece].dst + q.off, host, q.bytes);
       host += q.bytes;
     }
   };
@@ -316,12 +247,12 @@ hipError_t fetch_fields(pfg_handle *h, int k, float *const host[4]) {
     }
     return launch_lb_fields_window(h, k, (uint32_t)lo, (uint32_t)hi, win);
   };
-  auto list = [&](int b, const char *src, std::vector<Segment> &out) {
+  auto list = [&](int b, const char *src, SegmentList &out) {
     const int64_t lo = room * b, hi = std::min(n, lo + room);
     const size_t bytes = sizeof(float) * (size_t)(hi - lo);
     for (int c = 0; c < 4; ++c) {
       if (!host[c]) continue;
-      out.push_back({(char *)(host[c] + lo), src, bytes});
+      out.add((char *)(host[c] + lo), src, bytes);
       src += bytes;
     }
   };
