@@ -795,12 +795,15 @@ pfg_status load_impl(pfg_handle *h, const pfg_model &M, const int32_t *minst,
    * starting positions (along the longest extent, at a multiple of the
    * chunk length) into compact chunks, so that a chunk covers a patch of a
    * membrane (or a cluster of fibrin nodes) and its stencils a small box.
-   * Chunks whose box already exceeds IB_BOX_CELLS nodes at load (markers
-   * far apart, as sparse fibrin nodes are) are listed for direct spreading
-   * instead.  The chunk length (16..IB_CHUNK, a power of two) aims at
-   * IB_CHUNKS_MIN chunks, so that a single platelet still spreads over many
-   * workgroups ---- */
-  int chunk_len = 16;
+   * A leaf whose box exceeds IB_BOX_CELLS nodes at load is cut in halves, to
+   * IB_CHUNK_MIN markers; one that still does (markers far apart, as sparse
+   * fibrin nodes are) is listed for direct spreading instead.  us per step of
+   * a clot of fibrin nodes two cells apart, whole leaves listed / halved:
+   * 20 000 nodes 154 / 107, 40 000 219 / 128, 80 000 323 / 166, 150 000
+   * 586 / 255; three to five cells apart the same to 2 %.  The chunk length
+   * (IB_CHUNK_MIN..IB_CHUNK, a power of two) aims at IB_CHUNKS_MIN chunks, so
+   * that a single platelet still spreads over many workgroups ---- */
+  int chunk_len = IB_CHUNK_MIN;
   while (chunk_len < IB_CHUNK && (int64_t)chunk_len * 2 * IB_CHUNKS_MIN <= n) chunk_len *= 2;
   std::vector<int32_t> chunk_start, chunk_items, direct_items;
   /* body spreading: the groups that are compact platelets (elements only, at
@@ -858,9 +861,10 @@ pfg_status load_impl(pfg_handle *h, const pfg_model &M, const int32_t *minst,
         int32_t *b = todo.back().first;
         const int cnt = todo.back().second;
         todo.pop_back();
-        /* a body's leaf is cut in halves until its box fits */
-        const bool split = cnt > chunk_len ||
-                           (body && cnt > 1 && box_volume(b, cnt) > IB_BOX_CELLS);
+        /* a leaf is cut in halves until its box fits, a body's to the last
+         * marker */
+        const bool split = cnt > chunk_len || (cnt > (body ? 1 : IB_CHUNK_MIN) &&
+                                               box_volume(b, cnt) > IB_BOX_CELLS);
         if (!split) {
           leaf(b, cnt);
           continue;

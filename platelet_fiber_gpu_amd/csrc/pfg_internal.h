@@ -28,7 +28,7 @@ constexpr int SCAN_SPAN = 8192; /* bins per block of the bin-count scan */
  * reads them), their bins are COARSE_BINS bins of the full grid along each
  * axis: a scan over 64 times fewer bins for a few more candidates. */
 constexpr int COARSE_BINS = 4;
-constexpr int IB_CHUNK = 128;
+constexpr int IB_CHUNK_MIN = 16, IB_CHUNK = 128; /* markers of a chunk */
 /* Chunks to have before they are made longer: two per CU.  A longer chunk
  * adds fewer of its nodes to the lattice twice; us per step with 2048 and
  * 512: 16625 markers 82 and 77, 31200 148 and 137, 62400 211 and 187, 25344 in

@@ -387,6 +387,42 @@ def test_scattered_markers_beside_chunks(gpu, fibrin, kick):
         assert np.abs(a - b).max() <= 1e-5 * 128
 
 
+@pytest.mark.parametrize("n, spacing", [(15, 2), (16, 2), (17, 2), (33, 3), (5000, 3),
+                                        (33000, 2), (66000, 1.5)])
+def test_clots_are_cut_until_their_chunks_fit(gpu, n, spacing):
+    """Fibrin nodes close together beside as many far apart: chunks halved until their
+    boxes fit, part of them listed.  The force field and the velocities of the direct
+    form; a node's some 30 terms of at most 0.3 of a force in all, summed in another
+    order on both sides, differ by less than 1e-6 of the largest force."""
+    pfg = gpu
+    rng = np.random.default_rng(n)
+    side = int(np.ceil(n ** (1 / 3)))
+    nx = int(side * spacing) + 24
+    g = np.stack(np.meshgrid(*[np.arange(side)] * 3, indexing="ij"), -1).reshape(-1, 3)[:n]
+    P = np.concatenate([g * spacing + 8 + rng.uniform(-0.3, 0.3, g.shape),
+                        rng.random((n, 3)) * nx])
+    p = pfg.default_params(nx=nx, ny=nx, nz=nx)
+    p.wall[1] = pfg.WALL_BOUNCE
+    ma = ModelArrays(*P.T, kind=np.full(2 * n, pfg.MARKER_FIBER), body=np.full(2 * n, -1))
+    f = rng.standard_normal((3, 2 * n)).astype(np.float32) * 1e-3
+    out = []
+    for form in (1, 2):
+        with pfg.Solver(p) as s:
+            s.load(ma.model)
+            s.set_ib_staging(form)
+            s.set_marker_forces(*f)
+            s.stage(pfg.STAGE_SPREAD)
+            F = s.aux()
+            s.stage(pfg.STAGE_LB)
+            s.stage(pfg.STAGE_INTERP)
+            m = s.markers()
+            out.append((F, np.stack([m["vx"], m["vy"], m["vz"]])))
+    fmax = np.abs(f).max() * abs(p.ib_force_scale)
+    assert np.abs(out[1][0]).max() > 0.1 * fmax
+    assert np.abs(out[0][0] - out[1][0]).max() <= 1e-6 * fmax
+    assert np.abs(out[0][1] - out[1][1]).max() <= 2e-6
+
+
 @pytest.mark.parametrize("store", [0, 1])
 @pytest.mark.parametrize("force", [(1e-3, 0, 0), (0, 0, -1e-30), (0, float("nan"), 0)])
 def test_force_field_is_empty_after_the_lb_update(gpu, store, force):
