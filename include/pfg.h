@@ -396,9 +396,10 @@ pfg_status pfg_set_fluid_only(pfg_handle *h, int fluid_only);
 pfg_status pfg_set_halt_on_detach(pfg_handle *h, int enable);
 /* IB spreading form (LB_kernel.cu:1419-1520 restated four ways): 0 automatic
  * (4 from 2^20 markers up when the model has compact platelets; else 1 from
- * 2560 markers up, or from 1280 where the force pass cannot spread itself; 2
- * below), 1 always staged (a workgroup per run
- * of up to 128 markers of one platelet accumulates them in LDS first),
+ * 2560 markers in chunks up, or from 1280 where the force pass cannot spread
+ * itself; 2 below), 1 always staged (a workgroup per chunk of up to 128
+ * markers of one platelet, or of fibrin nodes close together, accumulates
+ * them in LDS first; markers far apart are in no chunk),
  * 2 always direct (FP32 atomics per marker and node), 3 tile gather (a
  * wavefront per 4x4x4 tile that this step's stencils meet sums the
  * contributions of the markers on the cell lists near it in LDS and writes

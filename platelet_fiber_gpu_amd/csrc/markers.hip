@@ -3833,7 +3833,8 @@ static int spread_form(const pfg_handle *h) {
    * tile alone, so that runs in 16-bit storage repeat closely, for 0.7 % of a
    * step: 2000 platelets in 1024x512x512 5201 against 5165 us. */
   if (h->m.n >= SPREAD_BODY_MIN && h->m.n_bodies > 0) return 4;
-  return h->m.n >= (spread_rides_along(h) ? IB_STAGED_MIN : IB_STAGED_MIN_ALONE) ? 1 : 2;
+  return h->m.n_chunk_items >= (spread_rides_along(h) ? IB_STAGED_MIN : IB_STAGED_MIN_ALONE) ? 1
+                                                                                              : 2;
 }
 
 static bool staged_spreading(const pfg_handle *h) { return spread_form(h) != 2; }

@@ -72,11 +72,15 @@ constexpr float FB_SKIN = 0.25f;
 constexpr int MORSE_RUN = 64, MORSE_RUNS_MAX = 64;
 /* lanes of the per-body workgroups (force pass, second spreading pass) */
 constexpr int BODY_THREADS = 1024;
-/* Marker counts from which spreading is staged through LDS by default: when
+/* Markers in chunks from which spreading is staged through LDS by default: when
  * the force launch could spread as well, and when spreading is a launch of its
  * own anyway.  us per step, direct / staged, on 160x96x96 FP32: fused 1536
  * markers 60.5 / 62.8, 2048 62.0 / 64.4, 3000 66.9 / 62.6, 6000 77 / 66; own
- * launch 1024 62.0 / 62.7, 1536 65.2 / 63.6, 2048 67.7 / 65.3. */
+ * launch 1024 62.0 / 62.7, 1536 65.2 / 63.6, 2048 67.7 / 65.3.  Scattered
+ * markers do not count: nothing of them is staged, and they take a wavefront
+ * each in the direct form (fibrin nodes alone, 160^3 FP16: 3000 118 / 134,
+ * 10 000 162 / 211, 30 000 265 / 302, 60 000 257 / 291; 30 000 beside 2000
+ * elements 180 / 212; 100 000 in 256^3 605 / 616, 600 000 in 448^3 3591 / 3529). */
 constexpr int IB_STAGED_MIN = 2560, IB_STAGED_MIN_ALONE = 1280;
 /* ... and from which it goes by body when the model has compact platelets. */
 constexpr int SPREAD_BODY_MIN = 1 << 20;

@@ -423,6 +423,38 @@ def test_clots_are_cut_until_their_chunks_fit(gpu, n, spacing):
     assert np.abs(out[0][1] - out[1][1]).max() <= 2e-6
 
 
+@pytest.mark.parametrize("elements", [0, 2559, 2560])
+@pytest.mark.parametrize("halt", [False, True])
+def test_spreading_of_scattered_models(gpu, elements, halt):
+    """The automatic form follows the markers in chunks, not the scattered ones beside
+    them: one step of either form from the same state (velocities of order 1e-2 from
+    sums in another order, forces through them at most the same)."""
+    pfg = gpu
+    rng = np.random.default_rng(elements)
+    n, nx = 6000, 160
+    E = rng.random((elements, 3)) * 0.9 * max(elements, 1) ** (1 / 3) + 70
+    P = np.concatenate([E, rng.random((n, 3)) * nx])
+    kind = np.repeat([pfg.MARKER_ELEMENT, pfg.MARKER_FIBER], [elements, n])
+    kw = dict(plt_elem_start=[0, elements], plt_tri_start=[0, 0], tri_S0=[], plt_S0=[1.0],
+              plt_V0=[1.0]) if elements else {}
+    ma = ModelArrays(*P.T, kind=kind, body=np.where(kind == pfg.MARKER_ELEMENT, 0, -1), **kw)
+    p = pfg.default_params(nx=nx, ny=nx, nz=nx)
+    p.morse_u0, p.morse_cutoff = 1e-4, 1.2
+    p.body_force[0] = 1e-5
+    out = []
+    for form in (0, 1, 2):
+        with pfg.Solver(p) as s:
+            s.load(ma.model)
+            s.set_ib_staging(form)
+            s.set_halt_on_detach(halt)
+            s.step(1)
+            m = s.markers()
+            out.append(np.stack([m[k] for k in ("vx", "vy", "vz", "x", "y", "z")]))
+    for a in out[:2]:
+        assert np.abs(a[:3] - out[2][:3]).max() <= 1e-6
+        assert np.abs(a[3:] - out[2][3:]).max() <= 1e-6 * nx
+
+
 @pytest.mark.parametrize("store", [0, 1])
 @pytest.mark.parametrize("force", [(1e-3, 0, 0), (0, 0, -1e-30), (0, float("nan"), 0)])
 def test_force_field_is_empty_after_the_lb_update(gpu, store, force):
