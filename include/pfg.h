@@ -417,7 +417,8 @@ pfg_status pfg_set_halt_on_detach(pfg_handle *h, int enable);
 pfg_status pfg_set_ib_staging(pfg_handle *h, int mode);
 /* Lanes per marker in the SEM/fibrin force pass (sem_Force_kernel,
  * sem_kernel.cu:320-513, with the Morse pairs over the cell lists): 0
- * automatic (64 below 65536 markers, else 4), or 1, 2, 4, 8, 16, 32 or 64.  With
+ * automatic (64 below 65536 markers, in a model without platelets below 32768,
+ * else 4), or 1, 2, 4, 8, 16, 32 or 64.  With
  * fewer than 64 the markers are taken in cell-list order.  Same result up
  * to FP32 summation order. */
 pfg_status pfg_set_forces_lanes(pfg_handle *h, int lanes);

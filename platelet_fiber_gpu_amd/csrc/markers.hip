@@ -3804,10 +3804,15 @@ hipError_t launch_resolve(pfg_handle *h) {
   return hipGetLastError();
 }
 
+/* markers from which a model's force pass takes 4 lanes each */
+static int forces_sorted_min(const pfg_handle *h) {
+  return h->m.n_plt > 0 ? FORCES_SORTED_MIN : FORCES_SORTED_MIN_FIBRIN;
+}
+
 static int forces_lanes(const pfg_handle *h) {
   /* few markers: a wavefront each, for parallelism; many: 4 lanes each in
    * bin order, for fewer instructions per marker */
-  return h->forces_lanes ? h->forces_lanes : (h->m.n >= FORCES_SORTED_MIN ? 4 : 64);
+  return h->forces_lanes ? h->forces_lanes : (h->m.n >= forces_sorted_min(h) ? 4 : 64);
 }
 
 static bool contact_on(const pfg_handle *h) {

@@ -87,8 +87,12 @@ constexpr int SPREAD_BODY_MIN = 1 << 20;
 /* Marker count from which the forces take 4 lanes per marker in bin order, or
  * the pass by body where it applies (below it, a wavefront per marker).  us
  * per step, wavefront / by body: 31 200 markers 187 / 224, 46 800 246 / 259,
- * 83 200 442 / 441, 156 000 497 / 477. */
-constexpr int FORCES_SORTED_MIN = 65536;
+ * 83 200 442 / 441, 156 000 497 / 477.  Platelets of 5000 elements, too long
+ * for the runs, wavefront / 4 lanes: 40 000 markers 157 / 195, 60 000 216 / 233.
+ * Without platelets a marker has a few links and no Morse partners for its
+ * lanes: clots of 34 000 fibrin nodes 122 / 113, 50 000 146 / 133, 64 000
+ * 173 / 157 (below, few wavefronts are left: the same to 5 %). */
+constexpr int FORCES_SORTED_MIN = 65536, FORCES_SORTED_MIN_FIBRIN = 32768;
 /* Marker count from which the force pass by body is taken without being asked
  * for (where the library does not take a wavefront per marker), and
  * pfg_download_cells leaves the elements of such models out. */

@@ -423,6 +423,35 @@ def test_clots_are_cut_until_their_chunks_fit(gpu, n, spacing):
     assert np.abs(out[0][1] - out[1][1]).max() <= 2e-6
 
 
+def forces_after_a_step(pfg, p, ma, lanes):
+    with pfg.Solver(p) as s:
+        s.load(ma.model)
+        s.set_forces_lanes(lanes)
+        s.step(1)
+        m = s.markers()
+        return np.stack([m["fx"], m["fy"], m["fz"]])
+
+
+@pytest.mark.parametrize("n, lanes", [(32767, 64), (32768, 4)])
+def test_automatic_lanes_of_a_fibrin_network(gpu, n, lanes):
+    """A model without platelets takes 4 lanes per node from 32768 nodes: bit for bit
+    the forces of the lanes set by hand (eight links a node, summed in another order
+    by other lanes)."""
+    pfg = gpu
+    rng = np.random.default_rng(n)
+    P = (rng.random((3, n)) * 96).astype(np.float32)
+    a = np.arange(n)
+    link = np.stack([np.repeat(a, 4), (np.repeat(a, 4) + np.tile([1, 7, 57, 401], n)) % n], 1)
+    d = np.linalg.norm(P[:, link[:, 0]] - P[:, link[:, 1]], axis=0)
+    ma = ModelArrays(*P, kind=np.full(n, pfg.MARKER_FIBER), body=np.full(n, -1),
+                     link=link.ravel(), link_l0=0.9 * d)
+    p = pfg.default_params(nx=96, ny=96, nz=96)
+    p.fiber_k = 1e-3
+    F = {k: forces_after_a_step(pfg, p, ma, k) for k in (0, 4, 64)}
+    assert not np.array_equal(F[4], F[64])
+    assert np.array_equal(F[0], F[lanes])
+
+
 @pytest.mark.parametrize("elements", [0, 2559, 2560])
 @pytest.mark.parametrize("halt", [False, True])
 def test_spreading_of_scattered_models(gpu, elements, halt):
