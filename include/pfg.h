@@ -424,8 +424,8 @@ pfg_status pfg_set_ib_staging(pfg_handle *h, int mode);
 pfg_status pfg_set_forces_lanes(pfg_handle *h, int lanes);
 /* Force pass by body (sem_Force_kernel's Morse term, sem_kernel.cu:320-513,
  * acts between the elements of one platelet): 0 automatic (on from 65536
- * markers, and from 32768 where fewer than 64 lanes per marker are set), 1
- * on, 2 off.  On: a workgroup per platelet of at most 2048
+ * markers, and from 32768 where fewer than 64 lanes per marker are set or a
+ * platelet has more than 4096 elements), 1 on, 2 off.  On: a workgroup per platelet of at most 2048
  * elements sorts its positions into a cell list of its own in LDS and sums
  * each element's Morse pairs there, then its other terms; the other
  * markers take the per-marker pass (pfg_set_forces_lanes).  It applies

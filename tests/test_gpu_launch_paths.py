@@ -452,6 +452,18 @@ def test_automatic_lanes_of_a_fibrin_network(gpu, n, lanes):
     assert np.array_equal(F[0], F[lanes])
 
 
+def test_a_wavefront_by_choice_is_the_automatic_one(gpu):
+    """64 lanes set by hand take the pass that the library takes by itself between 32768
+    and 65535 markers: the same forces bit for bit (other passes sum in another order)."""
+    pfg = gpu
+    ma = cloud_model((1000,) * 33, nx=96)
+    p = pfg.default_params(nx=96, ny=96, nz=96, bin_cells=2)
+    p.morse_u0, p.morse_cutoff = 1e-4, 1.2
+    F = {k: forces_after_a_step(pfg, p, ma, k) for k in (0, 4, 64)}
+    assert not np.array_equal(F[4], F[64])
+    assert np.array_equal(F[0], F[64])
+
+
 @pytest.mark.parametrize("elements", [0, 2559, 2560])
 @pytest.mark.parametrize("halt", [False, True])
 def test_spreading_of_scattered_models(gpu, elements, halt):
