@@ -1,5 +1,7 @@
 """Launch paths chosen by sizes, compared with the oracle or with the general path
 at the sizes where they can go wrong."""
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -82,6 +84,7 @@ def test_blocks_across_rows_and_planes(gpu, po, size, walls):
     assert np.abs(fg - fo)[:, fluid].max(initial=0.0) < 2e-7
     for got, want in zip(fields, po.fields(L, fo)):
         assert np.abs(got - want)[fluid].max(initial=0.0) < 1e-6
+        assert (got[~fluid] == 0).all()
 
 
 @pytest.mark.parametrize("nx", [60, 101])
@@ -138,7 +141,6 @@ def test_frames_of_any_size(gpu, n):
 def test_frames_from_several_threads(gpu):
     """Handles in threads of their own download at once (buffers are shared by the
     process, a call holds one): the same values as one after the other."""
-    import threading
     pfg = gpu
     solvers = []
     for k in range(4):
@@ -149,22 +151,51 @@ def test_frames_from_several_threads(gpu):
         s.step(3 + k)
         solvers.append(s)
     want = [s.fields() for s in solvers]
-    bad = []
 
     def work(k):
-        for _ in range(5):
-            got = solvers[k].fields()
-            if not all(np.array_equal(a, b) for a, b in zip(got, want[k])):
-                bad.append(k)
+        return [all(np.array_equal(a, b) for a, b in zip(solvers[k].fields(), want[k]))
+                for _ in range(5)]
 
-    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
-    for t in threads:
-        t.start()
-    for t in threads:
-        t.join()
+    with ThreadPoolExecutor(4) as pool:  # a failed download raises from map
+        same = list(pool.map(work, range(4)))
     for s in solvers:
         s.close()
-    assert not bad
+    assert np.all(same)
+
+
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("size", [(64, 6, 5), (33, 7, 5), (130, 65, 3)])
+def test_fields_of_solid_cells_are_zero(gpu, size, noalloc):
+    """Solid cells read 0, in blocks of 64 solid cells, in mixed ones and in a last block
+    partly empty, where the buffers still hold the frame of a larger lattice."""
+    import ctypes as C
+    pfg = gpu
+    nx, ny, nz = size
+    N = nx * ny * nz
+
+    def fields(s):
+        if not noalloc:
+            return s.fields()
+        out = [np.full(s.N, 7.0, np.float32) for _ in range(4)]
+        assert pfg.lib().pfg_download_fields_noalloc(
+            C.c_void_p(s._h.value), *[a.ctypes.data_as(C.POINTER(C.c_float)) for a in out]) == 0
+        return out
+
+    flags = (np.random.default_rng(N).random(N) < 0.1).astype(np.uint8)
+    flags[64:64 * 7] = 1
+    flags[N - N % 64 - 64:] = 1
+    p = pfg.default_params(nx=nx, ny=ny, nz=nz, use_flags=1)
+    big = pfg.default_params(nx=96, ny=64, nz=64)
+    for q in (p, big):
+        q.body_force[0] = q.body_force[1] = q.body_force[2] = 1e-5
+    with pfg.Solver(big) as b, pfg.Solver(p) as s:
+        b.step(2)
+        s.upload_flags(flags)
+        s.step(2)
+        assert all((a != 0).all() for a in fields(b))
+        for a in fields(s):
+            assert (a[flags != 0] == 0).all()
+            assert (a[flags == 0] != 0).any()
 
 
 def test_noalloc_fields_with_velocity_faces(gpu):
