@@ -3832,11 +3832,15 @@ static int spread_form(const pfg_handle *h) {
   if (h->ib_staging == 3 && !h->m.tile_gather_ok) return 1;
   if (h->ib_staging == 4 && h->m.n_bodies == 0) return 1;
   if (h->ib_staging) return h->ib_staging;
-  /* staged rather than by body: 500 platelets in the tube 1056 against 1080 us
-   * per step, a batch of 256 lattices 2076 against 2112.  From SPREAD_BODY_MIN
-   * markers by body, whose sums have a fixed order where a platelet meets a
-   * tile alone, so that runs in 16-bit storage repeat closely, for 0.7 % of a
-   * step: 2000 platelets in 1024x512x512 5201 against 5165 us. */
+  /* staged / by body, us per step of suspensions of platelets of 1000 elements
+   * and 4 % fibrin nodes: FP32 41 600 markers 246 / 300, 104 000 389 / 439,
+   * 260 000 917 / 972, 728 000 3627 / 3662, 988 000 4711 / 4717, 1 144 000
+   * 5502 / 5221, 1 560 000 6404 / 6080; FP16 41 600 160 / 209, 260 000
+   * 582 / 629, 988 000 2575 / 2629, 1 144 000 2963 / 3132, 1 560 000
+   * 3600 / 3669.  The line is FP32's; FP16 keeps it, 2-5 % slower above, for
+   * the order of its sums, fixed where a platelet meets a tile alone: 8 steps
+   * of these suspensions repeated bit for bit by body (but for the fibrin
+   * nodes' atomics) and to 1e-7 of the velocities staged. */
   if (h->m.n >= SPREAD_BODY_MIN && h->m.n_bodies > 0) return 4;
   return h->m.n_chunk_items >= (spread_rides_along(h) ? IB_STAGED_MIN : IB_STAGED_MIN_ALONE) ? 1
                                                                                               : 2;
