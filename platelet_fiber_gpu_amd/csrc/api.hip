@@ -1990,6 +1990,7 @@ pfg_status pfg_profile(pfg_handle *h, int nsteps, double *ms_total, double *ms_l
 pfg_status pfg_set_lb_tuning(pfg_handle *h, int cells_per_lane) {
   if (!h) return PFG_ERR_ARG;
   if (cells_per_lane != 1 && cells_per_lane != 2 && cells_per_lane != 4) return PFG_ERR_ARG;
+  if (cells_per_lane == h->lb_cpt) return PFG_OK;
   h->lb_cpt = cells_per_lane;
   drop_graph(h);
   return PFG_OK;
