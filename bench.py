@@ -489,7 +489,7 @@ def batch_workload(pfg, K, W, store, cpu_leg=True):
     persistent = int((TUNING.get("batch") or {}).get("lb_persistent", 0))
     b.set_fluid_only(True)
     lb_ms_by = {}
-    for form in (0, 1):  # one workgroup per x-block row; the persistent queue launch
+    for form in (0, 1):  # one workgroup per four blocks; the persistent queue launch
         b.set_lb_persistent(form)
         b.step(8)
         lb_ms_by[form] = b.time_lb(max(10, min(K, 60)))

@@ -433,9 +433,9 @@ pfg_status pfg_set_forces_lanes(pfg_handle *h, int lanes);
  * per-marker pass takes every marker.  Same forces up to FP32 summation
  * order. */
 pfg_status pfg_set_forces_by_body(pfg_handle *h, int mode);
-/* enable = 1: within a step, the LB update of the lattice rows that no IB
+/* enable = 1: within a step, the LB update of the lattice blocks that no IB
  * stencil touches runs on a second HIP stream concurrently with the marker
- * pipeline, and the touched rows update after the spreading (semLB.cu:303-438
+ * pipeline, and the touched blocks update after the spreading (semLB.cu:303-438
  * runs these phases one after the other); 0 (default): one LB launch after
  * the spreading.  Same result either way; on MI355X the concurrent LB launch
  * slows the latency-bound marker kernels as much as it hides them. */

@@ -388,7 +388,7 @@ pfg_status create_impl(const pfg_params *ps, int K, int device, pfg_handle **out
   h->K = K;
   h->esize = p.store == PFG_STORE_F32 ? 4 : 2;
   bool flags = false;
-  /* lattice k occupies cells [cell0, cell0 + N), x-blocks [fblk0, ...),
+  /* lattice k occupies cells [cell0, cell0 + N), blocks [fblk0, ...),
    * tiles [tile0, ...) and LB workgroups [lb_block0, ...) */
   h->inst.resize((size_t)K);
   int64_t cell = 0, fblk = 0, tile = 0;
@@ -459,7 +459,7 @@ pfg_status create_impl(const pfg_params *ps, int K, int device, pfg_handle **out
     for (const Inst &I : h->inst) nmax = std::max(nmax, I.N);
     h->red_blocks = std::min<int64_t>(2048, (nmax + 255) / 256);
     if (dalloc(h, &h->red, (size_t)4 * h->red_blocks) != hipSuccess) { st = PFG_ERR_ALLOC; break; }
-    /* z-cells per lane of the LB kernel */
+    /* cells (blocks in a row) per lane of the LB kernel */
     h->lb_cpt = 1;
     h->lb_xcd_rows = lb_default_xcd_rows(h);
     if (dalloc(h, &h->m.counters, N_COUNTERS) != hipSuccess) { st = PFG_ERR_ALLOC; break; }
@@ -1707,14 +1707,16 @@ static hipError_t run_stage(pfg_handle *h, int s) {
 /* One coupled step, in the order of the reference's per-step calls
  * (gpuSEM_LB.c:1441-1442 -> semLB.cu:441-531 then semLB.cu:303-438):
  * forces from X(n), spread, LB with F(n), interpolate, move.  The stages are
- * fused into seven to ten launches (cell lists, scan, scatter, sort + sums +
- * bond decisions, bond resolution, forces, spreading, LB, move; resolution
- * joins the sort launch with few receptors, spreading joins the forces with
- * a wavefront per marker); the LB update zeroes the force it reads, so the
+ * fused into four to thirteen launches (four: positions and run boxes, forces
+ * with spreading, LB, move; where something reads them, cell lists in a count,
+ * a scan and a scatter; sort + sums + bond decisions, bond resolution where
+ * there are many receptors; two more for the force pass by body, one or two
+ * for spreading that does not ride along; bending adds three, contact two);
+ * the LB update zeroes the force it reads, so the
  * next step's spreading adds into zeros without a clearing pass.
- * With overlap, the first marker launch stamps the rows the IB stencils
- * touch; the LB update of all other rows then runs on stream2 while the
- * marker pipeline runs on the main stream, and the stamped rows update
+ * With overlap, the first marker launch stamps the blocks the IB stencils
+ * touch; the LB update of all other blocks then runs on stream2 while the
+ * marker pipeline runs on the main stream, and the stamped blocks update
  * after the spreading.  Without overlap (or when the LB launch is timed by
  * lb0/lb1), one LB launch follows the spreading. */
 static hipError_t enqueue_step(pfg_handle *h, hipEvent_t lb0, hipEvent_t lb1) {

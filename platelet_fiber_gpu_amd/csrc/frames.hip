@@ -9,10 +9,11 @@
  * half being written meanwhile.  Bound by PCIe (53 GB/s) and by the page
  * faults of the caller's new arrays, which one thread takes at 7-9 GB/s.
  * Against a copy per array from pageable memory (us): report of a step 44 ->
- * 13, markers of 256 elements 205 -> 27, of 520 000 1000 -> 530, of 2.08 M
- * 9300 -> 4300; fields of 201x99x75 cells 1430 -> 680-1400, of 128^3
- * 4540 -> 1840, of 320x128x128 9390 -> 2780.  6 to 16 threads and halves of 4
- * to 16 MiB measured the same.
+ * 13-15, markers of 256 elements 205 -> 26-30, of 520 000 1000 -> 530-570, of
+ * 2.08 M 9300 -> 4300; fields into new arrays of 201x99x75 cells
+ * 1430 -> 1220-1510, of 128^3 4540 -> 1510-1760, of 320x128x128
+ * 9390 -> 2620-2960 (by host).  6 to 16 threads and halves of 4 to 16 MiB
+ * measured the same.
  */
 #include <hip/hip_runtime.h>
 #include <sched.h>

@@ -78,7 +78,7 @@ struct MArgs {
   int roles;
   int halt; /* 1: after the detach test fires, leave bonds, force field and
                markers unchanged (the step loop ends at detach) */
-  int mark_rows; /* 1: stamp the x-block rows this step's IB stencils touch */
+  int mark_rows; /* 1: stamp the blocks this step's IB stencils touch */
   int resolve_last; /* 1: the gather launch's last workgroup resolves the bonds */
   int count_spans;  /* 1: the counting launch adds the scan's span totals */
   int bin_elements; /* 0: the cell lists hold the markers other than elements
@@ -489,8 +489,8 @@ __global__ __launch_bounds__(256) void begin_kernel(MArgs a) {
   if (!a.again) a.m.pos4[i] = p;
   if (a.lists) bin_marker(a, i, L, kind_i, p);
   if (a.mark_rows && ib_coupled(a.m.kind[i], a.fiber_move) && !halted(a)) {
-    /* stamp the rows of this step's 4x4x4 stencil (the nodes spreading and
-     * interpolation use), so that the LB update of every other row may run
+    /* stamp the blocks of this step's 4x4x4 stencil (the nodes spreading and
+     * interpolation use), so that the LB update of every other block may run
      * before the spreading */
     const int step = (int)*a.m.d_step;
     const int ox = floor_index(wrap_coord(a.m.x[i], L.nx, L.periodic[0]), L.nx) - 1;
@@ -1337,7 +1337,7 @@ __device__ void bond_decide(const MArgs &a, int r, int *off, int *ends) {
 /* roles: A = sort bins (blocks0, one lane per marker: each marker takes its
  * rank by index among the scatter order of its bin, and writes its index and
  * packed position there), B = platelet sums (blocks1 = one block per platelet),
- * C = bond decisions (blocks2, four receptors per block; they read the
+ * C = bond decisions (blocks2, REC_PER_BLOCK receptors each; they read the
  * scatter order, which no role of this launch writes) */
 __device__ void gather_body(const MArgs &a) {
   int blk = blockIdx.x;

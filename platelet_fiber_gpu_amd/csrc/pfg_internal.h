@@ -419,7 +419,7 @@ struct pfg_handle {
   bool overlap = false;
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  int32_t *row_stamp = nullptr;    /* per x-block row of every lattice      */
+  int32_t *row_stamp = nullptr;    /* per block of every lattice            */
   int64_t h_step = 0;
   /* lattices: one, or a batch stepped together */
   int K = 1;
@@ -458,8 +458,7 @@ hipError_t launch_init_eq(pfg_handle *h, int k, const float *rho, const float *u
 hipError_t launch_convert_f(pfg_handle *h, float *f_out_or_null,
                             const float *f_in_or_null);
 hipError_t launch_conservation(pfg_handle *h, int k, double out[4]);
-/* persistent batched LB launch: row ranges (one per XCD) and x-block rows per
- * grab */
+/* persistent batched LB launch: ranges (one per XCD) and blocks per grab */
 constexpr int LB_QUEUES = 8;
 constexpr int LB_QUEUE_GRAB = 16;
 /* pfg_download_fields_noalloc: staging in a fixed device array of
