@@ -1638,13 +1638,13 @@ pfg_status pfg_cell_grid(const pfg_handle *h, int32_t dims[3]) {
   return PFG_OK;
 }
 
-/* The lists and boxes that the stages and pfg_download_cells read under the
+/* The lists (and boxes) that the stages and pfg_download_cells read under the
  * present settings, where the last steps or a CELLS stage under others left
  * different ones: made again from the positions they started from. */
-static hipError_t current_lists(pfg_handle *h) {
+static hipError_t current_lists(pfg_handle *h, bool boxes) {
   const int want = bin_elements(h) ? LISTS_FULL : LISTS_COARSE;
   if (h->lists_kept == LISTS_AS_LOADED ||
-      (h->lists_kept == want && (h->boxes_kept || h->m.n_runs == 0)))
+      (h->lists_kept == want && (!boxes || h->boxes_kept || h->m.n_runs == 0)))
     return hipSuccess;
   const hipError_t e = launch_cells_again(h);
   h->lists_kept = e == hipSuccess ? want : LISTS_NONE;
@@ -1656,7 +1656,7 @@ pfg_status pfg_download_cells(pfg_handle *h, int32_t *bin_start, int32_t *bin_it
   if (!h) return PFG_ERR_ARG;
   if (!h->model_loaded) return PFG_ERR_STATE;
   hipSetDevice(h->device);
-  PFG_TRY(current_lists(h));
+  PFG_TRY(current_lists(h, false));
   const int64_t nb = bin_elements(h) ? h->m.nbins : h->m.nbinsc;
   Piece p[2] = {{bin_start, h->m.bin_start, sizeof(int32_t) * ((size_t)nb + 1)},
                 {bin_items, h->m.bin_items, sizeof(int32_t) * (size_t)h->m.n}};
@@ -1675,7 +1675,7 @@ pfg_status pfg_download_aux(pfg_handle *h, float *a3n) {
 /* ---------------- stepping ---------------- */
 
 static hipError_t run_stage(pfg_handle *h, int s) {
-  hipError_t e = stage_reads_lists(h, s) ? current_lists(h) : hipSuccess;
+  hipError_t e = stage_reads_lists(h, s) ? current_lists(h, s == PFG_STAGE_FORCES) : hipSuccess;
   if (e != hipSuccess) return e;
   switch (s) {
     case PFG_STAGE_CELLS:
