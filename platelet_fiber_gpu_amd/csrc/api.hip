@@ -1638,13 +1638,15 @@ pfg_status pfg_cell_grid(const pfg_handle *h, int32_t dims[3]) {
   return PFG_OK;
 }
 
-/* The lists (and boxes) that the stages and pfg_download_cells read under the
+/* The lists (in order, and boxes) that the stages and pfg_download_cells read under the
  * present settings, where the last steps or a CELLS stage under others left
  * different ones: made again from the positions they started from. */
-static hipError_t current_lists(pfg_handle *h, bool boxes) {
+static hipError_t current_lists(pfg_handle *h, bool order, bool boxes) {
   const int want = bin_elements(h) ? LISTS_FULL : LISTS_COARSE;
+  const bool kept = h->lists_kept == want || (h->lists_kept == LISTS_COARSE_UNORDERED &&
+                                              want == LISTS_COARSE && !order);
   if (h->lists_kept == LISTS_AS_LOADED ||
-      (h->lists_kept == want && (!boxes || h->boxes_kept || h->m.n_runs == 0)))
+      (kept && (!boxes || h->boxes_kept || h->m.n_runs == 0)))
     return hipSuccess;
   const hipError_t e = launch_cells_again(h);
   h->lists_kept = e == hipSuccess ? want : LISTS_NONE;
@@ -1656,7 +1658,7 @@ pfg_status pfg_download_cells(pfg_handle *h, int32_t *bin_start, int32_t *bin_it
   if (!h) return PFG_ERR_ARG;
   if (!h->model_loaded) return PFG_ERR_STATE;
   hipSetDevice(h->device);
-  PFG_TRY(current_lists(h, false));
+  PFG_TRY(current_lists(h, true, false));
   const int64_t nb = bin_elements(h) ? h->m.nbins : h->m.nbinsc;
   Piece p[2] = {{bin_start, h->m.bin_start, sizeof(int32_t) * ((size_t)nb + 1)},
                 {bin_items, h->m.bin_items, sizeof(int32_t) * (size_t)h->m.n}};
@@ -1675,7 +1677,9 @@ pfg_status pfg_download_aux(pfg_handle *h, float *a3n) {
 /* ---------------- stepping ---------------- */
 
 static hipError_t run_stage(pfg_handle *h, int s) {
-  hipError_t e = stage_reads_lists(h, s) ? current_lists(h, s == PFG_STAGE_FORCES) : hipSuccess;
+  hipError_t e = hipSuccess;
+  if (stage_reads_lists(h, s))
+    e = current_lists(h, s != PFG_STAGE_BONDS, s == PFG_STAGE_FORCES);
   if (e != hipSuccess) return e;
   switch (s) {
     case PFG_STAGE_CELLS:
@@ -1809,7 +1813,7 @@ static hipError_t read_report(pfg_handle *h, int64_t r[N_COUNTERS + 2]) {
 static void note_step_lists(pfg_handle *h, int nsteps) {
   if (nsteps == 0 || !h->model_loaded || h->m.n == 0 || h->fluid_only) return;
   h->lists_kept = !step_lists(h) ? LISTS_NONE
-                  : step_bin_elements(h) ? LISTS_FULL : LISTS_COARSE;
+                  : step_bin_elements(h) ? LISTS_FULL : LISTS_COARSE_UNORDERED;
   h->boxes_kept = by_runs(h);
 }
 

@@ -116,8 +116,9 @@ constexpr int64_t LB_LARGE_CELLS = (int64_t)1 << 27;
 constexpr int BLOCK_FLUID = 0, BLOCK_MIXED = 1, BLOCK_SOLID = 2;
 /* Cell lists a handle holds: the empty ones of the load, none (a step that
  * reads no list keeps none), those of the markers other than elements on the
- * coarse grid, those of every marker. */
-enum { LISTS_AS_LOADED, LISTS_NONE, LISTS_COARSE, LISTS_FULL };
+ * coarse grid (a step's own have bin_scatter, which the bonds read, but not
+ * its order in bin_items), those of every marker. */
+enum { LISTS_AS_LOADED, LISTS_NONE, LISTS_COARSE_UNORDERED, LISTS_COARSE, LISTS_FULL };
 /* Device counters of a handle (Markers::counters). */
 constexpr int N_COUNTERS = 16;
 /* Morse pairs whose distance lies within this of the cutoff are counted: a

@@ -352,13 +352,15 @@ def test_stages_after_a_step_that_kept_other_lists(gpu, stage, stepped, then, fi
     assert np.abs(aux0 - aux1).max() <= 1e-5 * np.abs(aux0).max()
 
 
+@pytest.mark.parametrize("receptors", [-1, 16])
 @pytest.mark.parametrize("by_body", [0, 1])
-def test_cell_lists_after_steps_without_them(gpu, by_body):
-    """Steps that need no cell lists keep none; asked for afterwards, they are those
+def test_cell_lists_after_steps_without_them(gpu, by_body, receptors):
+    """Steps that need no cell lists keep none, and those whose bonds read the fibrin
+    nodes' lists keep these without an order; asked for afterwards, they are those
     of the positions the last step started from, as the CELLS stage gives them."""
     pfg = gpu
     sc = pfg.Scene(pfg.SCENE_LARGE, nx=96, ny=64, nz=64, n_platelets=3, elements=200,
-                   receptors=-1, ligands=-1, fibrin_nodes=128, fibrin_links=150)
+                   receptors=receptors, ligands=receptors, fibrin_nodes=128, fibrin_links=150)
     with pfg.Solver(sc.params) as s:
         s.load(sc)
         s.set_forces_by_body(by_body)
