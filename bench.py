@@ -142,7 +142,7 @@ def time_oracle(o, cells, budget_s=10.0, min_steps=2, max_steps=200):
 def cpu_leg_shear(pfg):
     """CPU leg of the headline workload.  Baseline: the FP64 oracle (the same
     algorithm, OpenMP over cells) on a bounded sample of the same workload,
-    about 10 s of coupled steps of the 256x128x128 shear scene.  Checker: the
+    about 10 s of coupled steps of the 256x128x128 shear scene.  Accuracy: the
     FP16-store (and BF16-store) velocity error against the oracle on a
     64x32x32 body-force channel, tau 0.8, F = 1e-6, 300 steps."""
     import numpy as np
@@ -178,7 +178,7 @@ def cpu_leg_shear(pfg):
 def cpu_leg_large(pfg, horizons=(50, 200)):
     """CPU leg of the large workload, on a 128^3 sub-box of its physics
     (16 platelets, fibrin and wall ligands at its densities, hard Morse
-    cutoff).  Checker: velocity and density L2 and platelet-centroid errors
+    cutoff).  Accuracy: velocity and density L2 and platelet-centroid errors
     of FP16-store and FP32-store device runs against the FP64 oracle after
     each horizon, beside the distance between two FP64 runs whose initial
     positions differ by 1e-6 (how far the trajectory itself departs: the
