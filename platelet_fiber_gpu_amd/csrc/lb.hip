@@ -42,25 +42,29 @@ namespace pfg {
 
 /* ---------------- storage formats ---------------- */
 
-/* load: the stored value as float (FP16 values stay scaled by 2^s);
- * pack: an already scaled value as it is stored. */
+/* Raw: a stored value in a register of its own (an array of 16-bit values that
+ * is carried across branches is packed in pairs, each wait for the load of
+ * one of a pair); value: a stored value as float (FP16 values stay scaled by
+ * 2^s); pack: an already scaled value as it is stored. */
 template <int S>
 struct Store;
 
 template <>
 struct Store<PFG_STORE_F32> {
   using T = float;
+  using Raw = float;
   static constexpr bool scaled = false;
-  __device__ static inline float load(const T *p) { return *p; }
+  __device__ static inline float value(Raw v) { return v; }
   __device__ static inline T pack(float v) { return v; }
 };
 
 template <>
 struct Store<PFG_STORE_F16> {
   using T = uint16_t;
+  using Raw = uint32_t;
   static constexpr bool scaled = true;
-  __device__ static inline float load(const T *p) {
-    return (float)__builtin_bit_cast(_Float16, *p);
+  __device__ static inline float value(Raw v) {
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)v);
   }
   __device__ static inline T pack(float v) {
     return __builtin_bit_cast(uint16_t, (_Float16)v); /* round to nearest even */
@@ -70,10 +74,9 @@ struct Store<PFG_STORE_F16> {
 template <>
 struct Store<PFG_STORE_BF16> {
   using T = uint16_t;
+  using Raw = uint32_t;
   static constexpr bool scaled = false;
-  __device__ static inline float load(const T *p) {
-    return __builtin_bit_cast(float, ((uint32_t)*p) << 16);
-  }
+  __device__ static inline float value(Raw v) { return __builtin_bit_cast(float, v << 16); }
   __device__ static inline T pack(float v) {
     uint32_t u = __builtin_bit_cast(uint32_t, v);
     u += 0x7FFFu + ((u >> 16) & 1u); /* round to nearest even */
@@ -256,6 +259,15 @@ __device__ __forceinline__ void lb_cell(const LBArgs &a, float (&dev)[Q], int x,
   }
 }
 
+/* The populations that come in from a wall: directions whose component along
+ * axis AX has sign SGN, each the opposite one that leaves the cell (bb). */
+template <int AX, int SGN, typename RAW, typename T>
+__device__ __forceinline__ void bounce_loads(RAW (&pop)[Q], const T *bb) {
+#pragma unroll
+  for (int d = 1; d < Q; ++d)
+    if ((AX == 0 ? CX[d] : (AX == 1 ? CY[d] : CZ[d])) == SGN) pop[d] = bb[BB[d] * XBLOCK];
+}
+
 /* One wavefront per block of 64 cells; workgroup `blk` of the lattice
  * described by `a` (in memory that the whole workgroup reads), the
  * wavefront's place in it `wave` (default: its place in the launch's
@@ -312,6 +324,7 @@ __device__ __forceinline__ void lb_update(const LBArgs &a, uint32_t blk, float *
       return;
     }
   }
+  const bool wall_moves = a.wall_moves != 0;
   const uint32_t nx = (uint32_t)a.nx, ny = (uint32_t)a.ny, nxy = nx * ny;
   const uint32_t wz = i0 / nxy, wr = i0 - wz * nxy, wy = wr / nx, wx = wr - wy * nx;
   /* rows and planes passed since the wavefront's first cell: at most one of a
@@ -328,8 +341,8 @@ __device__ __forceinline__ void lb_update(const LBArgs &a, uint32_t blk, float *
   if (M == LB_MODE_STEP || M == LB_MODE_REGION)
     stamp = a.tile_stamp[(x >> TILE_SHIFT_X) +
                          a.tnx * ((y >> TILE_SHIFT_Y) + a.tny * (z >> TILE_SHIFT_Z))];
-  /* offset to the upstream neighbour along each axis, 0 outside a wall (the
-   * edge pass replaces what that reads) */
+  /* offset to the upstream neighbour along each axis, 0 outside a wall (what
+   * that reads is replaced) */
   const bool xlo = x == 0, xhi = x == a.nx - 1, ylo = y == 0, yhi = y == a.ny - 1,
              zlo = z == 0, zhi = z == a.nz - 1;
   const bool oxm = xlo && !a.periodic[0], oxp = xhi && !a.periodic[0];
@@ -339,14 +352,56 @@ __device__ __forceinline__ void lb_update(const LBArgs &a, uint32_t blk, float *
   const int xm = xlo ? (oxm ? 0 : sx - 1) : -1, xp = xhi ? (oxp ? 0 : 1 - sx) : 1;
   const int ym = ylo ? (oym ? 0 : sy - sx) : -sx, yp = yhi ? (oyp ? 0 : sx - sy) : sx;
   const int zm = zlo ? (ozm ? 0 : sz - sy) : -sy, zp = zhi ? (ozp ? 0 : sy - sz) : sy;
-  float dev[Q];
-#pragma unroll
-  for (int d = 0; d < Q; ++d) {
+  const uint64_t own = (uint64_t)task * R + lane;
+  const bool edge = oxm || oxp || oym || oyp || ozm || ozp || mask != 0;
+  auto upstream = [&](int d) { /* element of direction 0 */
     const int off = (CX[d] > 0 ? xm : (CX[d] < 0 ? xp : 0)) +
                     (CY[d] > 0 ? ym : (CY[d] < 0 ? yp : 0)) +
                     (CZ[d] > 0 ? zm : (CZ[d] < 0 ? zp : 0));
     const uint32_t src = i + (uint32_t)off;
-    dev[d] = ST::load(fin + d * XBLOCK + ((uint64_t)(src >> 6) * R + (src & (XBLOCK - 1))));
+    return (uint64_t)(src >> 6) * R + (src & (XBLOCK - 1));
+  };
+  /* Upstream cell outside a wall or solid: halfway bounce-back, the
+   * population leaving this cell returns.  No lane waits for a load here: a
+   * second load of the same population comes after the first, and values are
+   * used when all are on their way (a pass that took both and added the wall's
+   * term in one branch waited once for each of a wavefront's directions).
+   * Streamed FP32, bound by HBM, selects the address instead and loads once.
+   * LB-only launches with walls on all sides, us, one pass after the other /
+   * now: FP16 192^3 119 / 87, 256^3 261 / 209, 100^3 19.8 / 13.7, 512x256x256
+   * 463 / 419; FP32 192^3 196 / 181, 256^3 463 / 434, 100^3 24.6 / 20.3,
+   * 512x256x256 893 / 869 (selecting in FP16: 256^3 284, its arithmetic being
+   * the limit; loading twice in FP32: 256^3 445, 512x256x256 899).  A tube's
+   * mixed blocks: 256^3 FP16 157 / 153, 201x99x75 FP16 16.3 / 14.5, FP32
+   * 20.6 / 19.2.  64x32x32 without walls 4.0 / 4.4, with 5.9 / 4.5. */
+  constexpr bool SELECT = S == PFG_STORE_F32 && !(MODE & LB_CACHED);
+  typename ST::Raw pop[Q];
+  if (!SELECT || __ballot(edge) == 0) {
+#pragma unroll
+    for (int d = 0; d < Q; ++d) pop[d] = fin[d * XBLOCK + upstream(d)];
+  } else {
+#pragma unroll
+    for (int d = 0; d < Q; ++d) {
+      const bool oz = CZ[d] > 0 ? ozm : (CZ[d] < 0 ? ozp : false);
+      const bool oy = CY[d] > 0 ? oym : (CY[d] < 0 ? oyp : false);
+      const bool ox = CX[d] > 0 ? oxm : (CX[d] < 0 ? oxp : false);
+      const bool out = oz || oy || ox || ((mask >> d) & 1u); /* never for d = 0 */
+      pop[d] = fin[out ? own + BB[d] * XBLOCK : d * XBLOCK + upstream(d)];
+    }
+  }
+  if (!SELECT && edge) {
+    const T *bb = fin + own;
+    if (oxm) bounce_loads<0, 1>(pop, bb);
+    if (oxp) bounce_loads<0, -1>(pop, bb);
+    if (oym) bounce_loads<1, 1>(pop, bb);
+    if (oyp) bounce_loads<1, -1>(pop, bb);
+    if (ozm) bounce_loads<2, 1>(pop, bb);
+    if (ozp) bounce_loads<2, -1>(pop, bb);
+    if (mask != 0) {
+#pragma unroll
+      for (int d = 1; d < Q; ++d)
+        if ((mask >> d) & 1u) pop[d] = bb[BB[d] * XBLOCK];
+    }
   }
   /* the IB force of the tiles this step's stencils meet, read and consumed
    * (the next step's spreading adds into zeros) */
@@ -360,22 +415,23 @@ __device__ __forceinline__ void lb_update(const LBArgs &a, uint32_t blk, float *
       az = a.aux[2 * a.plane + i];
     }
   }
-  /* edge pass: upstream cell outside a wall or solid: halfway bounce-back,
-   * the population leaving this cell returns plus the moving-wall momentum
-   * 6 w (c . u_wall) (z wall over y wall over x wall). */
-  const uint64_t own = (uint64_t)task * R + lane;
-  if (oxm || oxp || oym || oyp || ozm || ozp || mask != 0) {
+  float dev[Q];
+#pragma unroll
+  for (int d = 0; d < Q; ++d) dev[d] = ST::value(pop[d]);
+  /* the moving wall's momentum 6 w (c . u_wall), z wall over y wall over x */
+  if (wall_moves && edge) {
+    int k = 0; /* keeps the loads of the terms in here */
+    asm volatile("" : "+s"(k));
 #pragma unroll
     for (int d = 1; d < Q; ++d) {
       const bool oz = CZ[d] > 0 ? ozm : (CZ[d] < 0 ? ozp : false);
       const bool oy = CY[d] > 0 ? oym : (CY[d] < 0 ? oyp : false);
       const bool ox = CX[d] > 0 ? oxm : (CX[d] < 0 ? oxp : false);
-      if (oz || oy || ox || ((mask >> d) & 1u)) {
-        const int sxs = CX[d] > 0 ? 0 : 1, sys = CY[d] > 0 ? 0 : 1, szs = CZ[d] > 0 ? 0 : 1;
-        const float term = oz ? a.wall_term[2][szs][d]
-                              : (oy ? a.wall_term[1][sys][d] : (ox ? a.wall_term[0][sxs][d] : 0.f));
-        dev[d] = ST::load(fin + own + BB[d] * XBLOCK) + term;
-      }
+      const int sx = CX[d] > 0 ? 0 : 1, sy = CY[d] > 0 ? 0 : 1, sz = CZ[d] > 0 ? 0 : 1;
+      const float tx = CX[d] != 0 ? a.wall_term[0][sx][d + k] : 0.f;
+      const float ty = CY[d] != 0 ? a.wall_term[1][sy][d + k] : 0.f;
+      const float tz = CZ[d] != 0 ? a.wall_term[2][sz][d + k] : 0.f;
+      dev[d] += oz ? tz : (oy ? ty : (ox ? tx : 0.f));
     }
   }
   lb_cell<S, MODE>(a, dev, x, y, zlo, zhi, i, flagged, ax, ay, az, fout + own, orho, oux, ouy,
@@ -664,7 +720,7 @@ __global__ void convert_plane_kernel(LBArgs a, void *stored, float *buf, int d, 
   T *p = (T *)stored + felem(d, idx);
   const float w = weight(d);
   if (to_float) {
-    buf[idx] = w + ST::load(p) * (ST::scaled ? a.inv_scale : 1.0f);
+    buf[idx] = w + ST::value(*(p)) * (ST::scaled ? a.inv_scale : 1.0f);
   } else {
     put<S, false>(p, (buf[idx] - w) * (ST::scaled ? a.scale : 1.0f));
   }
@@ -686,7 +742,7 @@ __global__ __launch_bounds__(256) void conservation_kernel(LBArgs a, const void 
     double cm = 0, cx = 0, cy = 0, cz = 0;
 #pragma unroll
     for (int d = 0; d < Q; ++d) {
-      const double v = (double)ST::load(p + e0 + d * XBLOCK);
+      const double v = (double)ST::value(*(p + e0 + d * XBLOCK));
       cm += v;
       cx += CX[d] * v;
       cy += CY[d] * v;
@@ -779,12 +835,14 @@ void make_lb_args(const pfg_handle *h, int k, int cur, LBArgs *a) {
   /* halfway bounce-back with a moving wall (Ladd): the population entering
    * from the wall is f_bb(d) + 6 w_d rho_w (c_d . u_w), rho_w = 1; in the
    * storage units of the format */
+  a->wall_moves = 0;
   for (int ax = 0; ax < 3; ++ax)
     for (int s = 0; s < 2; ++s)
       for (int d = 0; d < Q; ++d) {
         const float *u = s == 0 ? p.wall_u_lo[ax] : p.wall_u_hi[ax];
         const float cu = CX[d] * u[0] + CY[d] * u[1] + CZ[d] * u[2];
         a->wall_term[ax][s][d] = 6.0f * weight(d) * cu * a->scale;
+        a->wall_moves |= a->wall_term[ax][s][d] != 0.0f;
       }
   a->zvel = p.wall[2] == PFG_WALL_VELOCITY ? 1 : 0;
   a->xcd_rows = h->lb_xcd_rows;

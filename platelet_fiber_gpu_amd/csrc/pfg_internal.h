@@ -150,6 +150,7 @@ struct LBArgs {
                              launch                                          */
   int tnx, tny;           /* tiles per axis                                   */
   int periodic[3];
+  int wall_moves;         /* some wall_term is not zero                       */
   float omega;            /* 1/tau                                           */
   float guo;              /* 1 - 1/(2 tau)                                   */
   float g[3];             /* body force                                      */

@@ -87,6 +87,42 @@ def test_blocks_across_rows_and_planes(gpu, po, size, walls):
         assert (got[~fluid] == 0).all()
 
 
+@pytest.mark.parametrize("solid", [False, True])
+@pytest.mark.parametrize("store, half_ulp", [(0, 0.0), (1, 2.0 ** -11)])
+@pytest.mark.parametrize("size", [(5, 7, 3), (64, 3, 2), (67, 66, 5), (131, 130, 132)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_moving_walls_of_every_axis(gpu, po, size, store, half_ulp, solid):
+    """Walls on every side, each with its own velocity, their edges and corners, solid
+    cells beside them, in lattices that stay in the cache and in one that does not
+    (where FP32 takes the loads in another way).  From the stored state: the rounding
+    of one FP32 step (3e-7), and half an ulp of the stored deviation."""
+    pfg = gpu
+    nx, ny, nz = size
+    N = nx * ny * nz
+    rng = np.random.default_rng(N + store)
+    flags = (rng.random(N) < 0.1).astype(np.uint8) if solid else None
+    p = pfg.default_params(nx=nx, ny=ny, nz=nz, store=store, use_flags=int(solid))
+    for a in range(3):
+        p.wall[a] = pfg.WALL_BOUNCE
+        for c in range(3):
+            if c != a:
+                p.wall_u_lo[a][c], p.wall_u_hi[a][c] = rng.uniform(-0.05, 0.05, 2)
+    w = np.array([po.load().orc_w(d) for d in range(19)])[:, None]
+    f = (w * (1 + 0.05 * rng.standard_normal((19, N)))).astype(np.float32)
+    with pfg.Solver(p) as s:
+        if solid:
+            s.upload_flags(flags)
+        s.set_f(f)
+        f = s.f().astype(np.float64)
+        s.set_fluid_only(True)
+        s.step(1)
+        fg = s.f().astype(np.float64)
+    fo = po.lb_step(po.lattice(p, flags), f)
+    fluid = slice(None) if flags is None else flags == 0
+    err = np.abs(fg - fo) - 1.01 * half_ulp * np.abs(fo - w)
+    assert err[:, fluid].max(initial=0.0) < 3e-7
+
+
 @pytest.mark.parametrize("nx", [60, 101])
 def test_overlap_equals_serial_on_rows_that_share_blocks(gpu, nx):
     """The blocks that the stencils touch are stamped by cell index: a platelet
